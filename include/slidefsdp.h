@@ -227,6 +227,38 @@ int sf_gather_rows_b16(const uint16_t* src, const int64_t* ids, size_t ntok,
                        uint32_t* bad, int max_workgroups, sf_stream_t stream);
 
 /* ---------------------------------------------------------------------
+ * Cross entropy of the output unit (libsf_hip.so): what lies between the
+ * three products of the fused linear + cross entropy that the reference's
+ * output unit uses when installed (slide_fsdp.py:57-63, 85-97).
+ * ------------------------------------------------------------------- */
+
+/* One chunk of logits, [rows, vocab] with ld elements from row to row, as
+ * dtype (SF_DTYPE_F32, SF_DTYPE_BF16 or SF_DTYPE_F16).  For each row with
+ * label y: row_loss = logsumexp(row) - row[y] in fp32, and the row becomes
+ * its gradient softmax(row) - onehot(y), computed in fp32 and rounded once
+ * to nearest even.  A row whose label is ignore_index: loss 0, gradient 0.
+ * A label outside [0, vocab): loss and gradient NaN.  16-bit logits start on
+ * 16-byte boundaries, every row of them (ld a multiple of 8; SF_EALIGN
+ * otherwise); the ld - vocab elements behind a row are scratch. */
+int sf_ce_rows(void* logits, int dtype, size_t ld, size_t rows, size_t vocab,
+               const int64_t* labels, int64_t ignore_index, float* row_loss,
+               sf_stream_t stream);
+
+/* *n_valid = number of labels != ignore_index, *loss = sum of row_loss over
+ * it (NaN if there are none), both in device memory. */
+int sf_ce_loss(const float* row_loss, const int64_t* labels, size_t n,
+               int64_t ignore_index, float* loss, float* n_valid,
+               sf_stream_t stream);
+
+/* Both gradients times *grad_loss / *n_valid: grad_h (n_h elements of dtype)
+ * into grad_h_out, grad_w (n_w fp32 elements) rounded once into grad_w_out
+ * (dtype).  All four arrays start on 16-byte boundaries (SF_EALIGN). */
+int sf_ce_scale(const float* grad_loss, const float* n_valid,
+                const void* grad_h, void* grad_h_out, size_t n_h,
+                const float* grad_w, void* grad_w_out, size_t n_w, int dtype,
+                sf_stream_t stream);
+
+/* ---------------------------------------------------------------------
  * Copies and pinned host memory (libsf_hip.so)
  * ------------------------------------------------------------------- */
 

@@ -47,7 +47,8 @@ def build_hip(verbose: bool = False) -> str:
     tmp = _atomic_out(out)
     _run([HIPCC, f"--offload-arch={OFFLOAD_ARCH}", "-O3", "-std=c++17", "-fPIC", "-shared",
           "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-          "-I", INCLUDE, "-o", tmp, os.path.join(CSRC, "sf_hip.hip"), "-lhsa-runtime64"], verbose)
+          "-I", INCLUDE, "-o", tmp, os.path.join(CSRC, "sf_hip.hip"), os.path.join(CSRC, "sf_ce.hip"),
+          "-lhsa-runtime64"], verbose)
     os.replace(tmp, out)
     return out
 

@@ -1,0 +1,472 @@
+// Cross entropy of the output unit over one chunk of logits, and the scaling
+// of its gradients, for MI355X (gfx950).
+//
+// The three products around these kernels (logits, hidden and weight
+// gradient) are library GEMMs; what lies between them is bound by HBM, and as
+// separate elementwise and reduction passes it cost more than the products
+// themselves: widening, logsumexp (three passes), gather, subtract, exp, the
+// one-hot update, the mask and the rounding back moved some 25 bytes per
+// logit and launched about 20 kernels per chunk.  ce_rows_kernel reads every
+// logit once and writes its gradient over it: 4 bytes per 16-bit logit.
+// Measured at 4092 rows of 128256 bf16 logits: ce_rows_kernel 0.389 ms (5.4
+// TB/s; a device copy reaches 5.1), ce_scale16_kernel for the 128256 x 4096
+// weight and 4092 x 4096 hidden gradients 0.521 ms (6.1 TB/s).  The same steps
+// as torch operations took 7.2 ms, and adding the chunks' weight gradients
+// into the fp32 sum 8.1 ms more; loss with both gradients 35.1 -> 11.3 ms, of
+// which 10.8 are the products.  At 510 rows of 4096 (hidden 512): 453 -> 263
+// us, 57 of them on the GPU, the rest host time of the launches.
+//
+// The C ABI is declared in include/slidefsdp.h.
+
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "../../include/slidefsdp.h"
+
+namespace {
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+
+constexpr float kLog2e = 1.44269504088896340736f;
+constexpr int kGroup = 8;   // 16-bit elements per 128-bit access
+
+// 16-bit formats: a pair in a 32-bit word <-> two floats.  The conversions
+// back round to nearest even (v_cvt_pk_bf16_f32, v_cvt_f16_f32), as torch's.
+struct Bf16 {
+    static constexpr uint32_t kNegInf2 = 0xFF80FF80u;
+    static constexpr uint32_t kNegInf = 0xFF80u;
+    static constexpr uint32_t kNan2 = 0x7FC07FC0u;
+    __device__ static float lo(uint32_t w) { return __uint_as_float(w << 16); }
+    __device__ static float hi(uint32_t w) { return __uint_as_float(w & 0xFFFF0000u); }
+    __device__ static uint32_t pack(float a, float b) {
+        const f32x2 f = {a, b};
+        return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf16x2));
+    }
+};
+struct F16 {
+    static constexpr uint32_t kNegInf2 = 0xFC00FC00u;
+    static constexpr uint32_t kNegInf = 0xFC00u;
+    static constexpr uint32_t kNan2 = 0x7E007E00u;
+    __device__ static float lo(uint32_t w) { return float(__builtin_bit_cast(f16x2, w).x); }
+    __device__ static float hi(uint32_t w) { return float(__builtin_bit_cast(f16x2, w).y); }
+    __device__ static uint32_t pack(float a, float b) {
+        const f32x2 f = {a, b};
+        return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, f16x2));
+    }
+};
+
+// exp(t) for t <= 0 or so, as 2^(t log2 e): v_exp_f32 has no range reduction
+// to pay for.  The product's rounding costs |t| 2^-24 relative, far below the
+// 16-bit rounding of what it feeds and, in the sum, below fp32 addition's.
+__device__ __forceinline__ float exp_fast(float t) { return __builtin_amdgcn_exp2f(t * kLog2e); }
+
+// A partial logsumexp: the maximum so far and the sum of exp(x - base(max)).
+// base() is the maximum itself, or 0 where that is infinite, so that rows
+// with infinities give what logsumexp gives: +inf, or -inf for a row of them.
+struct Lse {
+    float m, s;
+};
+__device__ __forceinline__ float base(float m) { return __builtin_isinf(m) ? 0.0f : m; }
+
+__device__ __forceinline__ Lse merge(Lse a, Lse b) {
+    const float m = fmaxf(a.m, b.m);
+    const float c = base(m);
+    // an empty part stays empty whatever the bases are; a NaN sum stays NaN
+    const float sa = a.s == 0.0f ? 0.0f : a.s * exp_fast(base(a.m) - c);
+    const float sb = b.s == 0.0f ? 0.0f : b.s * exp_fast(base(b.m) - c);
+    return {m, sa + sb};
+}
+
+// logsumexp over the workgroup, the same value in every lane.  Wave by
+// shuffles, then the waves' parts through LDS, merged by every lane in the
+// same order.
+template <int kT>
+__device__ __forceinline__ float block_lse(Lse p, Lse* parts) {
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) {
+        const Lse o = {__shfl_xor(p.m, d), __shfl_xor(p.s, d)};
+        p = merge(p, o);
+    }
+    if (kT > 64) {
+        if ((threadIdx.x & 63) == 0) parts[threadIdx.x >> 6] = p;
+    }
+    __syncthreads();
+    if (kT > 64) {
+        float m = parts[0].m;
+#pragma unroll
+        for (int w = 1; w < kT / 64; ++w) m = fmaxf(m, parts[w].m);
+        const float c = base(m);
+        float s = 0.0f;
+#pragma unroll
+        for (int w = 0; w < kT / 64; ++w)
+            s += parts[w].s == 0.0f ? 0.0f : parts[w].s * exp_fast(base(parts[w].m) - c);
+        p = {m, s};
+    }
+    return base(p.m) + logf(p.s);
+}
+
+// What a row's label asks for.
+enum RowKind { kValid, kIgnored, kBadLabel };
+__device__ __forceinline__ RowKind row_kind(int64_t y, int64_t ignore_index, uint32_t vocab) {
+    if (y == ignore_index) return kIgnored;
+    return (y < 0 || y >= int64_t(vocab)) ? kBadLabel : kValid;
+}
+
+// Make the compiler forget what the packed words were made of, so that it
+// unpacks them again in the next phase instead of keeping two floats alive
+// for each word (that is 152 VGPRs more at kG = 19, and it spilled).
+template <int kG>
+__device__ __forceinline__ void keep_packed(u32x4 (&v)[kG]) {
+#pragma unroll
+    for (int k = 0; k < kG; ++k)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            uint32_t w = v[k][j];
+            asm volatile("" : "+v"(w));
+            v[k][j] = w;
+        }
+}
+
+// ---------------------------------------------------------------------
+// One workgroup per row, the whole row in registers as packed 16-bit pairs:
+// kG groups of 8 per lane, so 4 kG VGPRs, up to 76 of the 128 a lane of a
+// 1024-lane workgroup has.  Read once, written once; between the two only
+// one barrier, since each lane sums against its own maximum and the parts
+// are merged with both.  All loads are issued before the first use (lanes
+// past the end of the row load its last group again and drop it).  The host
+// picks kG so that the row has more than kT kFull groups: the first kFull
+// groups of every lane need no check.
+// ---------------------------------------------------------------------
+template <typename Fmt, int kT, int kG, int kFull>
+__global__ __launch_bounds__(kT) void ce_rows_kernel(uint16_t* __restrict__ logits, uint64_t ld, uint32_t vocab,
+                                                     const int64_t* __restrict__ labels, int64_t ignore_index,
+                                                     float* __restrict__ row_loss) {
+    __shared__ Lse parts[kT / 64];
+    __shared__ float target;
+    const uint64_t row = blockIdx.x;
+    uint16_t* x = logits + row * ld;
+    u32x4* xv = reinterpret_cast<u32x4*>(x);
+    const int64_t y = labels[row];
+    const uint32_t groups = (vocab + kGroup - 1) / kGroup;
+    const RowKind kind = row_kind(y, ignore_index, vocab);
+    if (kind != kValid) {
+        const uint32_t w = kind == kIgnored ? 0u : Fmt::kNan2;
+        const u32x4 fill = {w, w, w, w};
+        for (uint32_t g = threadIdx.x; g < groups; g += kT) xv[g] = fill;
+        if (threadIdx.x == 0) row_loss[row] = kind == kIgnored ? 0.0f : __builtin_nanf("");
+        return;
+    }
+    u32x4 v[kG];
+#pragma unroll
+    for (int k = 0; k < kG; ++k) {
+        const uint32_t g = uint32_t(k) * kT + threadIdx.x;
+        v[k] = xv[k < kFull || g < groups ? g : groups - 1];
+    }
+    // Read before any lane writes: the barrier in block_lse stands between.
+    if (threadIdx.x == 0) target = Fmt::lo(x[y]);
+    const uint32_t rem = vocab % kGroup;
+#pragma unroll
+    for (int k = kFull; k < kG; ++k) {
+        const uint32_t g = uint32_t(k) * kT + threadIdx.x;
+        if (g >= groups) {
+            v[k] = u32x4{Fmt::kNegInf2, Fmt::kNegInf2, Fmt::kNegInf2, Fmt::kNegInf2};
+        } else if (rem != 0 && g == groups - 1) {
+            // the row's last, partial group: what follows it is padding
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                if (2 * uint32_t(j) >= rem) v[k][j] = Fmt::kNegInf2;
+                else if (2 * uint32_t(j) + 1 >= rem) v[k][j] = (v[k][j] & 0xFFFFu) | (Fmt::kNegInf << 16);
+            }
+        }
+    }
+    float m = -__builtin_inff();
+#pragma unroll
+    for (int k = 0; k < kG; ++k)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) m = fmaxf(fmaxf(m, Fmt::lo(v[k][j])), Fmt::hi(v[k][j]));
+    keep_packed<kG>(v);
+    const float c = base(m);
+    float s0 = 0.0f, s1 = 0.0f;
+#pragma unroll
+    for (int k = 0; k < kG; ++k)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            s0 += exp_fast(Fmt::lo(v[k][j]) - c);
+            s1 += exp_fast(Fmt::hi(v[k][j]) - c);
+        }
+    keep_packed<kG>(v);
+    const float lse = block_lse<kT>({m, s0 + s1}, parts);
+    if (threadIdx.x == 0) row_loss[row] = lse - target;
+#pragma unroll
+    for (int k = 0; k < kG; ++k) {
+        const uint32_t g = uint32_t(k) * kT + threadIdx.x;
+        u32x4 o;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            o[j] = Fmt::pack(exp_fast(Fmt::lo(v[k][j]) - lse), exp_fast(Fmt::hi(v[k][j]) - lse));
+        if (k < kFull || g < groups) xv[g] = o;
+    }
+    // The label's element, over what the same lane has just stored with its group.
+    if (threadIdx.x == uint32_t(y) / kGroup % kT)
+        x[y] = uint16_t(Fmt::pack(exp_fast(target - lse) - 1.0f, 0.0f));
+}
+
+// Element access of the streaming kernel below.
+struct Elem32 {
+    using S = float;
+    __device__ static float load(const S* p) { return *p; }
+    __device__ static void store(S* p, float f) { *p = f; }
+    __device__ static float exp(float t) { return expf(t); }   // results kept in fp32
+};
+template <typename Fmt>
+struct Elem16 {
+    using S = uint16_t;
+    __device__ static float load(const S* p) { return Fmt::lo(*p); }
+    __device__ static void store(S* p, float f) { *p = uint16_t(Fmt::pack(f, 0.0f)); }
+    __device__ static float exp(float t) { return exp_fast(t); }
+};
+
+// Rows that do not fit the registers (16-bit rows of more than 155,648
+// elements) and fp32 rows: one workgroup per row, two passes, the second one
+// over what the caches still hold.
+template <typename El, int kT>
+__global__ __launch_bounds__(kT) void ce_rows_stream_kernel(typename El::S* __restrict__ logits, uint64_t ld,
+                                                            uint32_t vocab, const int64_t* __restrict__ labels,
+                                                            int64_t ignore_index, float* __restrict__ row_loss) {
+    __shared__ Lse parts[kT / 64];
+    __shared__ float target;
+    const uint64_t row = blockIdx.x;
+    typename El::S* x = logits + row * ld;
+    const int64_t y = labels[row];
+    const RowKind kind = row_kind(y, ignore_index, vocab);
+    if (kind != kValid) {
+        const float f = kind == kIgnored ? 0.0f : __builtin_nanf("");
+        for (uint32_t i = threadIdx.x; i < vocab; i += kT) El::store(x + i, f);
+        if (threadIdx.x == 0) row_loss[row] = f;
+        return;
+    }
+    if (threadIdx.x == 0) target = El::load(x + y);
+    constexpr int kU = 4;
+    Lse p = {-__builtin_inff(), 0.0f};
+    for (uint32_t i = threadIdx.x; i < vocab; i += kT * kU) {
+        float f[kU];
+#pragma unroll
+        for (int k = 0; k < kU; ++k) f[k] = i + k * kT < vocab ? El::load(x + i + k * kT) : -__builtin_inff();
+        float m = p.m;
+#pragma unroll
+        for (int k = 0; k < kU; ++k) m = fmaxf(m, f[k]);
+        const float c = base(m);
+        float s = p.s == 0.0f ? 0.0f : p.s * El::exp(base(p.m) - c);
+#pragma unroll
+        for (int k = 0; k < kU; ++k) s += El::exp(f[k] - c);
+        p = {m, s};
+    }
+    const float lse = block_lse<kT>(p, parts);
+    if (threadIdx.x == 0) row_loss[row] = lse - target;
+    for (uint32_t i = threadIdx.x; i < vocab; i += kT) {
+        const float q = El::exp(El::load(x + i) - lse);
+        El::store(x + i, int64_t(i) == y ? q - 1.0f : q);
+    }
+}
+
+// Mean of the rows' losses and the number of rows it is taken over: one
+// workgroup, each row once, in an order fixed by n alone.
+constexpr int kLossThreads = 1024;
+__global__ __launch_bounds__(kLossThreads) void ce_loss_kernel(const float* __restrict__ row_loss,
+                                                               const int64_t* __restrict__ labels, uint64_t n,
+                                                               int64_t ignore_index, float* __restrict__ loss,
+                                                               float* __restrict__ n_valid) {
+    __shared__ double ssum[kLossThreads / 64];
+    __shared__ double scnt[kLossThreads / 64];
+    double sum = 0.0, cnt = 0.0;
+    for (uint64_t i = threadIdx.x; i < n; i += kLossThreads) {
+        sum += double(row_loss[i]);
+        cnt += labels[i] != ignore_index ? 1.0 : 0.0;
+    }
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) {
+        sum += __shfl_xor(sum, d);
+        cnt += __shfl_xor(cnt, d);
+    }
+    if ((threadIdx.x & 63) == 0) {
+        ssum[threadIdx.x >> 6] = sum;
+        scnt[threadIdx.x >> 6] = cnt;
+    }
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    for (int w = 1; w < kLossThreads / 64; ++w) {
+        sum += ssum[w];
+        cnt += scnt[w];
+    }
+    *loss = float(sum / cnt);
+    *n_valid = float(cnt);
+}
+
+// out = in * (grad_loss / n_valid) for both gradients in one launch: the
+// hidden gradient (n_h elements) and the fp32 weight gradient (n_w), each
+// rounded once into the output type.  Streaming, 8 elements per lane, one
+// group per lane as the staging cast; the weight's groups come first.
+constexpr int kScaleThreads = 128;
+template <typename Fmt>
+__device__ __forceinline__ u32x4 pack8(const f32x4 a, const f32x4 b) {
+    return u32x4{Fmt::pack(a.x, a.y), Fmt::pack(a.z, a.w), Fmt::pack(b.x, b.y), Fmt::pack(b.z, b.w)};
+}
+
+template <typename Fmt>
+__global__ __launch_bounds__(kScaleThreads) void ce_scale16_kernel(
+    const float* __restrict__ grad_loss, const float* __restrict__ n_valid, const uint16_t* __restrict__ h,
+    uint16_t* __restrict__ h_out, uint64_t n_h, const float* __restrict__ w, uint16_t* __restrict__ w_out,
+    uint64_t n_w, uint64_t w_blocks) {
+    const float scale = *grad_loss / *n_valid;
+    if (blockIdx.x < w_blocks) {
+        const uint64_t i = (uint64_t(blockIdx.x) * kScaleThreads + threadIdx.x) * kGroup;
+        if (i + kGroup <= n_w) {
+            const f32x4* p = reinterpret_cast<const f32x4*>(w + i);
+            const f32x4 a = __builtin_nontemporal_load(p), b = __builtin_nontemporal_load(p + 1);
+            __builtin_nontemporal_store(pack8<Fmt>(a * scale, b * scale), reinterpret_cast<u32x4*>(w_out + i));
+        } else {
+            for (uint64_t j = i; j < n_w; ++j) w_out[j] = uint16_t(Fmt::pack(w[j] * scale, 0.0f));
+        }
+        return;
+    }
+    const uint64_t i = ((uint64_t(blockIdx.x) - w_blocks) * kScaleThreads + threadIdx.x) * kGroup;
+    if (i + kGroup <= n_h) {
+        const u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(h + i));
+        u32x4 o;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) o[j] = Fmt::pack(Fmt::lo(v[j]) * scale, Fmt::hi(v[j]) * scale);
+        __builtin_nontemporal_store(o, reinterpret_cast<u32x4*>(h_out + i));
+    } else {
+        for (uint64_t j = i; j < n_h; ++j) h_out[j] = uint16_t(Fmt::pack(Fmt::lo(h[j]) * scale, 0.0f));
+    }
+}
+
+__global__ __launch_bounds__(kScaleThreads) void ce_scale32_kernel(
+    const float* __restrict__ grad_loss, const float* __restrict__ n_valid, const float* __restrict__ h,
+    float* __restrict__ h_out, uint64_t n_h, const float* __restrict__ w, float* __restrict__ w_out, uint64_t n_w,
+    uint64_t w_blocks) {
+    const float scale = *grad_loss / *n_valid;
+    const bool is_w = blockIdx.x < w_blocks;
+    const float* src = is_w ? w : h;
+    float* dst = is_w ? w_out : h_out;
+    const uint64_t n = is_w ? n_w : n_h;
+    const uint64_t b = is_w ? blockIdx.x : uint64_t(blockIdx.x) - w_blocks;
+    const uint64_t i = (b * kScaleThreads + threadIdx.x) * kGroup;
+    for (uint64_t j = i; j < n && j < i + kGroup; ++j) dst[j] = src[j] * scale;
+}
+
+inline int status() {
+    // the runtime keeps a failed launch as the thread's last error: reading it clears it
+    return int(hipGetLastError());
+}
+
+inline bool misaligned(const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) != 0; }
+
+template <typename Fmt, int kT, int kG, int kFull>
+void launch_rows(uint16_t* x, uint64_t ld, uint64_t rows, uint32_t vocab, const int64_t* labels, int64_t ignore,
+                 float* row_loss, hipStream_t st) {
+    hipLaunchKernelGGL((ce_rows_kernel<Fmt, kT, kG, kFull>), dim3(uint32_t(rows)), dim3(kT), 0, st, x, ld, vocab, labels,
+                       ignore, row_loss);
+}
+
+// The smallest workgroup that holds the row: lanes first (up to 1024), then
+// groups per lane, so that short rows keep many workgroups per CU and long
+// ones all their loads in flight at once.
+template <typename Fmt>
+void dispatch_rows16(uint16_t* x, uint64_t ld, uint64_t rows, uint32_t vocab, const int64_t* labels, int64_t ignore,
+                     float* row_loss, hipStream_t st) {
+    const uint32_t groups = (vocab + kGroup - 1) / kGroup;
+    // (lanes, groups per lane, of them full: what the line above could not hold)
+#define SF_ROWS(T, G, FULL)                                                                 \
+    if (groups <= uint32_t(T) * G) {                                                        \
+        launch_rows<Fmt, T, G, FULL>(x, ld, rows, vocab, labels, ignore, row_loss, st);     \
+        return;                                                                             \
+    }
+    SF_ROWS(64, 2, 0)
+    SF_ROWS(256, 2, 0)
+    SF_ROWS(256, 4, 2)
+    SF_ROWS(512, 4, 2)
+    SF_ROWS(1024, 4, 2)
+    SF_ROWS(1024, 8, 4)
+    SF_ROWS(1024, 12, 8)
+    SF_ROWS(1024, 16, 12)
+    SF_ROWS(1024, 19, 16)
+#undef SF_ROWS
+    hipLaunchKernelGGL((ce_rows_stream_kernel<Elem16<Fmt>, 1024>), dim3(uint32_t(rows)), dim3(1024), 0, st, x, ld,
+                       vocab, labels, ignore, row_loss);
+}
+
+}  // namespace
+
+extern "C" {
+
+int sf_ce_rows(void* logits, int dtype, size_t ld, size_t rows, size_t vocab, const int64_t* labels,
+               int64_t ignore_index, float* row_loss, sf_stream_t stream) {
+    if (rows == 0) return SF_OK;
+    if (logits == nullptr || labels == nullptr || row_loss == nullptr) return SF_EINVAL;
+    if (vocab == 0 || vocab > (size_t(1) << 31) || rows >= (size_t(1) << 31) || ld < vocab) return SF_EINVAL;
+    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    if (dtype == SF_DTYPE_F32) {
+        if (misaligned(logits, 4)) return SF_EINVAL;
+        hipLaunchKernelGGL((ce_rows_stream_kernel<Elem32, 1024>), dim3(uint32_t(rows)), dim3(1024), 0, st,
+                           static_cast<float*>(logits), uint64_t(ld), uint32_t(vocab), labels, ignore_index,
+                           row_loss);
+        return status();
+    }
+    if (dtype != SF_DTYPE_BF16 && dtype != SF_DTYPE_F16) return SF_EDTYPE;
+    // whole 128-bit groups: every row starts on one and its last one is inside the row's ld elements
+    if (misaligned(logits, 16) || ld % kGroup != 0) return SF_EALIGN;
+    uint16_t* x = static_cast<uint16_t*>(logits);
+    if (dtype == SF_DTYPE_BF16)
+        dispatch_rows16<Bf16>(x, ld, rows, uint32_t(vocab), labels, ignore_index, row_loss, st);
+    else
+        dispatch_rows16<F16>(x, ld, rows, uint32_t(vocab), labels, ignore_index, row_loss, st);
+    return status();
+}
+
+int sf_ce_loss(const float* row_loss, const int64_t* labels, size_t n, int64_t ignore_index, float* loss,
+               float* n_valid, sf_stream_t stream) {
+    if (loss == nullptr || n_valid == nullptr || (n > 0 && (row_loss == nullptr || labels == nullptr)))
+        return SF_EINVAL;
+    hipLaunchKernelGGL(ce_loss_kernel, dim3(1), dim3(kLossThreads), 0, reinterpret_cast<hipStream_t>(stream),
+                       row_loss, labels, uint64_t(n), ignore_index, loss, n_valid);
+    return status();
+}
+
+int sf_ce_scale(const float* grad_loss, const float* n_valid, const void* grad_h, void* grad_h_out, size_t n_h,
+                const float* grad_w, void* grad_w_out, size_t n_w, int dtype, sf_stream_t stream) {
+    if (n_h == 0 && n_w == 0) return SF_OK;
+    if (grad_loss == nullptr || n_valid == nullptr) return SF_EINVAL;
+    if ((n_h > 0 && (grad_h == nullptr || grad_h_out == nullptr)) ||
+        (n_w > 0 && (grad_w == nullptr || grad_w_out == nullptr)))
+        return SF_EINVAL;
+    if (misaligned(grad_h, 16) || misaligned(grad_h_out, 16) || misaligned(grad_w, 16) || misaligned(grad_w_out, 16))
+        return SF_EALIGN;
+    constexpr uint64_t kPer = uint64_t(kScaleThreads) * kGroup;
+    const uint64_t wb = (n_w + kPer - 1) / kPer, hb = (n_h + kPer - 1) / kPer;
+    if (wb + hb > ((uint64_t(1) << 31) / kScaleThreads)) return SF_EINVAL;
+    const dim3 grid(uint32_t(wb + hb)), block(kScaleThreads);
+    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    if (dtype == SF_DTYPE_F32) {
+        hipLaunchKernelGGL(ce_scale32_kernel, grid, block, 0, st, grad_loss, n_valid,
+                           static_cast<const float*>(grad_h), static_cast<float*>(grad_h_out), uint64_t(n_h), grad_w,
+                           static_cast<float*>(grad_w_out), uint64_t(n_w), wb);
+    } else if (dtype == SF_DTYPE_BF16) {
+        hipLaunchKernelGGL(ce_scale16_kernel<Bf16>, grid, block, 0, st, grad_loss, n_valid,
+                           static_cast<const uint16_t*>(grad_h), static_cast<uint16_t*>(grad_h_out), uint64_t(n_h),
+                           grad_w, static_cast<uint16_t*>(grad_w_out), uint64_t(n_w), wb);
+    } else if (dtype == SF_DTYPE_F16) {
+        hipLaunchKernelGGL(ce_scale16_kernel<F16>, grid, block, 0, st, grad_loss, n_valid,
+                           static_cast<const uint16_t*>(grad_h), static_cast<uint16_t*>(grad_h_out), uint64_t(n_h),
+                           grad_w, static_cast<uint16_t*>(grad_w_out), uint64_t(n_w), wb);
+    } else {
+        return SF_EDTYPE;
+    }
+    return status();
+}
+
+}  // extern "C"

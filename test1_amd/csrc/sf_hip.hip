@@ -460,6 +460,7 @@ const char* sf_error_string(int status) {
         case SF_EDTYPE: return "sf: dtype combination not supported";
         case SF_ENOOPT: return "sf: unknown optimizer id";
         case SF_EOVERLAP: return "sf: source and destination overlap";
+        case SF_EALIGN: return "sf: array not aligned as the entry point requires";
         case SF_ETOOBIG: return "sf: piece larger than the library's device scratch (SF_STAGE_SCRATCH_ELEMS)";
         case SF_ETIMEDOUT: return "sf: wait ended at its deadline with work still pending";
         default:

@@ -6,25 +6,128 @@ The reference's output unit uses a fused linear-cross-entropy kernel when one
 is installed (slide_fsdp.py:57-63, 85-97: ``LigerFusedLinearCrossEntropyLoss``,
 mean reduction, no logits returned) and full logits + ``nn.CrossEntropyLoss``
 otherwise.  This is the fused variant built from hipBLASLt GEMMs: rows are
-processed in chunks of ``chunk_rows``; for each chunk the logits are formed in
-fp32, the chunk's loss terms are summed, and since the step's backward follows
-at once, the gradients with respect to the hidden rows and the weight are
-formed right away from ``softmax - onehot`` (as the fused kernel does) and
-only scaled in the backward.  Peak extra memory is one chunk of fp32 logits
-plus an fp32 weight-gradient accumulator, instead of the [N, V] logits in bf16
-and fp32 and their gradient.
+processed in chunks of ``chunk_rows``; for each chunk the logits are formed,
+one kernel (``csrc/sf_ce.hip``) turns them into the chunk's loss terms and, in
+place, into ``softmax - onehot``, and since the step's backward follows at
+once, the gradients with respect to the hidden rows and the weight are formed
+right away (as the fused kernel does) and only scaled in the backward.  Peak
+extra memory is one chunk of logits plus an fp32 weight gradient, instead of
+the [N, V] logits in bf16 and fp32 and their gradient.
 
 Numerics: logsumexp, softmax and the loss are fp32; the logits are the bf16
 GEMM's output widened, as ``nn.CrossEntropyLoss`` on bf16 logits sees them;
 the gradient of the logits is rounded to bf16 for the two gradient GEMMs and
-the weight gradient is accumulated over chunks in fp32.  Rows whose label is
-``ignore_index`` contribute nothing; the mean is over the other rows (NaN if
-there are none, as ``nn.CrossEntropyLoss``).
+the weight gradient stays in fp32 until the backward has scaled it.  Rows whose
+label is ``ignore_index`` contribute nothing; the mean is over the other rows
+(NaN if there are none, as ``nn.CrossEntropyLoss``).
+
+On a host, and for inputs the kernels do not take (``_kernels_take``), the
+same steps run as torch operations.
 """
 
 from __future__ import annotations
 
 import torch
+
+from . import kernels
+
+
+_DTYPES = (torch.bfloat16, torch.float16, torch.float32)
+
+
+def _kernels_take(hidden: torch.Tensor, weight: torch.Tensor, labels: torch.Tensor) -> bool:
+    """Inputs the HIP kernels run on: one GPU, one float type, int64 labels, at
+    least one row.  Left to torch: what its operations refuse by themselves
+    (mixed types or devices, other label types), the empty cases, autocast to
+    another type (it would round the products), a traced call (the kernels are
+    called through pointers), and tensor subclasses."""
+    return (hidden.device.type == "cuda" and weight.device == hidden.device and labels.device == hidden.device
+            and hidden.dtype in _DTYPES and weight.dtype == hidden.dtype and labels.dtype == torch.int64
+            and hidden.numel() > 0 and weight.numel() > 0 and weight.shape[0] < 1 << 31
+            and hidden.shape[0] < 1 << 31
+            and not (torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != hidden.dtype)
+            and not torch.compiler.is_compiling()
+            and all(type(t) in (torch.Tensor, torch.nn.Parameter) for t in (hidden, weight, labels)))
+
+
+def auto_chunk_rows(vocab: int, hidden_size: int, element_size: int) -> int:
+    """Rows per chunk when the caller names none.  One chunk where possible:
+    the products run at 0.80-1.47 PFLOP/s on 523 rows against 4092 (hidden
+    4096, vocabulary 128256), and every chunk after the first reads and writes
+    the whole fp32 weight gradient again.  The chunk of logits may take what a
+    16-bit product of the weight gradient's size would (``hidden_size`` rows
+    of it), and at least 384 MiB (fp32: 256 MiB): with that the call's peak is
+    no higher than with chunks of 256 MiB of fp32 logits, their 16-bit copy
+    and that product beside the accumulator."""
+    least = (384 << 20) // (2 * vocab) if element_size == 2 else (256 << 20) // (4 * vocab)
+    return max(1, hidden_size, least)
+
+
+def _forward_kernels(ctx, hidden: torch.Tensor, weight: torch.Tensor, labels: torch.Tensor, ignore_index: int,
+                     chunk_rows: int) -> torch.Tensor:
+    n, h = hidden.shape
+    v = weight.shape[0]
+    dev = hidden.device
+    labels = labels.contiguous()
+    grad_hidden = torch.empty((n, h), dtype=hidden.dtype, device=dev)
+    grad_weight = torch.empty((v, h), dtype=torch.float32, device=dev)
+    row_loss = torch.empty(n, dtype=torch.float32, device=dev)
+    loss = torch.empty((), dtype=torch.float32, device=dev)
+    n_valid = torch.empty((), dtype=torch.float32, device=dev)
+    step = max(1, min(n, int(chunk_rows)))
+    # Rows 128 bytes apart or a multiple of it: the kernel's 128-bit accesses
+    # and the products' operand loads stay aligned for any vocabulary.
+    ld = -(-v // 64) * 64
+    buf = torch.empty((step, ld), dtype=hidden.dtype, device=dev)
+    wt = weight.t()
+    f32_out = {} if hidden.dtype == torch.float32 else dict(out_dtype=torch.float32)
+    for s in range(0, n, step):
+        e = min(n, s + step)
+        hc = hidden[s:e]
+        g = buf[:e - s, :v]
+        torch.mm(hc, wt, out=g)
+        kernels.ce_rows_(g, labels[s:e], ignore_index, row_loss[s:e])
+        torch.mm(g, weight, out=grad_hidden[s:e])
+        if s == 0:
+            torch.mm(g.t(), hc, **f32_out, out=grad_weight)
+        else:
+            torch.addmm(grad_weight, g.t(), hc, **f32_out, out=grad_weight)
+    kernels.ce_loss(row_loss, labels, ignore_index, loss, n_valid)
+    ctx.save_for_backward(grad_hidden, grad_weight, n_valid)
+    return loss
+
+
+def _forward_torch(ctx, hidden: torch.Tensor, weight: torch.Tensor, labels: torch.Tensor, ignore_index: int,
+                   chunk_rows: int) -> torch.Tensor:
+    n, h = hidden.shape
+    v = weight.shape[0]
+    dev = hidden.device
+    grad_hidden = torch.empty_like(hidden)
+    grad_weight = torch.zeros((v, h), dtype=torch.float32, device=dev)
+    loss_sum = torch.zeros((), dtype=torch.float32, device=dev)
+    valid_all = labels != ignore_index
+    n_valid = valid_all.sum().to(torch.float32)
+    wt = weight.t()
+    for s in range(0, n, max(1, int(chunk_rows))):
+        e = min(n, s + int(chunk_rows))
+        hc = hidden[s:e]
+        yc = labels[s:e]
+        valid = valid_all[s:e]
+        ysafe = torch.where(valid, yc, torch.zeros_like(yc))
+        logits = torch.mm(hc, wt).float()                       # [C, V], widened bf16 GEMM output
+        lse = torch.logsumexp(logits, dim=1)
+        target = logits.gather(1, ysafe.unsqueeze(1)).squeeze(1)
+        loss_sum += torch.where(valid, lse - target, torch.zeros_like(lse)).sum()
+        logits.sub_(lse.unsqueeze(1)).exp_()                    # softmax, in place
+        rows = torch.arange(e - s, device=dev)
+        logits[rows, ysafe] -= 1.0                              # - onehot
+        logits.mul_(valid.unsqueeze(1).to(logits.dtype))        # ignored rows: no gradient
+        g = logits.to(hidden.dtype)
+        del logits
+        grad_hidden[s:e] = torch.mm(g, weight)
+        grad_weight.add_(torch.mm(g.t(), hc))
+    ctx.save_for_backward(grad_hidden, grad_weight, n_valid)
+    return loss_sum / n_valid
 
 
 class ChunkedLinearCrossEntropy(torch.autograd.Function):
@@ -35,40 +138,28 @@ class ChunkedLinearCrossEntropy(torch.autograd.Function):
             raise ValueError("chunked linear cross entropy: hidden [N, H] and weight [V, H] expected")
         if labels.shape != hidden.shape[:1]:
             raise ValueError("chunked linear cross entropy: one label per hidden row expected")
-        n, h = hidden.shape
-        v = weight.shape[0]
-        dev = hidden.device
-        grad_hidden = torch.empty_like(hidden)
-        grad_weight = torch.zeros((v, h), dtype=torch.float32, device=dev)
-        loss_sum = torch.zeros((), dtype=torch.float32, device=dev)
-        valid_all = labels != ignore_index
-        n_valid = valid_all.sum().to(torch.float32)
-        wt = weight.t()
-        for s in range(0, n, max(1, int(chunk_rows))):
-            e = min(n, s + int(chunk_rows))
-            hc = hidden[s:e]
-            yc = labels[s:e]
-            valid = valid_all[s:e]
-            ysafe = torch.where(valid, yc, torch.zeros_like(yc))
-            logits = torch.mm(hc, wt).float()                       # [C, V], widened bf16 GEMM output
-            lse = torch.logsumexp(logits, dim=1)
-            target = logits.gather(1, ysafe.unsqueeze(1)).squeeze(1)
-            loss_sum += torch.where(valid, lse - target, torch.zeros_like(lse)).sum()
-            logits.sub_(lse.unsqueeze(1)).exp_()                    # softmax, in place
-            rows = torch.arange(e - s, device=dev)
-            logits[rows, ysafe] -= 1.0                              # - onehot
-            logits.mul_(valid.unsqueeze(1).to(logits.dtype))        # ignored rows: no gradient
-            g = logits.to(hidden.dtype)
-            del logits
-            grad_hidden[s:e] = torch.mm(g, weight)
-            grad_weight.add_(torch.mm(g.t(), hc))
-        ctx.save_for_backward(grad_hidden, grad_weight, n_valid)
         ctx.weight_dtype = weight.dtype
-        return loss_sum / n_valid
+        if not _kernels_take(hidden, weight, labels):
+            return _forward_torch(ctx, hidden, weight, labels, ignore_index, chunk_rows)
+        with torch.cuda.device(hidden.device):
+            return _forward_kernels(ctx, hidden, weight, labels, ignore_index, chunk_rows)
 
     @staticmethod
     def backward(ctx, grad_loss: torch.Tensor):
         grad_hidden, grad_weight, n_valid = ctx.saved_tensors
+        # The kernel takes what the forward saved, unless hooks brought it back
+        # otherwise or the backward itself is differentiated.
+        if (grad_hidden.device.type == "cuda" and grad_weight.device == grad_hidden.device == n_valid.device
+                and grad_hidden.dtype == ctx.weight_dtype and grad_hidden.numel() > 0 and grad_weight.numel() > 0
+                and grad_hidden.is_contiguous() and grad_weight.is_contiguous()
+                and grad_loss.device == n_valid.device and grad_loss.dtype == torch.float32
+                and not (torch.is_grad_enabled() and grad_loss.requires_grad)
+                and not torch.compiler.is_compiling()
+                and all(type(t) is torch.Tensor for t in (grad_loss, grad_hidden, grad_weight, n_valid))
+                and grad_hidden.dtype in _DTYPES
+                and grad_hidden.data_ptr() % 16 == 0 and grad_weight.data_ptr() % 16 == 0):
+            with torch.cuda.device(grad_hidden.device):
+                return (*kernels.ce_scale(grad_loss, n_valid, grad_hidden, grad_weight), None, None, None)
         scale = (grad_loss.to(torch.float32) / n_valid)
         gh = (grad_hidden.to(torch.float32) * scale).to(grad_hidden.dtype)
         gw = (grad_weight * scale).to(ctx.weight_dtype)
@@ -78,7 +169,11 @@ class ChunkedLinearCrossEntropy(torch.autograd.Function):
 def chunked_linear_cross_entropy(hidden: torch.Tensor, weight: torch.Tensor, labels: torch.Tensor,
                                  ignore_index: int = -100, chunk_rows: int = 0) -> torch.Tensor:
     """Mean cross entropy of ``hidden @ weight.T`` against ``labels``.
-    ``chunk_rows`` <= 0 picks chunks of ~256 MiB of fp32 logits."""
+    ``chunk_rows`` <= 0 picks the chunks (``auto_chunk_rows`` on a GPU, else
+    ~256 MiB of fp32 logits)."""
     if chunk_rows <= 0:
-        chunk_rows = max(1, (256 << 20) // (4 * weight.shape[0]))
+        if hidden.dim() == 2 and _kernels_take(hidden, weight, labels):
+            chunk_rows = auto_chunk_rows(weight.shape[0], weight.shape[-1], hidden.element_size())
+        else:
+            chunk_rows = max(1, (256 << 20) // (4 * weight.shape[0]))
     return ChunkedLinearCrossEntropy.apply(hidden, weight, labels, int(ignore_index), int(chunk_rows))

@@ -301,6 +301,74 @@ def gather_rows(table: torch.Tensor, ids: torch.Tensor, dst: torch.Tensor, bad: 
     return dst
 
 
+_CE_DTYPES = {torch.float32: _native.SF_DTYPE_F32, torch.bfloat16: _native.SF_DTYPE_BF16,
+              torch.float16: _native.SF_DTYPE_F16}
+
+
+def ce_rows_(logits: torch.Tensor, labels: torch.Tensor, ignore_index: int, row_loss: torch.Tensor,
+             stream: Optional[torch.cuda.Stream] = None) -> None:
+    """``row_loss[r] = logsumexp(logits[r]) - logits[r, labels[r]]`` and
+    ``logits[r] = softmax(logits[r]) - onehot(labels[r])`` in place (0 and zeros
+    for an ignored row, NaN for a label outside the vocabulary).
+
+    ``logits`` is 2-D with unit column stride (16-bit: rows on 16-byte
+    boundaries; what lies between its rows is overwritten), ``labels`` int64
+    and ``row_loss`` float32, contiguous, one per row."""
+    if logits.dtype not in _CE_DTYPES or labels.dtype != torch.int64 or row_loss.dtype != torch.float32:
+        raise TypeError("ce_rows_: need float logits, int64 labels and a float32 row_loss")
+    if logits.dim() != 2 or (logits.shape[1] > 1 and logits.stride(1) != 1):
+        raise ValueError("ce_rows_: logits must be 2-D with unit column stride")
+    rows, vocab = logits.shape
+    if labels.shape != (rows,) or row_loss.shape != (rows,):
+        raise ValueError("ce_rows_: one label and one row_loss element per row expected")
+    for t, what in ((logits, "logits"), (labels, "labels"), (row_loss, "row_loss")):
+        _require_cuda(t, what)
+    _require_contig(labels, "labels")
+    _require_contig(row_loss, "row_loss")
+    ld = logits.stride(0) if rows > 1 else max(logits.stride(0), -(-vocab // 8) * 8)
+    # the last row's groups of 8 end inside the storage
+    room = logits.untyped_storage().nbytes() // logits.element_size() - logits.storage_offset()
+    if rows > 0 and (ld < vocab or room < (rows - 1) * ld + (-(-vocab // 8) * 8 if logits.element_size() == 2 else vocab)):
+        raise ValueError("ce_rows_: the rows overlap or end outside the storage")
+    _native.check(_native.hip().sf_ce_rows(logits.data_ptr(), _CE_DTYPES[logits.dtype], ld, rows, vocab,
+                                           labels.data_ptr(), int(ignore_index), row_loss.data_ptr(),
+                                           _stream_ptr(stream)), "sf_ce_rows")
+
+
+def ce_loss(row_loss: torch.Tensor, labels: torch.Tensor, ignore_index: int, loss: torch.Tensor,
+            n_valid: torch.Tensor, stream: Optional[torch.cuda.Stream] = None) -> None:
+    """``n_valid`` = labels that are not ``ignore_index``, ``loss`` = sum of
+    ``row_loss`` over it; both float32 GPU tensors of one element."""
+    for t, what in ((row_loss, "row_loss"), (labels, "labels"), (loss, "loss"), (n_valid, "n_valid")):
+        _require_cuda(t, what)
+        _require_contig(t, what)
+    if labels.dtype != torch.int64 or any(t.dtype != torch.float32 for t in (row_loss, loss, n_valid)):
+        raise TypeError("ce_loss: need int64 labels and float32 row_loss, loss and n_valid")
+    if row_loss.numel() != labels.numel() or loss.numel() != 1 or n_valid.numel() != 1:
+        raise ValueError("ce_loss: one row_loss per label and one-element results expected")
+    _native.check(_native.hip().sf_ce_loss(row_loss.data_ptr(), labels.data_ptr(), labels.numel(), int(ignore_index),
+                                           loss.data_ptr(), n_valid.data_ptr(), _stream_ptr(stream)), "sf_ce_loss")
+
+
+def ce_scale(grad_loss: torch.Tensor, n_valid: torch.Tensor, grad_h: torch.Tensor, grad_w: torch.Tensor,
+             stream: Optional[torch.cuda.Stream] = None) -> Tuple[torch.Tensor, torch.Tensor]:
+    """``grad_h`` and the float32 ``grad_w`` times ``grad_loss / n_valid``, both in ``grad_h``'s dtype."""
+    if grad_h.dtype not in _CE_DTYPES or any(t.dtype != torch.float32 for t in (grad_loss, n_valid, grad_w)):
+        raise TypeError("ce_scale: need a float grad_h and float32 grad_loss, n_valid and grad_w")
+    if grad_loss.numel() != 1 or n_valid.numel() != 1:
+        raise ValueError("ce_scale: one-element grad_loss and n_valid expected")
+    for t, what in ((grad_loss, "grad_loss"), (n_valid, "n_valid"), (grad_h, "grad_h"), (grad_w, "grad_w")):
+        _require_cuda(t, what)
+    _require_contig(grad_h, "grad_h")
+    _require_contig(grad_w, "grad_w")
+    gh = torch.empty_like(grad_h)
+    gw = torch.empty(grad_w.shape, dtype=grad_h.dtype, device=grad_w.device)
+    _native.check(_native.hip().sf_ce_scale(grad_loss.data_ptr(), n_valid.data_ptr(), grad_h.data_ptr(), gh.data_ptr(),
+                                            gh.numel(), grad_w.data_ptr(), gw.data_ptr(), gw.numel(),
+                                            _CE_DTYPES[grad_h.dtype], _stream_ptr(stream)), "sf_ce_scale")
+    return gh, gw
+
+
 def memcpy_async(dst: torch.Tensor, src: torch.Tensor, stream: Optional[torch.cuda.Stream] = None,
                  nbytes: Optional[int] = None) -> None:
     """Asynchronous byte copy between contiguous tensors on ``stream``.

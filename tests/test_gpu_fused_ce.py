@@ -1,0 +1,184 @@
+"""The cross-entropy kernels of the fused output unit, against float64."""
+
+import pytest
+import torch
+
+from test1_amd import fused_ce, kernels
+from test1_amd.fused_ce import chunked_linear_cross_entropy
+
+pytestmark = pytest.mark.gpu
+
+# Rounding of one result to the type, relative and absolute: half a unit in the
+# last of 8, 11 or 24 significant bits is at most 2^-8, 2^-11 or 2^-24 of the
+# value; below the normal range it is half the smallest subnormal.
+EPS = {torch.bfloat16: (2.0 ** -8, 2.0 ** -134), torch.float16: (2.0 ** -11, 2.0 ** -25),
+       torch.float32: (2.0 ** -24, 2.0 ** -126)}
+# vocabularies at the edges of every workgroup shape (64 x 16, 256 x 16, 256 x 32,
+# 512 x 32, 1024 x 32, x 64, x 96, x 128, x 152 elements, then the streaming kernel)
+EDGES = [1, 7, 8, 9, 1024, 1025, 4096, 4097, 8192, 8195, 16384, 16391, 32768, 32769, 65536, 65537, 98304, 98312,
+         131072, 131079, 155648, 155649, 160001]
+
+
+def rows_reference(x, y, ignore_index=-100):
+    """(row_loss, gradient) in float64."""
+    x = x.double()
+    lse = torch.logsumexp(x, dim=1)
+    ys = y.clamp(0, x.shape[1] - 1).unsqueeze(1)
+    loss = lse - x.gather(1, ys).squeeze(1)
+    g = torch.exp(x - lse.unsqueeze(1))
+    p = g.clone()
+    g.scatter_add_(1, ys, -torch.ones_like(ys, dtype=g.dtype))
+    ignored = y == ignore_index
+    loss[ignored] = 0.0
+    g[ignored] = 0.0
+    return loss, g, p
+
+
+def strided(rows, vocab, dtype, dev):
+    return torch.empty(rows, -(-vocab // 64) * 64, dtype=dtype, device=dev)[:, :vocab]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("vocab", EDGES)
+def test_rows_match_float64(dev, vocab, dtype):
+    rows = 5
+    gen = torch.Generator(device=dev).manual_seed(vocab)
+    x = (torch.randn(rows, vocab, generator=gen, device=dev) * 3).to(dtype)
+    y = torch.randint(0, vocab, (rows,), generator=gen, device=dev)
+    y[0], y[1], y[2] = 0, vocab - 1, -100
+    ref_loss, ref_g, p = rows_reference(x, y)
+    got = strided(rows, vocab, dtype, dev)
+    got.copy_(x)
+    loss = torch.full((rows,), 7.0, device=dev)
+    kernels.ce_rows_(got, y, -100, loss)
+    torch.cuda.synchronize()
+    # fp32 terms: exp's argument is rounded at |x - lse| <= 40, twice
+    assert ((loss.double() - ref_loss).abs() <= 1e-6 * (4 + ref_loss.abs())).all()
+    half_ulp, tiny = EPS[dtype]
+    bound = half_ulp * ref_g.abs() + 6e-6 * p + tiny
+    assert ((got.double() - ref_g).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("vocab", [40, 70_003])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_rows_special_values(dev, vocab, dtype):
+    """Infinities and NaN give what logsumexp and softmax give; a label outside
+    the vocabulary gives NaN; an ignored row gives zeros whatever it holds."""
+    inf, nan = float("inf"), float("nan")
+    x = torch.randn(8, vocab, device=dev).to(dtype)
+    x[0, 3] = inf
+    x[1, 5] = nan
+    x[2] = -inf
+    x[3, 10:] = -inf          # most lanes see only -inf
+    x[4, 7] = nan
+    y = torch.tensor([1, 2, 3, 4, -100, vocab, -1, 6], device=dev)
+    ref_loss, ref_g, _ = rows_reference(x, y)
+    ref_loss[5:7] = nan
+    ref_g[5:7] = nan
+    got = strided(8, vocab, dtype, dev)
+    got.copy_(x)
+    loss = torch.empty(8, device=dev)
+    kernels.ce_rows_(got, y, -100, loss)
+    torch.testing.assert_close(loss.double(), ref_loss, rtol=1e-5, atol=1e-5, equal_nan=True)
+    torch.testing.assert_close(got.double(), ref_g, rtol=1e-2, atol=1e-5, equal_nan=True)
+
+
+def exact(h, w, y, scale):
+    h, w = h.detach().double().requires_grad_(True), w.detach().double().requires_grad_(True)
+    loss = torch.nn.functional.cross_entropy(h @ w.t(), y)
+    (scale * loss).backward()
+    return loss.detach(), h.grad, w.grad
+
+
+def rel(a, b):
+    return ((a.double() - b).norm() / b.norm()).item()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("n,h,v,chunk", [(1, 64, 16, 0), (300, 72, 1003, 128), (300, 72, 1003, 0), (65, 256, 32_001, 7),
+                                         (129, 512, 50_257, 0)])
+def test_loss_and_gradients_no_further_off_than_torch_operations(dev, monkeypatch, n, h, v, chunk, dtype):
+    """The kernels' loss and gradients against float64, beside those of the
+    same steps as torch operations: within the type's rounding, and no further
+    off (a tenth allowed: both round the same values in another order)."""
+    gen = torch.Generator(device=dev).manual_seed(n + v)
+    hid = torch.randn(n, h, generator=gen, device=dev).to(dtype)
+    wgt = (torch.randn(v, h, generator=gen, device=dev) * 0.05).to(dtype)
+    y = torch.randint(0, v, (n,), generator=gen, device=dev)
+    y[n - n // 8:] = -100
+
+    def run():
+        a, b = hid.clone().requires_grad_(True), wgt.clone().requires_grad_(True)
+        loss = chunked_linear_cross_entropy(a, b, y, chunk_rows=chunk)
+        (3.0 * loss).backward()
+        return loss.detach(), a.grad, b.grad
+
+    got = run()
+    monkeypatch.setattr(fused_ce, "_kernels_take", lambda *a: False)
+    plain = run()
+    ref = exact(hid, wgt, y, 3.0)
+    tol = {torch.bfloat16: 1e-2, torch.float16: 2e-3, torch.float32: 1e-5}[dtype]
+    for k, (a, p, r) in enumerate(zip(got, plain, ref)):
+        assert a.dtype == p.dtype and a.shape == p.shape
+        assert rel(a, r) <= tol, k
+        assert rel(a, r) <= 1.1 * rel(p, r) + 1e-6, k
+
+
+def test_strided_inputs_side_stream_and_repeated_backward(dev):
+    """Transposed hidden states and a strided weight on a side stream; the
+    saved gradients survive a second backward through the same loss."""
+    gen = torch.Generator(device=dev).manual_seed(2)
+    hid = torch.randn(96, 40, generator=gen, device=dev).bfloat16().t()           # [40, 96]
+    wgt = (torch.randn(501, 192, generator=gen, device=dev) * 0.05).bfloat16()[:, ::2]
+    y = torch.randint(0, 501, (80,), generator=gen, device=dev)[::2]
+    a, b = hid.detach().requires_grad_(True), wgt.detach().requires_grad_(True)
+    st = torch.cuda.Stream()
+    st.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(st):
+        loss = chunked_linear_cross_entropy(a, b, y)
+        g1 = torch.autograd.grad(loss, (a, b), retain_graph=True)
+        g2 = torch.autograd.grad(loss, (a, b))
+    st.synchronize()
+    ref = exact(hid, wgt, y, 1.0)
+    assert rel(loss, ref[0]) < 1e-3
+    for x1, x2, r in zip(g1, g2, ref[1:]):
+        assert torch.equal(x1, x2) and rel(x1, r) < 1e-2
+
+
+def test_all_rows_ignored_is_nan(dev):
+    w = torch.randn(32, 16, device=dev).bfloat16()
+    loss = chunked_linear_cross_entropy(torch.randn(4, 16, device=dev).bfloat16(), w,
+                                        torch.full((4,), -100, device=dev))
+    assert torch.isnan(loss)
+
+
+def test_loss_in_a_captured_graph(dev):
+    """Forward and backward captured; four replays with eager work between."""
+    gen = torch.Generator(device=dev).manual_seed(3)
+    hid = torch.randn(70, 64, generator=gen, device=dev).bfloat16().requires_grad_(True)
+    wgt = (torch.randn(900, 64, generator=gen, device=dev) * 0.05).bfloat16().requires_grad_(True)
+    y = torch.randint(0, 900, (70,), generator=gen, device=dev)
+
+    def step():
+        loss = chunked_linear_cross_entropy(hid, wgt, y, chunk_rows=32)
+        return (loss, *torch.autograd.grad(loss, (hid, wgt)))
+
+    want = [t.detach().clone() for t in step()]
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        step()
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = step()
+    for rep in range(4):
+        for t in out:
+            t.detach().fill_(float(rep + 7))
+        step()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        for t, w in zip(out, want):
+            assert torch.equal(t.detach(), w), rep
