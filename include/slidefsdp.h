@@ -169,7 +169,7 @@ int sf_cast_scatter_f32_bf16(const sf_seg* segs, int nsegs,
  * ------------------------------------------------------------------- */
 
 /* The segment-copy entry points below take max_workgroups: <= 0 launches
- * one workgroup per 8192-element tile (device-to-device work, all CUs);
+ * one workgroup per tile (device-to-device work, all CUs);
  * a positive value caps the grid, each workgroup then striding over tiles.
  * A capped grid is meant for a destination in pinned host memory (the
  * device address from sf_host_device_pointer), where a few dozen

@@ -32,12 +32,15 @@ constexpr int kUnroll = 4;     // 8-element groups per lane per workgroup tile
 constexpr int kCastUnroll = 1; // the same for the flat cast (measured best, see below)
 constexpr int kCastThreads = 128;  // lanes per workgroup of the flat cast (2 wave64s, see below)
 constexpr int kGroup = 8;      // elements per 128-bit bf16 store
-constexpr uint64_t kTileElems = uint64_t(kThreads) * kUnroll * kGroup;  // 8192
+constexpr uint64_t kSizeUnit = 8192;  // elements; a segment table's size limit is counted in these
 
 // Native vector types: the nontemporal builtins need them (HIP's float4 is a
 // struct), and they map one-to-one onto 128-bit global_load/store_dwordx4.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+// The same 128 bits at the alignment of one element: still one access.
+typedef f32x4 f32x4_any __attribute__((aligned(4)));
+typedef u32x4 u32x4_any __attribute__((aligned(2)));
 
 // fp32 -> bf16 with round-to-nearest-even on the bit pattern, NaN -> 0xFFFF.
 // This is the arithmetic of torch's vectorised CPU cast that the reference
@@ -289,10 +292,31 @@ __global__ __launch_bounds__(kThreads) void fill_b16_kernel(
 // ---------------------------------------------------------------------
 // Segment-table kernels.  The table travels in the kernel arguments
 // (about 2 KiB for SF_MAX_SEGS segments), so no device allocation is
-// needed.  Each workgroup owns one tile of kTileElems elements inside a
-// single segment: tiles are numbered across segments and tile_start[s]
-// is the first tile of segment s.  A workgroup finds its segment with a
-// binary search over tile_start, whose loads are uniform (scalar).
+// needed.  Each workgroup owns one tile of kTile elements inside a single
+// segment: tiles are numbered across segments and tile_start[s] is the first
+// tile of segment s.  A workgroup finds its segment with a binary search
+// over tile_start, whose loads are uniform (scalar).
+//
+// Bound by HBM (or, with a destination in host memory, by the host link).
+// Tiles and groups of 8 are laid out from the 16-byte boundary at or before
+// the segment's destination, so every store but those of a segment's two
+// ends is one aligned 128-bit access whatever the destination's alignment;
+// the source is loaded as 128-bit accesses too, at whatever alignment that
+// leaves it (the hardware takes any multiple of the element size; within 2 %
+// of aligned ones).  Elements of the partial groups at the two ends go one
+// by one.  Before, a segment with either side off a 16-byte boundary went
+// element by element: 61 tensors of odd sizes, 218 M elements in all, 257 ->
+// 132 us (copy, 6.1 TB/s) and 278 -> 205 us (cast); 8.4 M elements 14.9 ->
+// 9.5 us and 22.1 -> 12.0; packed into host memory 592 -> 327 us.
+//
+// Shape, 218 M elements aligned | 2.4 M | 8.4 M ragged, us: cast 64 lanes x 1
+// group per lane 207.9 | 5.4 | 12.3, 128 x 1 205.8 | 5.5 | 12.1, 256 x 1 211.0
+// | 5.2 | 12.0, 256 x 2 216.0 | 5.5 | 12.7, 256 x 4 (the shape before) 215.0 |
+// 6.2 | 14.1, 512 x 1 207.6 | 5.6 | 12.2; copy 256 x 1 144.1 | 4.2 | 9.5, 256
+// x 4 142.5 | 4.6 | 10.2.  Small tiles: few elements still fill the chip.  A
+// capped grid instead has few workgroups, each with kHostUnroll groups per
+// lane in flight: one layer into host memory with 16 workgroups of 256 x 8
+// 7802 us, 256 x 4 7926, 256 x 2 8062, 512 x 1 8145.
 // ---------------------------------------------------------------------
 struct SegTable {
     uint64_t src[SF_MAX_SEGS];
@@ -311,63 +335,83 @@ __device__ __forceinline__ uint32_t find_seg(const SegTable& t, uint64_t tile) {
     return lo;
 }
 
-// Element operations: fp32 -> bf16 cast, or 16-bit copy.
+// Elements between the 16-byte boundary at or before a 16-bit destination
+// and the destination itself (0 to 7).
+__host__ __device__ inline uint32_t lead_elems(uint64_t dst) { return uint32_t(dst & 15) >> 1; }
+
+// Element operations: fp32 -> bf16 cast, or 16-bit copy.  Raw is what a lane
+// holds of a group between its loads and its store.
 struct OpCast {
     using S = float;
-    __device__ static u32x4 load_convert(const S* p) {
-        const f32x4* q = reinterpret_cast<const f32x4*>(p);
-        return cast8(__builtin_nontemporal_load(q), __builtin_nontemporal_load(q + 1));
+    struct Raw {
+        f32x4 a, b;
+    };
+    __device__ static Raw load(const S* p) {
+        const f32x4_any* q = reinterpret_cast<const f32x4_any*>(p);
+        return {__builtin_nontemporal_load(q), __builtin_nontemporal_load(q + 1)};
     }
+    __device__ static u32x4 convert(const Raw& r) { return cast8(r.a, r.b); }
     __device__ static uint16_t convert1(S x) { return uint16_t(rne_bf16(__float_as_uint(x))); }
-    static constexpr uint64_t kAlign = 16;  // both sides need 16-byte alignment
 };
 
 struct OpCopy16 {
     using S = uint16_t;
-    __device__ static u32x4 load_convert(const S* p) {
-        return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
+    using Raw = u32x4;
+    __device__ static Raw load(const S* p) {
+        return __builtin_nontemporal_load(reinterpret_cast<const u32x4_any*>(p));
     }
+    __device__ static u32x4 convert(const Raw& r) { return r; }
     __device__ static uint16_t convert1(S x) { return x; }
-    static constexpr uint64_t kAlign = 16;
 };
 
+// One group of 8 at element offset e (a multiple of 8 from the boundary the
+// pointers start at) of a run occupying [lead, end): the whole group, or its
+// elements inside the run one by one.
 template <typename Op>
+__device__ __forceinline__ void move_group(const typename Op::S* src, uint16_t* dst, int64_t e, int64_t lead,
+                                           int64_t end) {
+    if (e >= lead && e + kGroup <= end) {
+        __builtin_nontemporal_store(Op::convert(Op::load(src + e)), reinterpret_cast<u32x4*>(dst + e));
+    } else {
+        for (int64_t j = e < lead ? lead : e; j < e + kGroup && j < end; ++j) dst[j] = Op::convert1(src[j]);
+    }
+}
+
+constexpr int kSegUnroll = 1;   // groups per lane and tile: one workgroup per tile
+constexpr int kHostUnroll = 8;  // the same for a capped grid
+
+template <typename Op, int kU>
 __global__ __launch_bounds__(kThreads) void seg_kernel(const SegTable t) {
     using S = typename Op::S;
+    constexpr int64_t kTile = int64_t(kThreads) * kU * kGroup;
     const uint64_t ntiles = t.tile_start[t.nsegs];
     // Grid-stride over tiles: one workgroup per tile when the grid covers
     // them all, or a capped grid (e.g. a copy into host memory, which only
     // needs enough workgroups to keep the host link busy).
     for (uint64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
         const uint32_t s = find_seg(t, tile);
-        const uint64_t first = (tile - t.tile_start[s]) * kTileElems;  // element offset in segment
-        const uint64_t n = t.n[s];
-        const uint64_t len = (n - first < kTileElems) ? (n - first) : kTileElems;
-        const S* src = reinterpret_cast<const S*>(t.src[s]) + first;
-        uint16_t* dst = reinterpret_cast<uint16_t*>(t.dst[s]) + first;
-
-        const bool aligned = ((reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(dst)) &
-                              (Op::kAlign - 1)) == 0;
-        if (aligned && len == kTileElems) {
-            // Full aligned tile: unpredicated loads, all in flight together.
-            u32x4 v[kUnroll];
+        const int64_t lead = lead_elems(t.dst[s]);
+        const int64_t end = int64_t(t.n[s]) + lead;
+        // from the boundary on: never dereferenced below `lead`
+        const S* src = reinterpret_cast<const S*>(t.src[s] - uint64_t(lead) * sizeof(S));
+        uint16_t* dst = reinterpret_cast<uint16_t*>(t.dst[s] - uint64_t(lead) * 2);
+        const int64_t first = int64_t(tile - t.tile_start[s]) * kTile;
+        if (((t.dst[s] & 1) | (t.src[s] & (sizeof(S) - 1))) != 0) {
+            // not aligned to its own elements: byte-exact element accesses
+            for (int64_t j = first + threadIdx.x; j < first + kTile && j < end; j += kThreads)
+                if (j >= lead) dst[j] = Op::convert1(src[j]);
+        } else if (first >= lead && first + kTile <= end) {
+            // Whole tile: unpredicated loads, all in flight together.
+            typename Op::Raw v[kU];
 #pragma unroll
-            for (int k = 0; k < kUnroll; ++k) v[k] = Op::load_convert(src + (k * kThreads + threadIdx.x) * kGroup);
+            for (int k = 0; k < kU; ++k) v[k] = Op::load(src + first + (k * kThreads + threadIdx.x) * kGroup);
 #pragma unroll
-            for (int k = 0; k < kUnroll; ++k)
-                __builtin_nontemporal_store(v[k], reinterpret_cast<u32x4*>(dst + (k * kThreads + threadIdx.x) * kGroup));
-        } else if (aligned) {
-            // Last tile of a segment: predicated groups, then the < 8 element tail.
-            const uint64_t n8 = len / kGroup;
-            for (int k = 0; k < kUnroll; ++k) {
-                const uint64_t g = k * kThreads + threadIdx.x;
-                if (g < n8) __builtin_nontemporal_store(Op::load_convert(src + g * kGroup),
-                                                        reinterpret_cast<u32x4*>(dst + g * kGroup));
-            }
-            const uint64_t rem = len - n8 * kGroup;
-            if (threadIdx.x < rem) dst[n8 * kGroup + threadIdx.x] = Op::convert1(src[n8 * kGroup + threadIdx.x]);
+            for (int k = 0; k < kU; ++k)
+                __builtin_nontemporal_store(Op::convert(v[k]),
+                                            reinterpret_cast<u32x4*>(dst + first + (k * kThreads + threadIdx.x) * kGroup));
         } else {
-            for (uint64_t i = threadIdx.x; i < len; i += kThreads) dst[i] = Op::convert1(src[i]);
+            for (int k = 0; k < kU; ++k)
+                move_group<Op>(src, dst, first + (k * kThreads + threadIdx.x) * kGroup, lead, end);
         }
     }
 }
@@ -381,31 +425,35 @@ constexpr uint64_t kMaxBlocks = (uint64_t(1) << 31) / kThreads;
 template <typename Op>
 int launch_segs(const sf_seg* segs, int nsegs, int max_workgroups, hipStream_t stream) {
     if (nsegs < 0 || (nsegs > 0 && segs == nullptr)) return SF_EINVAL;
+    const bool capped = max_workgroups > 0;
+    const uint64_t tile_elems = uint64_t(kThreads) * kGroup * (capped ? kHostUnroll : kSegUnroll);
     // Tables longer than SF_MAX_SEGS are split into several launches.
     for (int base = 0; base < nsegs; base += SF_MAX_SEGS) {
         const int cnt = (nsegs - base < SF_MAX_SEGS) ? (nsegs - base) : SF_MAX_SEGS;
         SegTable t;
         memset(&t, 0, sizeof(t));
-        uint64_t tiles = 0;
+        uint64_t tiles = 0, size_units = 0;
         uint32_t m = 0;
         for (int i = 0; i < cnt; ++i) {
             const sf_seg& g = segs[base + i];
             if (g.n == 0) continue;
             if (g.src == 0 || g.dst == 0) return SF_EINVAL;
+            size_units += ceil_div(g.n, kSizeUnit);
             t.src[m] = g.src;
             t.dst[m] = g.dst;
             t.n[m] = g.n;
             t.tile_start[m] = tiles;
-            tiles += ceil_div(g.n, kTileElems);
+            tiles += ceil_div(g.n + lead_elems(g.dst), tile_elems);
             ++m;
         }
         if (m == 0) continue;
         t.tile_start[m] = tiles;
         t.nsegs = m;
-        if (tiles > kMaxBlocks) return SF_EINVAL;  // > 17.6e12 elements: not a real layer
-        uint64_t grid = tiles;
-        if (max_workgroups > 0 && grid > uint64_t(max_workgroups)) grid = uint64_t(max_workgroups);
-        hipLaunchKernelGGL(seg_kernel<Op>, dim3(uint32_t(grid)), dim3(kThreads), 0, stream, t);
+        if (size_units > kMaxBlocks) return SF_EINVAL;  // > 68e9 elements: not a real layer
+        uint64_t grid = tiles < kMaxBlocks ? tiles : kMaxBlocks;
+        if (capped && grid > uint64_t(max_workgroups)) grid = uint64_t(max_workgroups);
+        hipLaunchKernelGGL((capped ? seg_kernel<Op, kHostUnroll> : seg_kernel<Op, kSegUnroll>), dim3(uint32_t(grid)),
+                           dim3(kThreads), 0, stream, t);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return int(e);
     }
