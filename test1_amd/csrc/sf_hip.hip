@@ -57,23 +57,14 @@ __device__ __forceinline__ uint32_t rne_bf16(uint32_t u) {
 // infinity; NaN -> quiet NaN keeping the sign and the top 9 payload bits.
 // This is what torch's CPU cast gives (`.to(torch.float16)`, the reference's
 // staging of fp16 units, layer_state.py:301); the tests pin it against that
-// routine.  Integer arithmetic only, so the result does not depend on the
-// shader's floating-point modes.
+// routine.  v_cvt_f16_f32 does exactly this under the rounding and denormal
+// modes that the compiler sets for every kernel (nearest even, fp16
+// subnormals kept): compared with the same conversion in integer arithmetic
+// over all 2^32 inputs, no bit differs, NaN payloads included.  The integer
+// form took some 25 instructions per element and bound the cast: 12.6 M
+// elements 17.8 us, with the instruction 14.2.
 __device__ __forceinline__ uint32_t rne_f16(uint32_t u) {
-    const uint32_t sign = (u >> 16) & 0x8000u;
-    const uint32_t a = u & 0x7FFFFFFFu;
-    if (a > 0x7F800000u) return sign | 0x7E00u | ((a >> 13) & 0x1FFu);   // NaN
-    if (a >= 0x477FF000u) return sign | 0x7C00u;                          // rounds past 65504
-    if (a >= 0x38800000u) {                                               // normal half
-        const uint32_t r = a - 0x38000000u;                               // exponent rebias 127 -> 15
-        return sign | ((r + 0xFFFu + ((r >> 13) & 1u)) >> 13);
-    }
-    const uint32_t e = a >> 23;                                           // subnormal half or zero
-    if (e < 102u) return sign;                                            // below half the smallest subnormal
-    const uint32_t m = (a & 0x7FFFFFu) | 0x800000u;
-    const uint32_t s = 126u - e;                                          // 14 .. 24
-    const uint32_t q = m >> s, rem = m & ((1u << s) - 1u), half = 1u << (s - 1u);
-    return sign | (q + ((rem > half) | ((rem == half) & (q & 1u))));
+    return __builtin_bit_cast(uint16_t, static_cast<_Float16>(__uint_as_float(u)));
 }
 
 __device__ __forceinline__ uint32_t pack2(uint32_t lo, uint32_t hi) {
