@@ -15,6 +15,7 @@
 #include <hip/hip_runtime.h>
 #include <hsa/hsa.h>
 #include <hsa/hsa_ext_amd.h>
+#include <math.h>
 #include <stdint.h>
 #include <string.h>
 
@@ -192,87 +193,6 @@ __global__ __launch_bounds__(kCastThreads) void cast_flat_f16_kernel(
     cast_flat_body<ToF16>(src, dst, lead, n);
 }
 
-// ---------------------------------------------------------------------
-// Row gather: dst row t = src row ids[t] (rows of row_len elements), cast
-// fp32 -> bf16 (kCast) or copied as 16-bit values.  One workgroup per row
-// per iteration, grid-stride over the rows; src may be pinned host memory
-// (the row-sparse embedding load) and dst may be pinned host memory (the
-// row-sparse gradient offload, then with a capped grid).  An id outside
-// [0, nrows) yields a row of 0xFFFF (a NaN in bf16) and sets *bad.
-//
-// Each lane issues the loads of kRows 8-element groups of its row (kRows =
-// whole groups per lane, 1 to 4, picked at launch from the row length) before
-// the first store, so a row crosses the host link in one round trip.  Those
-// passes carry no per-lane predicate: under one, the compiler waits for all
-// outstanding memory operations before each store, and since stores count as
-// outstanding, each store into host memory would wait for the previous one
-// to be acknowledged over the link.  The groups left over (fewer than
-// kThreads * kRows) go one per lane with a predicate.  With a capped
-// 8-workgroup grid for the gradient-row offload (HBM -> pinned host, rows of
-// 4096 bf16) the unpredicated two-group pass measured 52.1-53.7 GB/s alone
-// against 47.7-48.3 GB/s with one group in flight per lane or with
-// predicated stores, and 55.6 GB/s with the offload's 16 workgroups; the
-// lookup (host -> HBM, one workgroup per row) is at the link's rate either
-// way (53.9 GB/s).
-// ---------------------------------------------------------------------
-template <bool kCast>
-__device__ __forceinline__ u32x4 gather_group(const void* __restrict__ src, uint64_t base, uint64_t g) {
-    if (kCast) {
-        const f32x4* p = reinterpret_cast<const f32x4*>(static_cast<const float*>(src) + base + g * kGroup);
-        return cast8(p[0], p[1]);
-    }
-    return reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(src) + base)[g];
-}
-
-template <bool kCast, int kRows>
-__global__ __launch_bounds__(kThreads) void gather_rows_kernel(
-    const void* __restrict__ src, const int64_t* __restrict__ ids, uint64_t ntok, uint64_t row_len,
-    uint64_t nrows, uint16_t* __restrict__ dst, uint32_t* __restrict__ bad, int vec) {
-    for (uint64_t t = blockIdx.x; t < ntok; t += gridDim.x) {
-        const int64_t r = ids[t];
-        uint16_t* out = dst + t * row_len;
-        if (r < 0 || uint64_t(r) >= nrows) {
-            for (uint64_t j = threadIdx.x; j < row_len; j += kThreads) out[j] = 0xFFFFu;
-            if (bad != nullptr && threadIdx.x == 0) bad[0] = 1u;
-            continue;
-        }
-        const uint64_t base = uint64_t(r) * row_len;
-        if (vec) {
-            constexpr uint64_t kPass = uint64_t(kThreads) * kRows;
-            const uint64_t g8 = row_len / kGroup;
-            const uint64_t full = g8 / kPass * kPass;
-            for (uint64_t g0 = 0; g0 < full; g0 += kPass) {
-                f32x4 a[kRows], b[kRows];
-                u32x4 v[kRows];
-#pragma unroll
-                for (int k = 0; k < kRows; ++k) {
-                    const uint64_t g = g0 + uint64_t(k) * kThreads + threadIdx.x;
-                    if (kCast) {
-                        const f32x4* p = reinterpret_cast<const f32x4*>(static_cast<const float*>(src) + base +
-                                                                       g * kGroup);
-                        a[k] = p[0];
-                        b[k] = p[1];
-                    } else {
-                        v[k] = reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(src) + base)[g];
-                    }
-                }
-#pragma unroll
-                for (int k = 0; k < kRows; ++k) {
-                    const uint64_t g = g0 + uint64_t(k) * kThreads + threadIdx.x;
-                    __builtin_nontemporal_store(kCast ? cast8(a[k], b[k]) : v[k], reinterpret_cast<u32x4*>(out) + g);
-                }
-            }
-            for (uint64_t g = full + threadIdx.x; g < g8; g += kThreads)
-                __builtin_nontemporal_store(gather_group<kCast>(src, base, g), reinterpret_cast<u32x4*>(out) + g);
-        } else {
-            for (uint64_t j = threadIdx.x; j < row_len; j += kThreads) {
-                out[j] = kCast ? uint16_t(rne_bf16(__float_as_uint(static_cast<const float*>(src)[base + j])))
-                               : static_cast<const uint16_t*>(src)[base + j];
-            }
-        }
-    }
-}
-
 // Scalar cast for pointers that are not aligned to their own elements.
 template <typename Fmt>
 __global__ __launch_bounds__(kThreads) void cast_scalar_kernel(
@@ -355,6 +275,11 @@ struct OpCast {
         const f32x4_any* q = reinterpret_cast<const f32x4_any*>(p);
         return {__builtin_nontemporal_load(q), __builtin_nontemporal_load(q + 1)};
     }
+    // a load that the caches may keep
+    __device__ static Raw load_kept(const S* p) {
+        const f32x4_any* q = reinterpret_cast<const f32x4_any*>(p);
+        return {q[0], q[1]};
+    }
     __device__ static u32x4 convert(const Raw& r) { return cast8(r.a, r.b); }
     __device__ static uint16_t convert1(S x) { return uint16_t(rne_bf16(__float_as_uint(x))); }
 };
@@ -365,6 +290,7 @@ struct OpCopy16 {
     __device__ static Raw load(const S* p) {
         return __builtin_nontemporal_load(reinterpret_cast<const u32x4_any*>(p));
     }
+    __device__ static Raw load_kept(const S* p) { return *reinterpret_cast<const u32x4_any*>(p); }
     __device__ static u32x4 convert(const Raw& r) { return r; }
     __device__ static uint16_t convert1(S x) { return x; }
 };
@@ -384,12 +310,22 @@ __device__ __forceinline__ void move_group(const typename Op::S* src, uint16_t* 
 
 constexpr int kSegUnroll = 1;   // groups per lane and tile: one workgroup per tile
 constexpr int kHostUnroll = 8;  // the same for a capped grid
+constexpr int kStageBlocks = 48;   // workgroups that read one array over the host link
+
+template <typename Op, int kU>
+__device__ __forceinline__ void store_tile(const typename Op::Raw (&v)[kU], uint16_t* out) {
+#pragma unroll
+    for (int k = 0; k < kU; ++k)
+        __builtin_nontemporal_store(Op::convert(v[k]), reinterpret_cast<u32x4*>(out + (k * kThreads + threadIdx.x) * kGroup));
+}
 
 template <typename Op, int kU>
 __global__ __launch_bounds__(kThreads) void seg_kernel(const SegTable t) {
     using S = typename Op::S;
     constexpr int64_t kTile = int64_t(kThreads) * kU * kGroup;
     const uint64_t ntiles = t.tile_start[t.nsegs];
+    typename Op::Raw v[kU];       // the last whole tile read
+    uint16_t* out = nullptr;      // and where it goes
     // Grid-stride over tiles: one workgroup per tile when the grid covers
     // them all, or a capped grid (e.g. a copy into host memory, which only
     // needs enough workgroups to keep the host link busy).
@@ -406,18 +342,334 @@ __global__ __launch_bounds__(kThreads) void seg_kernel(const SegTable t) {
             for (int64_t j = first + threadIdx.x; j < first + kTile && j < end; j += kThreads)
                 if (j >= lead) dst[j] = Op::convert1(src[j]);
         } else if (first >= lead && first + kTile <= end) {
-            // Whole tile: unpredicated loads, all in flight together.
-            typename Op::Raw v[kU];
+            // Whole tile: unpredicated loads, all in flight together.  With a
+            // capped grid they are issued before the stores of the tile before
+            // it, so that they don't wait for those to be acknowledged.
+            typename Op::Raw next[kU];
 #pragma unroll
-            for (int k = 0; k < kU; ++k) v[k] = Op::load(src + first + (k * kThreads + threadIdx.x) * kGroup);
+            for (int k = 0; k < kU; ++k) next[k] = Op::load(src + first + (k * kThreads + threadIdx.x) * kGroup);
+            if (kU > 1 && out != nullptr) store_tile<Op, kU>(v, out);
 #pragma unroll
-            for (int k = 0; k < kU; ++k)
-                __builtin_nontemporal_store(Op::convert(v[k]),
-                                            reinterpret_cast<u32x4*>(dst + first + (k * kThreads + threadIdx.x) * kGroup));
+            for (int k = 0; k < kU; ++k) v[k] = next[k];
+            out = dst + first;
+            if (kU == 1) store_tile<Op, kU>(v, out);
         } else {
             for (int k = 0; k < kU; ++k)
                 move_group<Op>(src, dst, first + (k * kThreads + threadIdx.x) * kGroup, lead, end);
         }
+    }
+    if (kU > 1 && out != nullptr) store_tile<Op, kU>(v, out);
+}
+
+// ---------------------------------------------------------------------
+// Row gather: dst row t = src row ids[t] (rows of row_len elements), cast
+// fp32 -> bf16 or copied as 16-bit values.  src may be pinned host memory
+// (the row-sparse embedding load) and dst may be pinned host memory (the
+// row-sparse gradient offload, then with a capped grid).  An id outside
+// [0, nrows) yields a row of 0xFFFF (a NaN in bf16) and sets *bad.
+//
+// A row is per_row groups of 8 elements, laid out from the 16-byte boundary
+// at or before its destination (kVec: every row starts on one and ends on
+// one), and a workgroup's tile is kU groups per lane of the rows put end to
+// end, so rows of any length fill its lanes.  All loads of a whole tile are
+// issued before its first store, without a per-lane predicate: under one, the
+// compiler waits for all outstanding memory operations before each store,
+// and each store into host memory would wait for the previous one to be
+// acknowledged over the link.  Bound by the link (about 57 GB/s; a DMA copy
+// of 128 MB reaches 55-57) or, inside HBM, by HBM.  Before, a workgroup took
+// one row at a time, so that short rows left it idle, and rows of a length
+// that is no multiple of 8 went element by element.  us, before -> now, fp32
+// rows from host memory: 4,096 rows of 4096 1250 -> 1125; 8,192 of 8192 4842
+// -> 3730.  16-bit rows into host memory, 16 workgroups: 8,192 of 64 139 ->
+// 26; 3,000 of 1003 224 -> 123; 4,096 of 4096 616 either way.
+// ---------------------------------------------------------------------
+struct RowShape {
+    uint64_t row_len, nrows;
+    uint64_t per_row;    // groups per row
+    uint32_t recip;      // ceil(2^31 / per_row), read where per_row < a tile
+};
+
+// Group x of rows put end to end, x - (row0 * per_row) = loc + rem0 < per_row
+// + kTile: its row past row0 and its place in that row.  A division by
+// multiplication: exact for loc + rem0 < 2^12 and per_row < 2^12.
+template <uint32_t kTile>
+__device__ __forceinline__ void split_group(const RowShape& s, uint64_t rem0, uint32_t loc, uint32_t& row,
+                                            uint64_t& j) {
+    static_assert(kTile <= 2048, "split_group's product");
+    if (s.per_row >= kTile) {
+        const uint64_t x = rem0 + loc;
+        row = x >= s.per_row ? 1u : 0u;
+        j = row ? x - s.per_row : x;
+    } else {
+        const uint32_t x = uint32_t(rem0) + loc;
+        row = __umulhi(2 * x, s.recip);
+        j = x - row * uint32_t(s.per_row);
+    }
+}
+
+// How rows lie: every one starts and ends on a 16-byte boundary of the
+// destination (and the source is aligned so), rows of at least 8 elements
+// that start anywhere, or what is left: shorter rows, and a source that is
+// not aligned to its own elements.
+enum RowMode { kWhole, kEdges, kElements };
+
+// A tile between its loads and its stores (kWhole, kEdges).
+template <typename Op, int kU, RowMode kMode>
+struct Held {
+    typename Op::Raw v[kU];
+    uint16_t* out[kU];
+    uint32_t part[kMode == kEdges ? kU : 1];   // bit d: element d of v goes to out + d
+    bool ok[kU];
+};
+
+// Loads of a tile that starts at group rem0 of row row0; lanes past its group
+// `last` load that one again.  row_of(i, t, id): destination row and id of
+// row i.  kEdges: of a row's first and last group, which can be partial, the
+// nearest 8 elements of the row are loaded.
+template <typename Op, int kU, RowMode kMode, typename RowOf>
+__device__ __forceinline__ void load_rows(Held<Op, kU, kMode>& h, const typename Op::S* src, uint16_t* dst,
+                                          const RowShape& s, uint64_t row0, uint64_t rem0, uint32_t last,
+                                          RowOf row_of) {
+#pragma unroll
+    for (int k = 0; k < kU; ++k) {
+        const uint32_t loc = k * kThreads + threadIdx.x;
+        uint32_t i;
+        uint64_t j, t;
+        int64_t id;
+        split_group<kThreads * kU>(s, rem0, loc < last ? loc : last, i, j);
+        row_of(row0 + i, t, id);
+        h.ok[k] = id >= 0 && uint64_t(id) < s.nrows;
+        uint16_t* row = dst + t * s.row_len;
+        int64_t at = int64_t(j) * kGroup;
+        if (kMode == kEdges) {
+            const int64_t e = at - int64_t(lead_elems(reinterpret_cast<uint64_t>(row)));
+            const int64_t n = int64_t(s.row_len);
+            at = e < 0 ? 0 : (e + kGroup <= n ? e : n - kGroup);
+            // the group is [e, e + 8) of the row, the 8 loaded elements [at, at + 8)
+            const int64_t d = at - e;
+            h.part[k] = d >= kGroup || d <= -kGroup ? 0u : d >= 0 ? 0xFFu >> d : (0xFFu << -d) & 0xFFu;
+        }
+        h.out[k] = row + at;
+        h.v[k] = Op::load_kept(src + (h.ok[k] ? uint64_t(id) : 0) * s.row_len + at);
+    }
+}
+
+// Its stores: of all groups (kAll) or of the first n.
+template <typename Op, int kU, RowMode kMode, bool kAll>
+__device__ __forceinline__ bool store_rows(const Held<Op, kU, kMode>& h, uint32_t n) {
+    const u32x4 nan = {~0u, ~0u, ~0u, ~0u};
+    bool any_bad = false;
+#pragma unroll
+    for (int k = 0; k < kU; ++k) {
+        const u32x4 c = Op::convert(h.v[k]);
+        const u32x4 o = h.ok[k] ? c : nan;
+        any_bad |= !h.ok[k];
+        if (!kAll && k * kThreads + threadIdx.x >= n) continue;
+        if (kMode == kWhole || h.part[k] == 0xFFu) {
+            __builtin_nontemporal_store(o, reinterpret_cast<u32x4*>(h.out[k]));
+        } else {
+#pragma unroll
+            for (int d = 0; d < kGroup; ++d)
+                if (h.part[k] >> d & 1) h.out[k][d] = uint16_t(o[d / 2] >> (d % 2 * 16));
+        }
+    }
+    return any_bad;
+}
+
+// One tile of n groups (up to kThreads * kU) from group rem0 of row row0 on.
+template <typename Op, int kU, RowMode kMode, typename RowOf>
+__device__ __forceinline__ bool gather_tile(const typename Op::S* src, uint16_t* dst, const RowShape& s, uint64_t row0,
+                                            uint64_t rem0, uint32_t n, RowOf row_of) {
+    constexpr uint32_t kTile = kThreads * kU;
+    bool any_bad = false;
+    if (kMode != kElements) {
+        Held<Op, kU, kMode> h;
+        load_rows<Op, kU, kMode>(h, src, dst, s, row0, rem0, n - 1, row_of);
+        return n == kTile ? store_rows<Op, kU, kMode, true>(h, n) : store_rows<Op, kU, kMode, false>(h, n);
+    }
+    for (uint32_t loc = threadIdx.x; loc < n; loc += kThreads) {
+        uint32_t i;
+        uint64_t j, t;
+        int64_t id;
+        split_group<kTile>(s, rem0, loc, i, j);
+        row_of(row0 + i, t, id);
+        const bool ok = id >= 0 && uint64_t(id) < s.nrows;
+        any_bad |= !ok;
+        const typename Op::S* from = src + (ok ? uint64_t(id) * s.row_len : 0);
+        uint16_t* row = dst + t * s.row_len;
+        for (uint64_t q = j * kGroup; q < (j + 1) * kGroup && q < s.row_len; ++q)
+            row[q] = ok ? Op::convert1(from[q]) : uint16_t(0xFFFFu);
+    }
+    return any_bad;
+}
+
+// Rows of a table in HBM; short rows, or rows of fewer than 8 elements, of one
+// in host memory.  A workgroup takes span groups, up to one per lane.
+template <bool kCast> struct GatherOp { using T = OpCopy16; };
+template <> struct GatherOp<true> { using T = OpCast; };
+
+template <bool kCast, RowMode kMode>
+__global__ __launch_bounds__(kThreads) void gather_rows_kernel(const void* __restrict__ src,
+                                                               const int64_t* __restrict__ ids, uint64_t ntok,
+                                                               RowShape s, uint32_t span, uint16_t* __restrict__ dst,
+                                                               uint32_t* __restrict__ bad) {
+    using Op = typename GatherOp<kCast>::T;
+    const uint64_t total = ntok * s.per_row;
+    bool any_bad = false;
+    for (uint64_t b = blockIdx.x; b * span < total; b += gridDim.x) {
+        const uint64_t tile0 = b * span, row0 = span == s.per_row ? b : tile0 / s.per_row;
+        any_bad |= gather_tile<Op, 1, kMode>(static_cast<const typename Op::S*>(src), dst, s, row0,
+                                             tile0 - row0 * s.per_row,
+                                             uint32_t(total - tile0 < span ? total - tile0 : span),
+                                             [&](uint64_t i, uint64_t& t, int64_t& id) { t = i; id = ids[i]; });
+    }
+    if (any_bad && bad != nullptr) bad[0] = 1u;
+}
+
+// Rows that cross the host link: of a table in pinned host memory, with at
+// most kLinkBlocks workgroups, or into pinned host memory with the caller's
+// cap; kU groups per lane in flight.  A few workgroups keep the link busy, and
+// more requests at once only get into each other's way (us, 1 workgroup per
+// tile | 128 | 64 | 32 | 16: 4,096 rows of 4096 fp32 1237 | 1198 | 1175 | 1171
+// | 1210; 1,581 of 480 74 | 72.5 | 61.6 | 59.4 | 59.8).  The ids are taken
+// from LDS, so that no second latency stands before the rows' own.  Host rows
+// shorter than kLinkRow bytes go one per workgroup instead, as fast or faster
+// (us, link | one per workgroup: 3,000 fp32 rows of 320 77.3 | 71.7, of 500
+// 120.8 | 116.3, of 640 140.2 | 139.9, of 1000 221 | 225).
+//
+// kOnce: a row that several tokens ask for crosses the link once.  The first
+// token of each window of kWindow that asks for it gathers it, and
+// repeat_gather_rows_kernel copies it to the others inside HBM.  Both find
+// the first token by a hash table of the window's ids in LDS, which every
+// workgroup makes for itself (some 5 us; no memory beside the operands).
+constexpr uint32_t kLinkBlocks = 32;
+constexpr size_t kLinkRow = 2560;
+constexpr uint32_t kWindow = 8192;
+constexpr uint32_t kSlots = 2 * kWindow;   // of the hash table, at most half full
+constexpr uint32_t kEmpty = ~0u;
+// A table entry is id * kWindow + token, so that entries of one id are
+// ordered by token.  nrows < kOnceRows leaves kNoRow free for ids outside the
+// table and keeps every entry different from kEmpty.
+constexpr uint64_t kOnceRows = (uint64_t(1) << 32) / kWindow - 1;
+constexpr uint32_t kNoRow = uint32_t(kOnceRows);
+
+__device__ __forceinline__ uint32_t first_slot(uint32_t id) { return id * 2654435761u >> (32 - 14); }
+static_assert(kSlots == 1u << 14, "first_slot");
+
+// slots[] = for every id of the window its first token.
+__device__ __forceinline__ void index_window(uint32_t* slots, const int64_t* ids, uint32_t n, uint64_t nrows) {
+    for (uint32_t i = threadIdx.x; i < kSlots; i += blockDim.x) slots[i] = kEmpty;
+    __syncthreads();
+    for (uint32_t t = threadIdx.x; t < n; t += blockDim.x) {
+        const int64_t id = ids[t];
+        if (id < 0 || uint64_t(id) >= nrows) continue;
+        const uint32_t entry = uint32_t(id) * kWindow + t;
+        for (uint32_t h = first_slot(uint32_t(id));; h = (h + 1) % kSlots) {
+            const uint32_t old = atomicCAS(&slots[h], kEmpty, entry);
+            if (old == kEmpty) break;
+            if (old / kWindow == uint32_t(id)) {
+                atomicMin(&slots[h], entry);
+                break;
+            }
+        }
+    }
+    __syncthreads();
+}
+
+// The first token of the window that asks for row id, which is in the table.
+__device__ __forceinline__ uint32_t first_token(const uint32_t* slots, uint32_t id) {
+    uint32_t h = first_slot(id);
+    while (slots[h] / kWindow != id) h = (h + 1) % kSlots;
+    return slots[h] % kWindow;
+}
+
+template <bool kCast, int kU, RowMode kMode, bool kOnce>
+__global__ __launch_bounds__(kThreads) void link_gather_rows_kernel(const void* __restrict__ src,
+                                                                    const int64_t* __restrict__ ids, uint64_t ntok,
+                                                                    RowShape s, uint16_t* __restrict__ dst,
+                                                                    uint32_t* __restrict__ bad) {
+    using Op = typename GatherOp<kCast>::T;
+    // this workgroup's tokens of the window: every gridDim.x-th
+    constexpr uint32_t kMine = kOnce ? kWindow / kLinkBlocks : kWindow;
+    __shared__ uint32_t slots[kOnce ? kSlots : 1];
+    __shared__ uint32_t own[kMine];   // kOnce: entries of the tokens to gather; else ids, ~0 outside the table
+    __shared__ uint32_t count;
+    const auto* table = static_cast<const typename Op::S*>(src);
+    const uint64_t tile_rows = kThreads * kU / s.per_row, tile_rem = kThreads * kU - tile_rows * s.per_row;
+    bool any_bad = false;
+    for (uint64_t w0 = 0; w0 < ntok; w0 += kWindow) {
+        const uint32_t n = uint32_t(ntok - w0 < kWindow ? ntok - w0 : kWindow);
+        const uint32_t mine = n > blockIdx.x ? (n - blockIdx.x + gridDim.x - 1) / gridDim.x : 0;
+        if (kOnce) {
+            if (threadIdx.x == 0) count = 0;
+            index_window(slots, ids + w0, n, s.nrows);
+        }
+        for (uint32_t i = threadIdx.x; i < mine; i += kThreads) {
+            const uint32_t t = blockIdx.x + i * gridDim.x;
+            const int64_t id = ids[w0 + t];
+            const bool ok = id >= 0 && uint64_t(id) < s.nrows;
+            if (!kOnce) own[i] = ok ? uint32_t(id) : ~0u;
+            else if (!ok || first_token(slots, uint32_t(id)) == t)
+                own[atomicAdd(&count, 1u)] = (ok ? uint32_t(id) : kNoRow) * kWindow + t;
+        }
+        __syncthreads();
+        const auto row_of = [&](uint64_t i, uint64_t& t, int64_t& id) {
+            const uint32_t e = own[i];
+            t = w0 + (kOnce ? e % kWindow : blockIdx.x + uint32_t(i) * gridDim.x);
+            id = kOnce ? e / kWindow : e;   // past the last row for one outside the table
+        };
+        constexpr uint32_t kTile = kThreads * kU;
+        uint64_t left = uint64_t(kOnce ? count : mine) * s.per_row, row0 = 0, rem0 = 0;
+        if (left > 0) {
+            // A tile's loads are issued before the stores of the one before it,
+            // so that they don't wait for those to be acknowledged.
+            Held<Op, kU, kMode> h;
+            uint32_t n = uint32_t(left < kTile ? left : kTile);
+            load_rows<Op, kU, kMode>(h, table, dst, s, row0, rem0, n - 1, row_of);
+            while (left > kTile) {
+                left -= kTile;
+                row0 += tile_rows;
+                rem0 += tile_rem;
+                if (rem0 >= s.per_row) {
+                    rem0 -= s.per_row;
+                    ++row0;
+                }
+                n = uint32_t(left < kTile ? left : kTile);
+                Held<Op, kU, kMode> next;
+                load_rows<Op, kU, kMode>(next, table, dst, s, row0, rem0, n - 1, row_of);
+                any_bad |= store_rows<Op, kU, kMode, true>(h, kTile);
+                h = next;
+            }
+            any_bad |= n == kTile ? store_rows<Op, kU, kMode, true>(h, n) : store_rows<Op, kU, kMode, false>(h, n);
+        }
+        __syncthreads();   // before the next window's ids
+    }
+    if (any_bad && bad != nullptr) bad[0] = 1u;
+}
+
+// The rows that link_gather_rows_kernel<kOnce> left out, from the row it
+// gathered: one wave per token.
+constexpr int kRepeatThreads = 1024;
+constexpr uint32_t kRepeatBlocks = 256;
+__global__ __launch_bounds__(kRepeatThreads) void repeat_gather_rows_kernel(const int64_t* __restrict__ ids,
+                                                                            uint64_t ntok, RowShape s, uint16_t* dst) {
+    __shared__ uint32_t slots[kSlots];
+    for (uint64_t w0 = 0; w0 < ntok; w0 += kWindow) {
+        const uint32_t n = uint32_t(ntok - w0 < kWindow ? ntok - w0 : kWindow);
+        index_window(slots, ids + w0, n, s.nrows);
+        for (uint32_t t = blockIdx.x * (kRepeatThreads / 64) + (threadIdx.x >> 6); t < n;
+             t += gridDim.x * (kRepeatThreads / 64)) {
+            const int64_t id = ids[w0 + t];
+            if (id < 0 || uint64_t(id) >= s.nrows) continue;
+            const uint32_t f = first_token(slots, uint32_t(id));
+            if (f == t) continue;
+            const uint16_t* from = dst + (w0 + f) * s.row_len;
+            uint16_t* row = dst + (w0 + t) * s.row_len;
+            const int64_t lead = lead_elems(reinterpret_cast<uint64_t>(row));
+            for (uint64_t j = threadIdx.x & 63; j < s.per_row; j += 64)
+                move_group<OpCopy16>(from - lead, row - lead, int64_t(j) * kGroup, lead, int64_t(s.row_len) + lead);
+        }
+        __syncthreads();   // before the next window's table
     }
 }
 
@@ -478,6 +730,65 @@ inline int hip_status(hipError_t e) {
 }  // namespace
 
 namespace {
+// The memory type the runtime records for ptr, or -1 for memory it does
+// not know (pageable host memory).
+int pointer_attributes(const void* p, hipPointerAttribute_t* a) {
+    const hipError_t e = hipPointerGetAttributes(a, p);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        return -1;
+    }
+    return int(a->type);
+}
+
+int memory_type(const void* p) {
+    hipPointerAttribute_t a;
+    return pointer_attributes(p, &a);
+}
+
+// Bytes that a gather over the host link would read again for ids it has met
+// before, were the ids drawn uniformly (those of text repeat more often).  A
+// table that fits the L2s crosses the link at most once for each of the 8.
+inline double repeated_bytes(size_t ntok, size_t nrows, size_t row_bytes) {
+    const double n = double(ntok < kWindow ? ntok : kWindow), v = double(nrows);
+    const double met = v * -expm1(-n / v) * (double(ntok) / n);
+    const double read = double(ntok) < 8.0 * v ? double(ntok) : 8.0 * v;
+    return (read - met) * double(row_bytes);
+}
+
+// Reading rows once pays from here on: 2 MiB are 37 us on the link; the hash
+// tables and the second kernel cost 5 (1,024 tokens) to 25 us (8,192).  fp32
+// rows of 4096: 4,096 tokens of 32,000 rows 1168 -> 1125 us, of 2,000 rows
+// 1076 -> 533; 1,024 of 32,000 rows, 0.3 MiB to save, 298 -> 306.  8,192
+// tokens of 256 rows of 1024 160 -> 45 us, of 256 rows of 64, 0.4 MiB, 15 -> 24.
+constexpr double kOnceBytes = 2 << 20;
+
+template <bool kCast, RowMode kMode>
+int launch_gather(const void* src, const int64_t* ids, uint64_t ntok, const RowShape& s, uint16_t* dst, uint32_t* bad,
+                  uint64_t cap, bool from_host, bool link, bool once, hipStream_t st) {
+    if constexpr (kMode != kElements) {
+        if (link) {
+            constexpr int kU = kCast ? 4 : 8;   // 128 bytes per lane in flight
+            hipLaunchKernelGGL((once ? link_gather_rows_kernel<kCast, kU, kMode, true>
+                                     : link_gather_rows_kernel<kCast, kU, kMode, false>),
+                               dim3(uint32_t(ntok < cap ? ntok : cap)), dim3(kThreads), 0, st, src, ids, ntok, s, dst,
+                               bad);
+            if (once) {
+                const hipError_t e = hipGetLastError();
+                if (e != hipSuccess) return hip_status(e);
+                hipLaunchKernelGGL(repeat_gather_rows_kernel, dim3(kRepeatBlocks), dim3(kRepeatThreads), 0, st, ids,
+                                   ntok, s, dst);
+            }
+            return hip_status(hipGetLastError());
+        }
+    }
+    const uint32_t span = from_host && s.per_row < uint64_t(kThreads) ? uint32_t(s.per_row) : uint32_t(kThreads);
+    const uint64_t tiles = ceil_div(ntok * s.per_row, span);
+    hipLaunchKernelGGL((gather_rows_kernel<kCast, kMode>), dim3(uint32_t(tiles < cap ? tiles : cap)), dim3(kThreads), 0,
+                       st, src, ids, ntok, s, span, dst, bad);
+    return hip_status(hipGetLastError());
+}
+
 template <bool kCast>
 int launch_gather_rows(const void* src, const int64_t* ids, size_t ntok, size_t row_len, size_t nrows,
                        uint16_t* dst, uint32_t* bad, int max_workgroups, hipStream_t st, size_t src_elem) {
@@ -487,19 +798,27 @@ int launch_gather_rows(const void* src, const int64_t* ids, size_t ntok, size_t 
     // the destination rows must not overlap the source table
     const uintptr_t s0 = reinterpret_cast<uintptr_t>(src), d0 = reinterpret_cast<uintptr_t>(dst);
     if (s0 < d0 + 2 * ntok * row_len && d0 < s0 + src_elem * nrows * row_len) return SF_EOVERLAP;
-    const int vec = (row_len % kGroup == 0) && ((s0 | d0) & 15) == 0;
-    uint64_t grid = ntok;
-    if (max_workgroups > 0 && grid > uint64_t(max_workgroups)) grid = uint64_t(max_workgroups);
-    if (grid > kMaxBlocks) grid = kMaxBlocks;
-    // whole groups of 8 per lane and pass, 1 to 4
-    const uint64_t per_lane = (row_len / kGroup) / kThreads;
-    auto kernel = per_lane >= 4 ? gather_rows_kernel<kCast, 4>
-                : per_lane == 3 ? gather_rows_kernel<kCast, 3>
-                : per_lane == 2 ? gather_rows_kernel<kCast, 2>
-                                : gather_rows_kernel<kCast, 1>;
-    hipLaunchKernelGGL(kernel, dim3(uint32_t(grid)), dim3(kThreads), 0, st, src, ids, uint64_t(ntok),
-                       uint64_t(row_len), uint64_t(nrows), dst, bad, vec);
-    return hip_status(hipGetLastError());
+    const RowMode mode = nrows == 0 || row_len < size_t(kGroup) || (s0 & (src_elem - 1)) != 0 ? kElements
+                         : row_len % kGroup == 0 && ((s0 | d0) & 15) == 0                     ? kWhole
+                                                                                              : kEdges;
+    RowShape s;
+    s.row_len = row_len;
+    s.nrows = nrows;
+    s.per_row = mode == kEdges ? (uint64_t(row_len) + 2 * kGroup - 2) / kGroup : ceil_div(row_len, kGroup);
+    s.recip = uint32_t(ceil_div(uint64_t(1) << 31, s.per_row));
+    uint64_t cap = max_workgroups > 0 ? uint64_t(max_workgroups) : kMaxBlocks;
+    const bool from_host = memory_type(src) == int(hipMemoryTypeHost);
+    const bool once = from_host && mode != kElements && cap > kLinkBlocks && ntok >= kLinkBlocks &&
+                      nrows < kOnceRows && repeated_bytes(ntok, nrows, row_len * src_elem) >= kOnceBytes &&
+                      memory_type(dst) == int(hipMemoryTypeDevice);
+    const bool link = (once || max_workgroups > 0 || (from_host && row_len * src_elem >= kLinkRow)) &&
+                      nrows < (uint64_t(1) << 31);
+    if (link && from_host && cap > kLinkBlocks) cap = kLinkBlocks;
+    switch (mode) {
+        case kWhole: return launch_gather<kCast, kWhole>(src, ids, ntok, s, dst, bad, cap, from_host, link, once, st);
+        case kEdges: return launch_gather<kCast, kEdges>(src, ids, ntok, s, dst, bad, cap, from_host, link, once, st);
+        default: return launch_gather<kCast, kElements>(src, ids, ntok, s, dst, bad, cap, from_host, link, once, st);
+    }
 }
 }  // namespace
 
@@ -694,43 +1013,24 @@ int sf_fill_b16(uint16_t* dst, size_t n, uint16_t value, sf_stream_t stream) {
 }  // extern "C"
 
 // ---------------------------------------------------------------------
-// Staging: pinned fp32 host array -> bf16 device array, through a device
-// fp32 buffer, all on one stream.  Each piece is copied into the buffer by
-// DMA and cast from it by cast_flat_kernel; the next piece's copy into the
-// same buffer follows that cast in stream order.  With one stream the copy
-// and the cast do not overlap; the cast moves 1.5x the copy's bytes over
-// HBM at ~100x the host link's rate, so it adds ~1-2 % to the copy.
+// Staging: pinned fp32 host array -> bf16 device array, by the segment cast
+// reading the host array over the link: one kernel, which the link bounds.
+// With kStageBlocks workgroups of kHostUnroll groups per lane it reads as
+// fast as a DMA copy, starts sooner and leaves no cast to follow: 147,712
+// elements 30.1 -> 14.3 us, 600,000 61 -> 48, 8 M 587 -> 572, 32 M 2287 ->
+// 2251.  One workgroup per tile reads 2 M elements in 181 us, 64 of 4 groups
+// per lane in 146, 16 to 96 of 8 in 146 to 153.
 // ---------------------------------------------------------------------
 namespace {
 
-// The memory type the runtime records for ptr, or -1 for memory it does
-// not know (pageable host memory).
-int memory_type(const void* p) {
-    hipPointerAttribute_t a;
-    const hipError_t e = hipPointerGetAttributes(&a, p);
-    if (e != hipSuccess) {
-        (void)hipGetLastError();
-        return -1;
-    }
-    return int(a.type);
-}
-
-int stage_launch(const float* host, uint16_t* dst, size_t n, float* buf, size_t chunk, hipStream_t st) {
+int stage_launch(const float* host, uint16_t* dst, size_t n, hipStream_t st) {
     if (n == 0) return SF_OK;
-    if (host == nullptr || dst == nullptr || buf == nullptr) return SF_EINVAL;
-    // an asynchronous copy needs pinned host memory; the cast writes device memory
-    if (memory_type(host) != int(hipMemoryTypeHost) || memory_type(dst) != int(hipMemoryTypeDevice))
+    hipPointerAttribute_t a;
+    // pinned host memory, which a kernel can read; the cast writes device memory
+    if (pointer_attributes(host, &a) != int(hipMemoryTypeHost) || memory_type(dst) != int(hipMemoryTypeDevice))
         return SF_EINVAL;
-    chunk -= chunk % kGroup;  // every piece starts 16-byte aligned in dst if dst does
-    if (chunk == 0) return SF_EINVAL;
-    for (size_t off = 0; off < n; off += chunk) {
-        const size_t c = n - off < chunk ? n - off : chunk;
-        const hipError_t e = hipMemcpyAsync(buf, host + off, c * sizeof(float), hipMemcpyHostToDevice, st);
-        if (e != hipSuccess) return hip_status(e);
-        const int rc = cast_launch(buf, dst + off, c, st, nullptr, nullptr);
-        if (rc != SF_OK) return rc;
-    }
-    return SF_OK;
+    const sf_seg seg = {reinterpret_cast<uint64_t>(a.devicePointer), reinterpret_cast<uint64_t>(dst), n};
+    return launch_segs<OpCast>(&seg, 1, kStageBlocks, st);
 }
 
 }  // namespace
@@ -739,93 +1039,29 @@ extern "C" {
 
 int sf_stage_f32_bf16(const float* host_src, uint16_t* dst, size_t n, float* workspace, size_t workspace_elems,
                       sf_stream_t stream) {
-    if (n > 0 && (workspace == nullptr || memory_type(workspace) != int(hipMemoryTypeDevice))) return SF_EINVAL;
-    return stage_launch(host_src, dst, n, workspace, workspace_elems, reinterpret_cast<hipStream_t>(stream));
+    if (n == 0) return SF_OK;
+    if (host_src == nullptr || dst == nullptr || workspace == nullptr || workspace_elems < size_t(kGroup) ||
+        memory_type(workspace) != int(hipMemoryTypeDevice))
+        return SF_EINVAL;
+    return stage_launch(host_src, dst, n, reinterpret_cast<hipStream_t>(stream));
 }
-
-}  // extern "C"
-
-// ---------------------------------------------------------------------
-// Staging without allocating: the pieces go through the library's own
-// device buffer instead of a caller workspace.  `scratch` is a static
-// device array, so every device the library's code object is loaded on
-// holds one for the life of the process.  In host code its name is not a
-// device address: the address comes from hipGetSymbolAddress, looked up
-// once per device with that device current, and only that address is
-// passed to the copies and the cast.
-// ---------------------------------------------------------------------
-namespace {
-
-__device__ __align__(256) float scratch[SF_STAGE_SCRATCH_ELEMS];
-
-constexpr int kMaxDevices = 64;
-// Per device: the address of `scratch`, and an event recorded after the last
-// cast of the previous call (the next call's stream waits on it).  The
-// mutex is held from the wait to the record, so the calls of several host
-// threads are ordered one after the other.
-struct ScratchState {
-    float* ptr = nullptr;
-    hipEvent_t last = nullptr;
-    bool recorded = false;
-};
-std::mutex g_scratch_mu;
-ScratchState g_scratch[kMaxDevices];
-
-// The current device, which must be the device of `st` (the null stream:
-// the current device), after the one-time set-up of its scratch state.
-int scratch_device_for_stream(hipStream_t st, int* dev) {
-    int cur = 0;
-    hipError_t e = hipGetDevice(&cur);
-    if (e != hipSuccess) return hip_status(e);
-    if (st != nullptr) {
-        hipDevice_t sd = 0;
-        e = hipStreamGetDevice(st, &sd);
-        if (e != hipSuccess) return hip_status(e);
-        if (int(sd) != cur) return SF_EINVAL;
-    }
-    if (cur < 0 || cur >= kMaxDevices) return SF_EINVAL;
-    ScratchState& s = g_scratch[cur];
-    if (s.ptr == nullptr) {
-        void* p = nullptr;
-        e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
-        if (e != hipSuccess) return hip_status(e);
-        if (p == nullptr) return SF_EINVAL;
-        if (s.last == nullptr) {
-            e = hipEventCreateWithFlags(&s.last, hipEventDisableTiming);
-            if (e != hipSuccess) return hip_status(e);
-        }
-        s.ptr = static_cast<float*>(p);
-    }
-    *dev = cur;
-    return SF_OK;
-}
-
-}  // namespace
-
-extern "C" {
 
 int sf_stage_f32_bf16_noalloc(const float* host_src, uint16_t* dst, size_t n, size_t chunk_elems,
                               sf_stream_t stream) {
     if (chunk_elems > SF_STAGE_SCRATCH_ELEMS) return SF_ETOOBIG;
     if (n == 0) return SF_OK;
-    if (host_src == nullptr || dst == nullptr) return SF_EINVAL;
+    if (host_src == nullptr || dst == nullptr || (chunk_elems != 0 && chunk_elems < size_t(kGroup))) return SF_EINVAL;
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    std::lock_guard<std::mutex> lk(g_scratch_mu);
-    int dev = 0;
-    int rc = scratch_device_for_stream(st, &dev);
-    if (rc != SF_OK) return rc;
-    ScratchState& s = g_scratch[dev];
-    if (s.recorded) {
-        const hipError_t e = hipStreamWaitEvent(st, s.last, 0);
+    // the stream must be the current device's
+    if (st != nullptr) {
+        int cur = 0;
+        hipDevice_t sd = 0;
+        hipError_t e = hipGetDevice(&cur);
+        if (e == hipSuccess) e = hipStreamGetDevice(st, &sd);
         if (e != hipSuccess) return hip_status(e);
+        if (int(sd) != cur) return SF_EINVAL;
     }
-    rc = stage_launch(host_src, dst, n, s.ptr, chunk_elems == 0 ? SF_STAGE_SCRATCH_ELEMS : chunk_elems, st);
-    // Recorded also after a failed launch: whatever was enqueued before the
-    // failure still uses the scratch buffer and must precede the next call.
-    const hipError_t e = hipEventRecord(s.last, st);
-    if (e == hipSuccess) s.recorded = true;
-    if (rc != SF_OK) return rc;
-    return hip_status(e);
+    return stage_launch(host_src, dst, n, st);
 }
 
 int sf_memcpy_async(void* dst, const void* src, size_t bytes, int kind, sf_stream_t stream) {
