@@ -13,6 +13,7 @@ interchangeable between the two.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
 import threading
 
@@ -21,6 +22,7 @@ import torch  # noqa: F401  (loads torch's HIP runtime first; see above)
 LIB_DIR = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib")
 HIP_LIB = os.path.join(LIB_DIR, "libsf_hip.so")
 CPU_LIB = os.path.join(LIB_DIR, "libsf_cpu.so")
+SEGS_LIB = os.path.join(LIB_DIR, "_sf_segs.so")
 
 SF_COPY_H2D = 1
 SF_COPY_D2H = 2
@@ -77,10 +79,11 @@ HIP_SIGNATURES = {
     "sf_event_create": [ctypes.POINTER(ctypes.c_void_p)],
     "sf_event_destroy": [_vp],
     "sf_event_elapsed_ms": [_vp, _vp, ctypes.POINTER(ctypes.c_float)],
-    "sf_cast_scatter_f32_bf16": [ctypes.POINTER(SfSeg), _i, _vp],
-    "sf_pack_b16": [ctypes.POINTER(SfSeg), _i, _vp, _i, _vp],
-    "sf_unpack_b16": [_vp, ctypes.POINTER(SfSeg), _i, _i, _vp],
-    "sf_copy_segs_b16": [ctypes.POINTER(SfSeg), _i, _i, _vp],
+    # the segment tables of the next four: an SfSeg array, or a bytes object of them
+    "sf_cast_scatter_f32_bf16": [_vp, _i, _vp],
+    "sf_pack_b16": [_vp, _i, _vp, _i, _vp],
+    "sf_unpack_b16": [_vp, _vp, _i, _i, _vp],
+    "sf_copy_segs_b16": [_vp, _i, _i, _vp],
     "sf_fill_b16": [_vp, _sz, ctypes.c_uint16, _vp],
     "sf_gather_rows_f32_bf16": [_vp, _vp, _sz, _sz, _sz, _vp, _vp, _i, _vp],
     "sf_gather_rows_b16": [_vp, _vp, _sz, _sz, _sz, _vp, _vp, _i, _vp],
@@ -136,16 +139,21 @@ CPU_SIGNATURES = {
 _lock = threading.Lock()
 _hip = None
 _cpu = None
+_segs = None
 
 _RESTYPES = {"sf_error_string": ctypes.c_char_p, "sf_dma_choose_engines": ctypes.c_uint32}
 
 
-def _bind(path: str, sigs: dict) -> ctypes.CDLL:
+def _require_built(path: str) -> None:
     if not os.path.exists(path):
         raise RuntimeError(
             f"native library not built: {path}. Build it with `python -c \"import "
             f"__graft_entry__ as g; g.build()\"` (or `python -m test1_amd.build`)."
         )
+
+
+def _bind(path: str, sigs: dict) -> ctypes.CDLL:
+    _require_built(path)
     lib = ctypes.CDLL(path)
     for name, args in sigs.items():
         fn = getattr(lib, name)
@@ -170,6 +178,22 @@ def cpu() -> ctypes.CDLL:
             if _cpu is None:
                 _cpu = _bind(CPU_LIB, CPU_SIGNATURES)
     return _cpu
+
+
+def segs():
+    """The module that reads segment tables from lists of tensors."""
+    global _segs
+    if _segs is None:
+        with _lock:
+            if _segs is None:
+                import torch  # noqa: F401  (its libraries are what the module links against)
+
+                _require_built(SEGS_LIB)
+                spec = importlib.util.spec_from_file_location("_sf_segs", SEGS_LIB)
+                module = importlib.util.module_from_spec(spec)
+                spec.loader.exec_module(module)
+                _segs = module
+    return _segs
 
 
 class NativeError(RuntimeError):

@@ -8,6 +8,8 @@ warns that it does not know the feature, which is expected.
 libsf_cpu.so: g++ with OpenMP; AVX-512 is selected per function at run time,
 and -ffp-contract=off keeps every scalar operation a single rounding.  The
 storage offload engine (worker threads, pread/pwrite) is in the same library.
+_sf_segs.so: g++ against torch's headers, a CPython module that reads segment
+tables from lists of tensors.
 """
 
 from __future__ import annotations
@@ -16,6 +18,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -64,9 +67,26 @@ def build_cpu(verbose: bool = False) -> str:
     return out
 
 
+def build_segs(verbose: bool = False) -> str:
+    import torch
+
+    os.makedirs(LIB, exist_ok=True)
+    out = os.path.join(LIB, "_sf_segs.so")
+    tmp = _atomic_out(out)
+    base = os.path.dirname(torch.__file__)
+    _run([CXX, "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-fvisibility=hidden",
+          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}", "-I", INCLUDE,
+          "-I", sysconfig.get_paths()["include"], "-isystem", os.path.join(base, "include"), "-o", tmp,
+          os.path.join(CSRC, "sf_segs.cpp"), "-L", os.path.join(base, "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10"],
+         verbose)
+    os.replace(tmp, out)
+    return out
+
+
 def build_all(verbose: bool = False) -> None:
     build_hip(verbose)
     build_cpu(verbose)
+    build_segs(verbose)
 
 
 if __name__ == "__main__":

@@ -21,13 +21,15 @@ from . import _native
 _B16 = (torch.bfloat16, torch.float16, torch.int16, torch.uint16)
 
 
-def _stream_ptr(stream: Optional[torch.cuda.Stream]) -> ctypes.c_void_p:
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return ctypes.c_void_p(s.cuda_stream)
+def _stream_ptr(stream: Optional[torch.cuda.Stream]) -> int:
+    if stream is not None:
+        return stream.cuda_stream
+    # torch.cuda.current_stream() makes a Stream object for it: 1.2 us
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _require_cuda(t: torch.Tensor, what: str) -> None:
-    if t.device.type != "cuda":
+    if not t.is_cuda:
         raise ValueError(f"{what} must be a GPU tensor, got {t.device}")
 
 
@@ -106,7 +108,7 @@ def cast_f32_bf16_(dst: torch.Tensor, src: torch.Tensor, stream: Optional[torch.
 def _check_stage_args(dst: torch.Tensor, host_src: torch.Tensor) -> None:
     if host_src.dtype != torch.float32 or dst.dtype != torch.bfloat16:
         raise TypeError(f"stage_f32_bf16_: need float32 -> bfloat16, got {host_src.dtype} -> {dst.dtype}")
-    if host_src.device.type != "cpu" or (host_src.numel() and not host_src.is_pinned()):
+    if not host_src.is_cpu or (host_src.numel() and not host_src.is_pinned()):
         raise ValueError("stage_f32_bf16_: the source must be a pinned host tensor")
     _require_cuda(dst, "dst")
     _require_contig(host_src, "host_src")
@@ -153,6 +155,12 @@ def _seg_array(segs: Sequence[Tuple[int, int, int]]):
 def cast_scatter_f32_bf16(pairs: Sequence[Tuple[torch.Tensor, torch.Tensor]],
                           stream: Optional[torch.cuda.Stream] = None) -> None:
     """For each (src fp32, dst bf16) pair of contiguous GPU tensors: dst = RNE(src)."""
+    fast = _native.segs().pair_table(pairs, True)
+    if fast is not None:
+        table, count = fast
+        _native.check(_native.hip().sf_cast_scatter_f32_bf16(table, count, _stream_ptr(stream)),
+                      "sf_cast_scatter_f32_bf16")
+        return
     segs = []
     for k, (src, dst) in enumerate(pairs):
         if src.dtype != torch.float32 or dst.dtype != torch.bfloat16:
@@ -172,7 +180,7 @@ def cast_scatter_f32_bf16(pairs: Sequence[Tuple[torch.Tensor, torch.Tensor]],
 def _check_b16(t: torch.Tensor, what: str, host_ok: bool = False) -> None:
     if t.dtype not in _B16:
         raise TypeError(f"{what}: need a 16-bit dtype, got {t.dtype}")
-    if host_ok and t.device.type == "cpu":
+    if host_ok and t.is_cpu:
         if not t.is_pinned():
             raise ValueError(f"{what}: a host tensor must be pinned to be written by a kernel")
     else:
@@ -180,10 +188,25 @@ def _check_b16(t: torch.Tensor, what: str, host_ok: bool = False) -> None:
     _require_contig(t, what)
 
 
+def _list_table(tensors: Sequence[torch.Tensor], name: str, as_dst: bool):
+    """Segment table of 16-bit GPU tensors (their addresses as destinations
+    or sources), the number of its entries and of its elements."""
+    fast = _native.segs().list_table(tensors, as_dst)
+    if fast is not None:
+        return fast
+    total = 0
+    segs = []
+    for k, t in enumerate(tensors):
+        _check_b16(t, f"{name}[{k}]")
+        segs.append((0, t.data_ptr(), t.numel()) if as_dst else (t.data_ptr(), 0, t.numel()))
+        total += t.numel()
+    return _seg_array(segs), len(segs), total
+
+
 def device_address(t: torch.Tensor) -> int:
     """Address at which a kernel reaches ``t``: its data pointer for a GPU
     tensor, the mapped device address of pinned host memory otherwise."""
-    if t.device.type == "cuda":
+    if t.is_cuda:
         return t.data_ptr()
     base = t.untyped_storage().data_ptr()
     dev = ctypes.c_void_p()
@@ -198,16 +221,10 @@ def pack_b16(srcs: Sequence[torch.Tensor], dst: torch.Tensor,
 
     ``dst`` may be pinned host memory (then pass a small ``max_workgroups``)."""
     _check_b16(dst, "dst", host_ok=True)
-    total = 0
-    segs = []
-    for k, s in enumerate(srcs):
-        _check_b16(s, f"srcs[{k}]")
-        segs.append((s.data_ptr(), 0, s.numel()))
-        total += s.numel()
+    table, count, total = _list_table(srcs, "srcs", as_dst=False)
     if total > dst.numel():
         raise ValueError(f"pack_b16: {total} elements do not fit in dst of {dst.numel()}")
-    arr = _seg_array(segs)
-    _native.check(_native.hip().sf_pack_b16(arr, len(segs), device_address(dst), int(max_workgroups),
+    _native.check(_native.hip().sf_pack_b16(table, count, device_address(dst), int(max_workgroups),
                                             _stream_ptr(stream)), "sf_pack_b16")
     return dst
 
@@ -217,6 +234,13 @@ def copy_segs_b16(pairs: Sequence[Tuple[torch.Tensor, torch.Tensor]],
     """For each (src, dst) pair of contiguous 16-bit tensors of equal numel,
     dst = src, all in one launch.  Sources are GPU tensors; destinations are
     GPU tensors or pinned host tensors."""
+    fast = _native.segs().pair_table(pairs, False)
+    if fast is not None:
+        table, count = fast
+        if count:
+            _native.check(_native.hip().sf_copy_segs_b16(table, count, int(max_workgroups), _stream_ptr(stream)),
+                          "sf_copy_segs_b16")
+        return
     segs = []
     for k, (src, dst) in enumerate(pairs):
         _check_b16(src, f"pair {k} src")
@@ -236,16 +260,10 @@ def unpack_b16(src: torch.Tensor, dsts: Sequence[torch.Tensor],
     """dsts[k].flatten() = src[off_k : off_k + n_k], the inverse of pack_b16.
     ``src`` may be pinned host memory."""
     _check_b16(src, "src", host_ok=True)
-    total = 0
-    segs = []
-    for k, d in enumerate(dsts):
-        _check_b16(d, f"dsts[{k}]")
-        segs.append((0, d.data_ptr(), d.numel()))
-        total += d.numel()
+    table, count, total = _list_table(dsts, "dsts", as_dst=True)
     if total > src.numel():
         raise ValueError(f"unpack_b16: src of {src.numel()} holds fewer than {total} elements")
-    arr = _seg_array(segs)
-    _native.check(_native.hip().sf_unpack_b16(device_address(src), arr, len(segs), int(max_workgroups),
+    _native.check(_native.hip().sf_unpack_b16(device_address(src), table, count, int(max_workgroups),
                                               _stream_ptr(stream)), "sf_unpack_b16")
 
 
@@ -278,13 +296,13 @@ def gather_rows(table: torch.Tensor, ids: torch.Tensor, dst: torch.Tensor, bad: 
     if dst.element_size() != 2 or dst.numel() < ids.numel() * row_len:
         raise ValueError("gather_rows: dst must be 16-bit with room for len(ids) rows")
     for t, what in ((table, "table"), (dst, "dst")):
-        if t.device.type == "cpu" and not t.is_pinned():
+        if t.is_cpu and not t.is_pinned():
             raise ValueError(f"gather_rows: a host {what} must be pinned")
     bad_ptr = None
     if bad is not None:
         if bad.element_size() != 4 or bad.numel() < 1:
             raise ValueError("gather_rows: bad must hold one 32-bit word")
-        if bad.device.type == "cpu" and not bad.is_pinned():
+        if bad.is_cpu and not bad.is_pinned():
             raise ValueError("gather_rows: a host bad flag must be pinned")
         bad_ptr = device_address(bad)
     if table.dtype == torch.float32:
