@@ -229,6 +229,17 @@ int sf_ce_rows(void* logits, int dtype, size_t ld, size_t rows, size_t vocab,
                const int64_t* labels, int64_t ignore_index, float* row_loss,
                sf_stream_t stream);
 
+/* The operands of the weight gradient's product, whose sum runs over the
+ * rows, padded to ldt of them (rows rounded up to a multiple of 64; SF_EINVAL
+ * otherwise): hidden_t[j, i] = hidden[i, j] of the 16-bit [rows, cols] array
+ * with ldh elements from row to row, 0 for rows <= i < ldt; and the ldt - rows
+ * rows of ld_tail 16-bit elements at `tail`, which follow the logits' last
+ * row, cleared.  hidden_t and tail start on 16-byte boundaries, ld_tail is a
+ * multiple of 8 (SF_EALIGN); tail is not read where ldt == rows. */
+int sf_ce_hidden(const void* hidden, size_t ldh, size_t rows, size_t cols,
+                 void* hidden_t, size_t ldt, void* tail, size_t ld_tail,
+                 sf_stream_t stream);
+
 /* *n_valid = number of labels != ignore_index, *loss = sum of row_loss over
  * it (NaN if there are none), both in device memory. */
 int sf_ce_loss(const float* row_loss, const int64_t* labels, size_t n,

@@ -12,9 +12,11 @@
 // TB/s; a device copy reaches 5.1), ce_scale16_kernel for the 128256 x 4096
 // weight and 4092 x 4096 hidden gradients 0.521 ms (6.1 TB/s).  The same steps
 // as torch operations took 7.2 ms, and adding the chunks' weight gradients
-// into the fp32 sum 8.1 ms more; loss with both gradients 35.1 -> 11.3 ms, of
-// which 10.8 are the products.  At 510 rows of 4096 (hidden 512): 453 -> 263
-// us, 57 of them on the GPU, the rest host time of the launches.
+// into the fp32 sum 8.1 ms more; loss with both gradients 35.1 -> 11.3 ms.  With
+// the hidden rows transposed for the weight gradient's product
+// (ce_hidden_kernel) 10.4, of which 9.5 are the products.  At 510 rows of 4096
+// (hidden 512): 453 -> 230 us, 57 of them on the GPU, the rest host time of the
+// launches.
 //
 // The C ABI is declared in include/slidefsdp.h.
 
@@ -359,6 +361,69 @@ __global__ __launch_bounds__(kScaleThreads) void ce_scale32_kernel(
     for (uint64_t j = i; j < n && j < i + kGroup; ++j) dst[j] = src[j] * scale;
 }
 
+// The chunk's hidden rows transposed, [hidden, tokens], for the product of the
+// weight gradient, whose sum runs over the tokens: with one operand laid out
+// along the sum, and the sum's length a multiple of 64, the product is up to a
+// third faster.  us, hidden rows as they are | transposed and padded, at tokens
+// x hidden x vocabulary: 4092 x 4096 x 128256 4198 | 3490, 2046 x 2560 x 151936
+// 1773 | 1474, 3001 x 5120 x 65000 2001 | 1662, 1023 x 4096 x 128256 1438 |
+// 1217, 777 x 1024 x 32000 79.9 | 68.6, 127 x 4096 x 128256 708 | 474.  (The
+// gradient of the logits transposed too: 3355, which its 0.4 ms does not pay.)
+//
+// Bound by HBM: 4 bytes per element, 67 MB at the first of these sizes.  A
+// workgroup takes a tile of 64 x 64 through LDS, 128-bit accesses on both
+// sides.  Rows of 66 elements in LDS put the 8 lanes that read 8 rows each, and
+// the 8 columns beside each other in a wave, into banks of their own.  The
+// same launch clears the rows of the gradient of the logits that pad the sum
+// (workgroups from `tiles` on).
+constexpr int kTr = 64;
+constexpr int kTrThreads = 256;
+constexpr int kTrLd = kTr + 2;
+template <bool kVec>   // rows on 16-byte boundaries, hidden a multiple of 8
+__global__ __launch_bounds__(kTrThreads) void ce_hidden_kernel(const uint16_t* __restrict__ hidden, uint64_t ldh,
+                                                               uint64_t rows, uint64_t cols, uint16_t* __restrict__ out,
+                                                               uint64_t ldt, uint32_t tiles, u32x4* __restrict__ tail,
+                                                               uint64_t tail_groups) {
+    __shared__ __attribute__((aligned(16))) uint16_t tile[kTr * kTrLd];
+    if (blockIdx.x >= tiles) {
+        const uint64_t stride = uint64_t(gridDim.x - tiles) * kTrThreads;
+        for (uint64_t g = uint64_t(blockIdx.x - tiles) * kTrThreads + threadIdx.x; g < tail_groups; g += stride)
+            tail[g] = u32x4{0, 0, 0, 0};
+        return;
+    }
+    const uint32_t across = uint32_t(ldt / kTr);
+    const uint64_t row0 = uint64_t(blockIdx.x % across) * kTr, col0 = uint64_t(blockIdx.x / across) * kTr;
+#pragma unroll
+    for (int k = 0; k < kTr * kTr / kGroup / kTrThreads; ++k) {
+        const uint32_t g = k * kTrThreads + threadIdx.x, r = g / (kTr / kGroup), c = g % (kTr / kGroup) * kGroup;
+        u32x4 v = {0, 0, 0, 0};
+        if (row0 + r < rows) {
+            const uint16_t* p = hidden + (row0 + r) * ldh + col0 + c;
+            if (kVec) {
+                if (col0 + c < cols) v = *reinterpret_cast<const u32x4*>(p);
+            } else {
+#pragma unroll
+                for (int j = 0; j < kGroup; ++j)
+                    if (col0 + c + j < cols) v[j / 2] |= uint32_t(p[j]) << (j % 2 * 16);
+            }
+        }
+        uint32_t* t = reinterpret_cast<uint32_t*>(tile + r * kTrLd + c);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) t[j] = v[j];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kTr * kTr / kGroup / kTrThreads; ++k) {
+        const uint32_t g = k * kTrThreads + threadIdx.x, c = g / (kTr / kGroup), r = g % (kTr / kGroup) * kGroup;
+        if (col0 + c >= cols) continue;
+        u32x4 v;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            v[j] = uint32_t(tile[(r + 2 * j) * kTrLd + c]) | uint32_t(tile[(r + 2 * j + 1) * kTrLd + c]) << 16;
+        *reinterpret_cast<u32x4*>(out + (col0 + c) * ldt + row0 + r) = v;
+    }
+}
+
 inline int status() {
     // the runtime keeps a failed launch as the thread's last error: reading it clears it
     return int(hipGetLastError());
@@ -425,6 +490,27 @@ int sf_ce_rows(void* logits, int dtype, size_t ld, size_t rows, size_t vocab, co
         dispatch_rows16<Bf16>(x, ld, rows, uint32_t(vocab), labels, ignore_index, row_loss, st);
     else
         dispatch_rows16<F16>(x, ld, rows, uint32_t(vocab), labels, ignore_index, row_loss, st);
+    return status();
+}
+
+int sf_ce_hidden(const void* hidden, size_t ldh, size_t rows, size_t cols, void* hidden_t, size_t ldt, void* tail,
+                 size_t ld_tail, sf_stream_t stream) {
+    if (rows == 0 || cols == 0) return SF_OK;
+    if (hidden == nullptr || hidden_t == nullptr || ldh < cols || ldt % kTr != 0 || ldt < rows || ldt - rows >= kTr)
+        return SF_EINVAL;
+    if (ldt > rows && (tail == nullptr || ld_tail == 0)) return SF_EINVAL;
+    if (misaligned(hidden, 2)) return SF_EINVAL;
+    if (misaligned(hidden_t, 16) || (ldt > rows && (misaligned(tail, 16) || ld_tail % kGroup != 0))) return SF_EALIGN;
+    const uint64_t tiles = uint64_t(ldt / kTr) * ((cols + kTr - 1) / kTr);
+    const uint64_t groups = uint64_t(ldt - rows) * (ldt > rows ? ld_tail / kGroup : 0);
+    // one group per lane of the cleared rows, in at most 2,048 workgroups
+    const uint64_t want = (groups + kTrThreads - 1) / kTrThreads, clear = want < 2048 ? want : 2048;
+    if (tiles + clear > (uint64_t(1) << 31) / kTrThreads) return SF_EINVAL;
+    const bool vec = !misaligned(hidden, 16) && ldh % kGroup == 0 && cols % kGroup == 0;
+    hipLaunchKernelGGL((vec ? ce_hidden_kernel<true> : ce_hidden_kernel<false>), dim3(uint32_t(tiles + clear)),
+                       dim3(kTrThreads), 0, reinterpret_cast<hipStream_t>(stream), static_cast<const uint16_t*>(hidden),
+                       uint64_t(ldh), uint64_t(rows), uint64_t(cols), static_cast<uint16_t*>(hidden_t), uint64_t(ldt),
+                       uint32_t(tiles), static_cast<u32x4*>(tail), groups);
     return status();
 }
 

@@ -350,6 +350,29 @@ def ce_rows_(logits: torch.Tensor, labels: torch.Tensor, ignore_index: int, row_
                                            _stream_ptr(stream)), "sf_ce_rows")
 
 
+def ce_hidden(hidden: torch.Tensor, hidden_t: torch.Tensor, logits: torch.Tensor,
+              stream: Optional[torch.cuda.Stream] = None) -> None:
+    """``hidden_t[:, :n] = hidden.T`` for the [n, H] 16-bit ``hidden`` with unit
+    column stride; the columns up to ``hidden_t``'s width, n rounded up to a
+    multiple of 64, and the rows from n on of the contiguous ``logits`` of that
+    many rows are cleared."""
+    n, h = hidden.shape
+    pad = hidden_t.shape[1]
+    if hidden.element_size() != 2 or hidden_t.dtype != hidden.dtype or logits.dtype != hidden.dtype:
+        raise TypeError("ce_hidden: need 16-bit tensors of one type")
+    if hidden.stride(1) != 1 or hidden_t.shape != (h, -(-n // 64) * 64) or logits.dim() != 2 or logits.shape[0] != pad:
+        raise ValueError("ce_hidden: hidden [n, H] with unit column stride, hidden_t [H, P] and logits [P, V] expected, "
+                         "P = n rounded up to a multiple of 64")
+    for t, what in ((hidden, "hidden"), (hidden_t, "hidden_t"), (logits, "logits")):
+        _require_cuda(t, what)
+    _require_contig(hidden_t, "hidden_t")
+    _require_contig(logits, "logits")
+    ldh = hidden.stride(0) if n > 1 else max(hidden.stride(0), h)
+    tail = logits.data_ptr() + n * logits.stride(0) * 2 if pad > n else None
+    _native.check(_native.hip().sf_ce_hidden(hidden.data_ptr(), ldh, n, h, hidden_t.data_ptr(), pad, tail,
+                                             logits.shape[1], _stream_ptr(stream)), "sf_ce_hidden")
+
+
 def ce_loss(row_loss: torch.Tensor, labels: torch.Tensor, ignore_index: int, loss: torch.Tensor,
             n_valid: torch.Tensor, stream: Optional[torch.cuda.Stream] = None) -> None:
     """``n_valid`` = labels that are not ``ignore_index``, ``loss`` = sum of
