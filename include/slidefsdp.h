@@ -240,6 +240,18 @@ int sf_ce_hidden(const void* hidden, size_t ldh, size_t rows, size_t cols,
                  void* hidden_t, size_t ldt, void* tail, size_t ld_tail,
                  sf_stream_t stream);
 
+/* The hidden gradient from its product's sum over the vocabulary taken in
+ * nparts parts (2, 4, 8 or 16): out[i, j] (dtype SF_DTYPE_BF16 or
+ * SF_DTYPE_F16, [rows, cols]) = the sum of parts[s, i, j] over s and of
+ * g_tail[i, k] * w_tail[k, j] over k < tail, in fp32, rounded once.  tail, less
+ * than 8 nparts, counts the terms that no part holds: columns of the 16-bit
+ * gradient of the logits (ld elements from row to row) and rows of the
+ * weight.  cols is a multiple of 8; parts, out and w_tail start on 16-byte
+ * boundaries (SF_EALIGN). */
+int sf_ce_sum(const float* parts, int nparts, size_t rows, size_t cols,
+              void* out, int dtype, const void* g_tail, size_t ld,
+              const void* w_tail, size_t tail, sf_stream_t stream);
+
 /* *n_valid = number of labels != ignore_index, *loss = sum of row_loss over
  * it (NaN if there are none), both in device memory. */
 int sf_ce_loss(const float* row_loss, const int64_t* labels, size_t n,

@@ -14,7 +14,7 @@
 // as torch operations took 7.2 ms, and adding the chunks' weight gradients
 // into the fp32 sum 8.1 ms more; loss with both gradients 35.1 -> 11.3 ms.  With
 // the hidden rows transposed for the weight gradient's product
-// (ce_hidden_kernel) 10.4, of which 9.5 are the products.  At 510 rows of 4096
+// (ce_hidden_kernel) 10.3, of which 9.4 are the products.  At 510 rows of 4096
 // (hidden 512): 453 -> 230 us, 57 of them on the GPU, the rest host time of the
 // launches.
 //
@@ -424,6 +424,59 @@ __global__ __launch_bounds__(kTrThreads) void ce_hidden_kernel(const uint16_t* _
     }
 }
 
+// The hidden gradient's product sums over the vocabulary, and for most shapes
+// [tokens, hidden] has too few tiles for the chip: the sum is taken in kParts
+// parts side by side (one batched product into fp32), and this kernel adds
+// them up and rounds once.  A part's length is a multiple of 8, so that every
+// operand starts on a 16-byte boundary; the up to 8 kParts - 1 terms that
+// leaves are summed here.  A whole call, one product | parts and this kernel,
+// us, tokens x hidden x vocabulary: 1023 x 4096 x 128256 4200 | 3504, 777 x
+// 1024 x 32000 371 | 285.  Bound by the parts' reads, at most 134 MB, which the
+// last-level cache still holds in part.
+constexpr int kSumThreads = 128;
+template <typename Fmt, int kParts>
+__global__ __launch_bounds__(kSumThreads) void ce_sum_kernel(const float* __restrict__ parts, uint32_t count,
+                                                             uint32_t cols, uint16_t* __restrict__ out,
+                                                             const uint16_t* __restrict__ g, uint64_t ld,
+                                                             const uint16_t* __restrict__ w, uint32_t tail) {
+    const uint32_t i = (blockIdx.x * kSumThreads + threadIdx.x) * kGroup;
+    if (i >= count) return;
+    f32x4 a[kParts], b[kParts];
+#pragma unroll
+    for (int s = 0; s < kParts; ++s) {
+        const f32x4* p = reinterpret_cast<const f32x4*>(parts + uint64_t(s) * count + i);
+        a[s] = __builtin_nontemporal_load(p);
+        b[s] = __builtin_nontemporal_load(p + 1);
+    }
+    // neighbours first: a tree, whose rounding error grows with log2(kParts)
+#pragma unroll
+    for (int d = 1; d < kParts; d *= 2)
+#pragma unroll
+        for (int s = 0; s < kParts; s += 2 * d) {
+            a[s] += a[s + d];
+            b[s] += b[s + d];
+        }
+    if (tail > 0) {
+        const uint32_t row = i / cols, col = i - row * cols;
+        f32x4 ta = {0.0f, 0.0f, 0.0f, 0.0f}, tb = ta;
+#pragma unroll 4
+        for (uint32_t k = 0; k < tail; ++k) {
+            const float f = Fmt::lo(g[row * ld + k]);
+            const u32x4 v = *reinterpret_cast<const u32x4*>(w + uint64_t(k) * cols + col);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                ta[2 * j] = fmaf(f, Fmt::lo(v[j]), ta[2 * j]);
+                ta[2 * j + 1] = fmaf(f, Fmt::hi(v[j]), ta[2 * j + 1]);
+                tb[2 * j] = fmaf(f, Fmt::lo(v[j + 2]), tb[2 * j]);
+                tb[2 * j + 1] = fmaf(f, Fmt::hi(v[j + 2]), tb[2 * j + 1]);
+            }
+        }
+        a[0] += ta;
+        b[0] += tb;
+    }
+    *reinterpret_cast<u32x4*>(out + i) = pack8<Fmt>(a[0], b[0]);
+}
+
 inline int status() {
     // the runtime keeps a failed launch as the thread's last error: reading it clears it
     return int(hipGetLastError());
@@ -436,6 +489,19 @@ void launch_rows(uint16_t* x, uint64_t ld, uint64_t rows, uint32_t vocab, const 
                  float* row_loss, hipStream_t st) {
     hipLaunchKernelGGL((ce_rows_kernel<Fmt, kT, kG, kFull>), dim3(uint32_t(rows)), dim3(kT), 0, st, x, ld, vocab, labels,
                        ignore, row_loss);
+}
+
+template <typename Fmt>
+int launch_sum(int nparts, const float* parts, uint32_t count, uint32_t cols, void* out, const void* g, size_t ld,
+               const void* w, uint32_t tail, hipStream_t st) {
+    const auto kernel = nparts == 2   ? ce_sum_kernel<Fmt, 2>
+                        : nparts == 4 ? ce_sum_kernel<Fmt, 4>
+                        : nparts == 8 ? ce_sum_kernel<Fmt, 8>
+                                      : ce_sum_kernel<Fmt, 16>;
+    hipLaunchKernelGGL(kernel, dim3((count / kGroup + kSumThreads - 1) / kSumThreads), dim3(kSumThreads), 0, st, parts,
+                       count, cols, static_cast<uint16_t*>(out), static_cast<const uint16_t*>(g), uint64_t(ld),
+                       static_cast<const uint16_t*>(w), tail);
+    return status();
 }
 
 // The smallest workgroup that holds the row: lanes first (up to 1024), then
@@ -512,6 +578,26 @@ int sf_ce_hidden(const void* hidden, size_t ldh, size_t rows, size_t cols, void*
                        uint64_t(ldh), uint64_t(rows), uint64_t(cols), static_cast<uint16_t*>(hidden_t), uint64_t(ldt),
                        uint32_t(tiles), static_cast<u32x4*>(tail), groups);
     return status();
+}
+
+int sf_ce_sum(const float* parts, int nparts, size_t rows, size_t cols, void* out, int dtype, const void* g_tail,
+              size_t ld, const void* w_tail, size_t tail, sf_stream_t stream) {
+    if (rows == 0 || cols == 0) return SF_OK;
+    if (parts == nullptr || out == nullptr || (nparts != 2 && nparts != 4 && nparts != 8 && nparts != 16))
+        return SF_EINVAL;
+    if (tail >= size_t(kGroup) * size_t(nparts) || (tail > 0 && (g_tail == nullptr || w_tail == nullptr || ld < tail)))
+        return SF_EINVAL;
+    if (cols > (size_t(1) << 31) || rows > (size_t(1) << 31) / cols) return SF_EINVAL;
+    if (cols % kGroup != 0 || misaligned(parts, 16) || misaligned(out, 16) || (tail > 0 && misaligned(w_tail, 16)) ||
+        (tail > 0 && misaligned(g_tail, 2)))
+        return SF_EALIGN;
+    const uint32_t count = uint32_t(rows * cols);
+    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    if (dtype == SF_DTYPE_BF16)
+        return launch_sum<Bf16>(nparts, parts, count, uint32_t(cols), out, g_tail, ld, w_tail, uint32_t(tail), st);
+    if (dtype == SF_DTYPE_F16)
+        return launch_sum<F16>(nparts, parts, count, uint32_t(cols), out, g_tail, ld, w_tail, uint32_t(tail), st);
+    return SF_EDTYPE;
 }
 
 int sf_ce_loss(const float* row_loss, const int64_t* labels, size_t n, int64_t ignore_index, float* loss,

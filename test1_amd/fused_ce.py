@@ -77,6 +77,57 @@ def _transposed_hidden_pays(rows: int, hidden: torch.Tensor, vocab: int) -> bool
             and 2 * rows * hidden.shape[1] * vocab >= 1 << 35)
 
 
+def _vocabulary_parts(rows: int, weight: torch.Tensor) -> int:
+    """Parts in which the hidden gradient's product of a chunk of ``rows`` sums
+    over the vocabulary (1: the product as it is).  The library sums each of
+    its 256 x 256 tiles in one workgroup; with as many parts as give every
+    compute unit one, at most 16 (powers of two: three, five or six parts ran
+    slower than two, four or eight), us, one product | parts before they are
+    added up, tokens x hidden x vocabulary: 1023 x 4096 x 128256 1461 | 807,
+    510 x 4096 x 32000 299 | 134, 777 x 1024 x 32000 174 | 69, 4000 x 768 x
+    30522 287 | 203.  Above 64 tiles a shape gains or loses (whole calls: 2046
+    x 2560 x 151936, 80 tiles, 5776 | 5362, of a 60000 vocabulary 1863 | 1989,
+    3500 x 1536 x 152064, 84 tiles, 6617 | 7454), as it does with short sums
+    (the product alone, 510 x 512 x 4096 19.2 | 17.9).  The parts are at most
+    512 tiles of fp32.  Adding them up is a launch more, which makes a call that
+    the host's 240 us bound 20 us slower (300 x 1024 x 17000, 64 x 1024 x
+    30000, 250 x 1024 x 32000); so only where the call moves 800 MB or its
+    products take 34 GFLOP each (whole calls: 4000 x 64 x 30522, 1.2 GB, 386 |
+    312; 100 x 2560 x 32000, 1.2 GB, 348 | 274; 777 x 1024 x 32000, 51 GFLOP,
+    380 | 286; 4092 x 1024 x 50257 in chunks of 256 6073 | 3654).  Operands that
+    start on 16-byte boundaries only."""
+    v, h = weight.shape
+    tiles = -(-rows // 256) * -(-h // 256)
+    if (weight.element_size() != 2 or tiles > 64 or v < 16384 or h % 8 != 0 or not weight.is_contiguous()
+            or weight.data_ptr() % 16 != 0):
+        return 1
+    # the weight read twice, its gradient written in fp32 and rounded; the
+    # logits written, turned into their gradient in place and read twice
+    moved = (14 * h + 10 * rows) * v
+    if moved < 800 << 20 and 2 * rows * h * v < 1 << 35:
+        return 1
+    parts = 2
+    while parts < 16 and parts * tiles < 256:
+        parts *= 2
+    return parts
+
+
+def _grad_hidden(g: torch.Tensor, ld: int, weight: torch.Tensor, out: torch.Tensor, scratch) -> None:
+    """out = g @ weight for the gradient of a chunk's logits, ``ld`` elements
+    from row to row.  ``scratch(elements)``: fp32 memory for the parts."""
+    n, v = g.shape
+    h = weight.shape[1]
+    nparts = _vocabulary_parts(n, weight)
+    if nparts == 1:
+        torch.mm(g, weight, out=out)
+        return
+    part = v // nparts // 8 * 8
+    parts = scratch(nparts * n * h).view(nparts, n, h)
+    torch.bmm(g.as_strided((nparts, n, part), (part, ld, 1)), weight[:nparts * part].view(nparts, part, h),
+              out_dtype=torch.float32, out=parts)
+    kernels.ce_grad_hidden(g, weight, parts, out)
+
+
 def _forward_kernels(ctx, hidden: torch.Tensor, weight: torch.Tensor, labels: torch.Tensor, ignore_index: int,
                      chunk_rows: int) -> torch.Tensor:
     n, h = hidden.shape
@@ -105,7 +156,10 @@ def _forward_kernels(ctx, hidden: torch.Tensor, weight: torch.Tensor, labels: to
         g = buf[:e - s, :v]
         torch.mm(hc, wt, out=g)
         kernels.ce_rows_(g, labels[s:e], ignore_index, row_loss[s:e])
-        torch.mm(g, weight, out=grad_hidden[s:e])
+        # the weight gradient's memory is free until its first product
+        _grad_hidden(g, ld, weight, grad_hidden[s:e],
+                     lambda k: (grad_weight.view(-1)[:k] if s == 0 and k <= grad_weight.numel()
+                                else torch.empty(k, dtype=torch.float32, device=dev)))
         if transposed:
             pad = height(e - s)
             ht = hidden_t[:h * pad].view(h, pad)

@@ -373,6 +373,29 @@ def ce_hidden(hidden: torch.Tensor, hidden_t: torch.Tensor, logits: torch.Tensor
                                              logits.shape[1], _stream_ptr(stream)), "sf_ce_hidden")
 
 
+def ce_grad_hidden(g: torch.Tensor, weight: torch.Tensor, parts: torch.Tensor, out: torch.Tensor,
+                   stream: Optional[torch.cuda.Stream] = None) -> None:
+    """``out`` = what the [S, n, H] fp32 ``parts`` add up to, rounded once, for
+    ``parts[s] = g[:, s c:(s + 1) c] @ weight[s c:(s + 1) c]`` with c = V // S
+    rounded down to a multiple of 8; the terms behind S c are added here."""
+    nparts, n, h = parts.shape
+    v = weight.shape[0]
+    done = nparts * (v // nparts // 8 * 8)
+    if g.dtype != weight.dtype or out.dtype != g.dtype or parts.dtype != torch.float32 or g.element_size() != 2:
+        raise TypeError("ce_grad_hidden: need 16-bit tensors of one type and float32 parts")
+    if g.shape != (n, v) or g.stride(1) != 1 or weight.shape != (v, h) or out.shape != (n, h):
+        raise ValueError("ce_grad_hidden: g [n, V] with unit column stride, weight [V, H], parts [S, n, H] and out "
+                         "[n, H] expected")
+    for t, what in ((weight, "weight"), (parts, "parts"), (out, "out")):
+        _require_cuda(t, what)
+        _require_contig(t, what)
+    _require_cuda(g, "g")
+    ld = g.stride(0) if n > 1 else max(g.stride(0), v)
+    _native.check(_native.hip().sf_ce_sum(parts.data_ptr(), nparts, n, h, out.data_ptr(), _CE_DTYPES[g.dtype],
+                                          g.data_ptr() + 2 * done, ld, weight.data_ptr() + 2 * done * h, v - done,
+                                          _stream_ptr(stream)), "sf_ce_sum")
+
+
 def ce_loss(row_loss: torch.Tensor, labels: torch.Tensor, ignore_index: int, loss: torch.Tensor,
             n_valid: torch.Tensor, stream: Optional[torch.cuda.Stream] = None) -> None:
     """``n_valid`` = labels that are not ``ignore_index``, ``loss`` = sum of

@@ -1,5 +1,5 @@
-"""What the fused output unit prepares for its products: the transposed,
-padded hidden rows."""
+"""What the fused output unit does around its products: the transposed,
+padded hidden rows, and the sum over the vocabulary in parts."""
 
 import pytest
 import torch
@@ -58,3 +58,68 @@ def test_weight_gradient_from_transposed_rows(dev, monkeypatch, n, h, v, chunk, 
     got, plain, ref = both(dev, monkeypatch, dtype, n, h, v, chunk, "_transposed_hidden_pays", True, False)
     assert torch.equal(got[0], plain[0]) and torch.equal(got[1], plain[1])
     assert rel(got[2], ref[2]) <= 1.1 * rel(plain[2], ref[2]) + 1e-6
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n,h,v", [(1, 8, 64), (3, 72, 128), (5, 64, 255), (130, 264, 1031)])
+@pytest.mark.parametrize("nparts", [2, 4, 8, 16])
+def test_parts_are_added_up_with_what_they_leave(dev, nparts, n, h, v, dtype):
+    gen = torch.Generator(device=dev).manual_seed(v)
+    g = (torch.randn(n, v + 5, generator=gen, device=dev)).to(dtype)[:, :v]
+    w = (torch.randn(v, h, generator=gen, device=dev)).to(dtype)
+    parts = torch.randn(nparts, n, h, generator=gen, device=dev)
+    out = torch.empty(n, h, dtype=dtype, device=dev)
+    kernels.ce_grad_hidden(g, w, parts, out)
+    done = nparts * (v // nparts // 8 * 8)
+    terms = torch.cat([parts.double().flatten(1).t(),
+                       (g[:, done:].double().unsqueeze(2) * w[done:].double().unsqueeze(0)).transpose(1, 2)
+                       .reshape(n * h, v - done)], dim=1)
+    want = terms.sum(1).view(n, h)
+    # fp32 additions of at most 16 + 127 + 1 terms, then half a unit in the last of 8 or 11 bits
+    bound = 144 * 2.0 ** -24 * terms.abs().sum(1).view(n, h)
+    half = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    assert ((out.double() - want).abs() <= half * want.abs() + (1 + half) * bound + 2.0 ** -25).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n,h,v,chunk,nparts", [(1, 64, 1003, 0, 16), (127, 72, 5001, 0, 8), (300, 64, 1003, 128, 4),
+                                                (300, 256, 32_000, 70, 2)])
+def test_hidden_gradient_summed_in_parts(dev, monkeypatch, n, h, v, chunk, nparts, dtype):
+    """No further from float64 than one sum: parts of it in fp32, rounded once."""
+    got, plain, ref = both(dev, monkeypatch, dtype, n, h, v, chunk, "_vocabulary_parts", nparts, 1)
+    assert torch.equal(got[0], plain[0]) and torch.equal(got[2], plain[2])
+    assert rel(got[1], ref[1]) <= 1.1 * rel(plain[1], ref[1]) + 1e-6
+
+
+def test_parts_and_transposed_rows_in_a_captured_graph(dev, monkeypatch):
+    """Replays with eager work between them; three chunks, the last one ragged."""
+    monkeypatch.setattr(fused_ce, "_vocabulary_parts", lambda *a: 4)
+    monkeypatch.setattr(fused_ce, "_transposed_hidden_pays", lambda *a: True)
+    gen = torch.Generator(device=dev).manual_seed(5)
+    hid = torch.randn(150, 64, generator=gen, device=dev).bfloat16().requires_grad_(True)
+    wgt = (torch.randn(1900, 64, generator=gen, device=dev) * 0.05).bfloat16().requires_grad_(True)
+    y = torch.randint(0, 1900, (150,), generator=gen, device=dev)
+
+    def step():
+        loss = chunked_linear_cross_entropy(hid, wgt, y, chunk_rows=64)
+        return (loss, *torch.autograd.grad(loss, (hid, wgt)))
+
+    want = [t.detach().clone() for t in step()]
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        step()
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = step()
+    for rep in range(4):
+        for t in out:
+            t.detach().fill_(float(rep + 7))
+        step()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        for t, w in zip(out, want):
+            assert torch.equal(t.detach(), w), rep
