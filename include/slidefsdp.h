@@ -266,6 +266,20 @@ int sf_ce_scale(const float* grad_loss, const float* n_valid,
                 const float* grad_w, void* grad_w_out, size_t n_w, int dtype,
                 sf_stream_t stream);
 
+/* Both gradients of up to 256 tokens times *grad_loss / *n_valid, the weight's
+ * from its factors: grad_w_out[v, j] = the sum of g[i, v] * hidden_t[j, i] over
+ * i < tokens (in fp32), scaled and rounded once, and grad_h (n_h elements)
+ * into grad_h_out.  g: the gradient of the logits, `tokens` rows (a multiple
+ * of 64; the padding rows and hidden_t's padding columns as sf_ce_hidden
+ * leaves them) of ld elements; grad_w_out [vocab, hidden].  All 16-bit, of
+ * dtype; ld, hidden and n_h are multiples of 8, the arrays start on 16-byte
+ * boundaries (SF_EALIGN). */
+int sf_ce_weight_grad(const float* grad_loss, const float* n_valid,
+                      const void* g, size_t ld, size_t vocab,
+                      const void* hidden_t, size_t tokens, size_t hidden,
+                      void* grad_w_out, const void* grad_h, void* grad_h_out,
+                      size_t n_h, int dtype, sf_stream_t stream);
+
 /* ---------------------------------------------------------------------
  * Copies and pinned host memory (libsf_hip.so)
  * ------------------------------------------------------------------- */

@@ -91,6 +91,7 @@ HIP_SIGNATURES = {
     "sf_ce_hidden": [_vp, _sz, _sz, _sz, _vp, _sz, _vp, _sz, _vp],
     "sf_ce_sum": [_vp, _i, _sz, _sz, _vp, _i, _vp, _sz, _vp, _sz, _vp],
     "sf_ce_loss": [_vp, _vp, _sz, ctypes.c_int64, _vp, _vp, _vp],
+    "sf_ce_weight_grad": [_vp, _vp, _vp, _sz, _sz, _vp, _sz, _sz, _vp, _vp, _vp, _sz, _i, _vp],
     "sf_ce_scale": [_vp, _vp, _vp, _vp, _sz, _vp, _vp, _sz, _i, _vp],
     "sf_stage_f32_bf16": [_vp, _vp, _sz, _vp, _sz, _vp],
     "sf_stage_f32_bf16_noalloc": [_vp, _vp, _sz, _sz, _vp],

@@ -477,6 +477,120 @@ __global__ __launch_bounds__(kSumThreads) void ce_sum_kernel(const float* __rest
     *reinterpret_cast<u32x4*>(out + i) = pack8<Fmt>(a[0], b[0]);
 }
 
+// The weight gradient of up to 256 tokens, [vocabulary, hidden], by the matrix
+// cores with the scaling at the end, and the hidden gradient's scaling in the
+// same launch.  With so few tokens its operands are small beside it and it is
+// bound by its own bytes; as a product into fp32 that another kernel scales
+// and rounds, it cost 10 bytes an element instead of 2.  Loss with both
+// gradients, product and scaling | this, us, tokens x hidden x vocabulary: 4 x
+// 4096 x 128256 1461 | 847, 1 x 5120 x 65000 906 | 565, 32 x 768 x 152064 398 |
+// 304, 127 x 4096 x 128256 1455 | 1033, 200 x 4096 x 32000 467 | 380, 256 x 4096
+// x 128256 1757 | 1555, 250 x 1024 x 32000 240 | 233.  Beyond, the operands no
+// longer fit the registers of two waves per SIMD with four tiles each, and with
+// two the loads of the hidden rows bind it: 300 x 2560 x 50257 591 | 658, 510 x
+// 4096 x 32000 635 | 852.
+//
+// A wave owns 16 kV columns of the gradient of the logits, all tokens of them,
+// as operands in registers, and walks over the hidden dimension 32 at a time
+// with the transposed hidden rows (from the caches: at most 256 tokens by
+// hidden).  Both index maps are permuted for wide accesses: the column of
+// lane l in tile t is kV (l % 16) + t, so that a lane reads kV neighbours of a
+// token at once, and the four hidden rows of lane l in tile u start at 8 (l /
+// 16) + 4 u, so that it ends up with 8 neighbours and stores 16 bytes.
+// Products of 16 x 16 x 32: operand lanes hold row or column l % 16, terms 8
+// (l / 16) to + 7; result lanes column l % 16, rows 4 (l / 16) to + 3.
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+__device__ __forceinline__ f32x4 mfma(Bf16, u32x4 a, u32x4 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0,
+                                                   0, 0);
+}
+__device__ __forceinline__ f32x4 mfma(F16, u32x4 a, u32x4 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0,
+                                                  0);
+}
+
+constexpr int kWgThreads = 256;
+constexpr int kWgTokens = 256;
+constexpr int kWgStep = 32;   // hidden rows a wave takes at once
+constexpr int kV = 4;         // tiles of 16 columns a wave owns
+constexpr int kWgColumns = kWgThreads / 64 * 16 * kV;   // of a workgroup
+
+template <typename Fmt, int kSteps>   // at least tokens / 32
+__global__ __launch_bounds__(kWgThreads, 2) void ce_weight_grad_kernel(
+    const float* __restrict__ grad_loss, const float* __restrict__ n_valid, const uint16_t* __restrict__ g, uint64_t ld,
+    uint32_t vocab, const uint16_t* __restrict__ hidden_t, uint32_t tokens, uint32_t hidden, uint16_t* __restrict__ out,
+    uint32_t col_blocks, uint32_t per_block, uint32_t w_blocks, const uint16_t* __restrict__ h,
+    uint16_t* __restrict__ h_out, uint64_t n_h) {
+    const float scale = *grad_loss / *n_valid;
+    if (blockIdx.x >= w_blocks) {
+        const uint64_t i = (uint64_t(blockIdx.x - w_blocks) * kWgThreads + threadIdx.x) * kGroup;
+        if (i < n_h) {   // a multiple of 8 elements
+            const u32x4 v = *reinterpret_cast<const u32x4*>(h + i);
+            u32x4 o;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) o[j] = Fmt::pack(Fmt::lo(v[j]) * scale, Fmt::hi(v[j]) * scale);
+            *reinterpret_cast<u32x4*>(h_out + i) = o;
+        }
+        return;
+    }
+    const uint32_t lane = threadIdx.x & 63, l16 = lane & 15, quad = lane >> 4;
+    const uint32_t col = (blockIdx.x % col_blocks) * uint32_t(kWgColumns) + (threadIdx.x >> 6) * (16 * kV) + l16 * kV;
+    const uint32_t steps = tokens / 32;   // <= kSteps
+    u32x4 b[kSteps][kV];
+#pragma unroll
+    for (int s = 0; s < kSteps; ++s) {
+        u32x2 e[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            // ld and col are multiples of 4: all of a lane's columns lie inside the row or none
+            e[j] = uint32_t(s) < steps && col < ld
+                       ? *reinterpret_cast<const u32x2*>(g + uint64_t(s * 32 + quad * 8 + j) * ld + col)
+                       : u32x2{0, 0};
+#pragma unroll
+        for (int t = 0; t < kV; ++t)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const uint32_t lo = e[2 * j][t / 2] >> (t % 2 * 16), hi = e[2 * j + 1][t / 2] >> (t % 2 * 16);
+                b[s][t][j] = (lo & 0xFFFFu) | hi << 16;
+            }
+    }
+    const uint32_t first = blockIdx.x / col_blocks * per_block;
+    const uint32_t last = first + per_block < hidden ? first + per_block : hidden;
+    for (uint32_t h0 = first; h0 < last; h0 += kWgStep) {
+        f32x4 acc[2][kV];
+        const uint16_t* row[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const uint32_t r = h0 + (l16 >> 2) * 8 + u * 4 + (l16 & 3);
+            row[u] = hidden_t + uint64_t(r < hidden ? r : hidden - 1) * tokens + quad * 8;
+#pragma unroll
+            for (int t = 0; t < kV; ++t) acc[u][t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+#pragma unroll
+        for (int s = 0; s < kSteps; ++s) {
+            if (uint32_t(s) < steps) {
+                const u32x4 a0 = *reinterpret_cast<const u32x4*>(row[0] + s * 32);
+                const u32x4 a1 = *reinterpret_cast<const u32x4*>(row[1] + s * 32);
+#pragma unroll
+                for (int t = 0; t < kV; ++t) {
+                    acc[0][t] = mfma(Fmt{}, a0, b[s][t], acc[0][t]);
+                    acc[1][t] = mfma(Fmt{}, a1, b[s][t], acc[1][t]);
+                }
+            }
+        }
+        const uint32_t hr = h0 + quad * 8;
+        if (hr < hidden) {   // a multiple of 8
+#pragma unroll
+            for (int t = 0; t < kV; ++t)
+                if (col + t < vocab)
+                    *reinterpret_cast<u32x4*>(out + uint64_t(col + t) * hidden + hr) =
+                        pack8<Fmt>(acc[0][t] * scale, acc[1][t] * scale);
+        }
+    }
+}
+
 inline int status() {
     // the runtime keeps a failed launch as the thread's last error: reading it clears it
     return int(hipGetLastError());
@@ -501,6 +615,27 @@ int launch_sum(int nparts, const float* parts, uint32_t count, uint32_t cols, vo
     hipLaunchKernelGGL(kernel, dim3((count / kGroup + kSumThreads - 1) / kSumThreads), dim3(kSumThreads), 0, st, parts,
                        count, cols, static_cast<uint16_t*>(out), static_cast<const uint16_t*>(g), uint64_t(ld),
                        static_cast<const uint16_t*>(w), tail);
+    return status();
+}
+
+template <typename Fmt>
+int launch_weight_grad(const float* grad_loss, const float* n_valid, const void* g, uint64_t ld, uint32_t vocab,
+                       const void* hidden_t, uint32_t tokens, uint32_t hidden, void* out, const void* h, void* h_out,
+                       uint64_t n_h, hipStream_t st) {
+    const uint32_t col_blocks = (vocab + kWgColumns - 1) / kWgColumns;
+    // some 1,024 workgroups, the hidden dimension split where the columns give fewer
+    const uint32_t steps = (hidden + kWgStep - 1) / kWgStep, want = (1024 + col_blocks - 1) / col_blocks;
+    const uint32_t per = (steps + want - 1) / want, splits = (steps + per - 1) / per;
+    const uint64_t h_blocks = (n_h / kGroup + kWgThreads - 1) / kWgThreads;
+    const uint64_t w_blocks = uint64_t(col_blocks) * splits;
+    if (w_blocks + h_blocks > (uint64_t(1) << 31) / kWgThreads) return SF_EINVAL;
+    const auto kernel = tokens <= 64    ? ce_weight_grad_kernel<Fmt, 2>
+                        : tokens <= 128 ? ce_weight_grad_kernel<Fmt, 4>
+                                        : ce_weight_grad_kernel<Fmt, 8>;
+    hipLaunchKernelGGL(kernel, dim3(uint32_t(w_blocks + h_blocks)), dim3(kWgThreads), 0, st, grad_loss, n_valid,
+                       static_cast<const uint16_t*>(g), ld, vocab, static_cast<const uint16_t*>(hidden_t), tokens,
+                       hidden, static_cast<uint16_t*>(out), col_blocks, per * kWgStep, uint32_t(w_blocks),
+                       static_cast<const uint16_t*>(h), static_cast<uint16_t*>(h_out), n_h);
     return status();
 }
 
@@ -639,6 +774,28 @@ int sf_ce_scale(const float* grad_loss, const float* n_valid, const void* grad_h
         return SF_EDTYPE;
     }
     return status();
+}
+
+int sf_ce_weight_grad(const float* grad_loss, const float* n_valid, const void* g, size_t ld, size_t vocab,
+                      const void* hidden_t, size_t tokens, size_t hidden, void* grad_w_out, const void* grad_h,
+                      void* grad_h_out, size_t n_h, int dtype, sf_stream_t stream) {
+    if (grad_loss == nullptr || n_valid == nullptr || g == nullptr || hidden_t == nullptr || grad_w_out == nullptr ||
+        (n_h > 0 && (grad_h == nullptr || grad_h_out == nullptr)))
+        return SF_EINVAL;
+    if (tokens == 0 || tokens % 64 != 0 || tokens > size_t(kWgTokens) || vocab == 0 || vocab > (size_t(1) << 31) ||
+        hidden == 0 || hidden > (size_t(1) << 31) || ld < vocab)
+        return SF_EINVAL;
+    if (ld % kGroup != 0 || hidden % kGroup != 0 || n_h % kGroup != 0 || misaligned(g, 16) || misaligned(hidden_t, 16) ||
+        misaligned(grad_w_out, 16) || misaligned(grad_h, 16) || misaligned(grad_h_out, 16))
+        return SF_EALIGN;
+    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    if (dtype == SF_DTYPE_BF16)
+        return launch_weight_grad<Bf16>(grad_loss, n_valid, g, ld, uint32_t(vocab), hidden_t, uint32_t(tokens),
+                                        uint32_t(hidden), grad_w_out, grad_h, grad_h_out, n_h, st);
+    if (dtype == SF_DTYPE_F16)
+        return launch_weight_grad<F16>(grad_loss, n_valid, g, ld, uint32_t(vocab), hidden_t, uint32_t(tokens),
+                                       uint32_t(hidden), grad_w_out, grad_h, grad_h_out, n_h, st);
+    return SF_EDTYPE;
 }
 
 }  // extern "C"

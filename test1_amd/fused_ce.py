@@ -10,7 +10,8 @@ processed in chunks of ``chunk_rows``; for each chunk the logits are formed,
 one kernel (``csrc/sf_ce.hip``) turns them into the chunk's loss terms and, in
 place, into ``softmax - onehot``, and since the step's backward follows at
 once, the gradients with respect to the hidden rows and the weight are formed
-right away (as the fused kernel does) and only scaled in the backward.  Peak
+right away (as the fused kernel does) and only scaled in the backward; the
+weight's of few tokens is formed there, where its scaling costs nothing.  Peak
 extra memory is one chunk of logits plus an fp32 weight gradient, instead of
 the [N, V] logits in bf16 and fp32 and their gradient.
 
@@ -128,6 +129,20 @@ def _grad_hidden(g: torch.Tensor, ld: int, weight: torch.Tensor, out: torch.Tens
     kernels.ce_grad_hidden(g, weight, parts, out)
 
 
+def _own_weight_grad(n: int, hidden: torch.Tensor) -> bool:
+    """Whether the weight gradient of ``n`` tokens in one chunk is formed in the
+    backward, from the gradient of the logits and the transposed hidden rows,
+    scaled as it is formed (``kernels.ce_weight_grad``): up to 256 tokens, whose
+    factors fit the registers (us a call, as a product into fp32 and a scaling
+    | so, tokens x hidden x vocabulary: 256 x 4096 x 128256 1757 | 1555, 4 x 4096
+    x 128256 1461 | 847; with half the columns a wave 300 x 2560 x 50257 591 |
+    658), and where they are no larger than the fp32 gradient that would be
+    kept instead."""
+    h = hidden.shape[1]
+    return (hidden.element_size() == 2 and n <= 256 and n <= 2 * h and h % 8 == 0 and hidden.stride(1) == 1
+            and hidden.stride(0) >= h)
+
+
 def _forward_kernels(ctx, hidden: torch.Tensor, weight: torch.Tensor, labels: torch.Tensor, ignore_index: int,
                      chunk_rows: int) -> torch.Tensor:
     n, h = hidden.shape
@@ -135,7 +150,6 @@ def _forward_kernels(ctx, hidden: torch.Tensor, weight: torch.Tensor, labels: to
     dev = hidden.device
     labels = labels.contiguous()
     grad_hidden = torch.empty((n, h), dtype=hidden.dtype, device=dev)
-    grad_weight = torch.empty((v, h), dtype=torch.float32, device=dev)
     row_loss = torch.empty(n, dtype=torch.float32, device=dev)
     loss = torch.empty((), dtype=torch.float32, device=dev)
     n_valid = torch.empty((), dtype=torch.float32, device=dev)
@@ -143,11 +157,13 @@ def _forward_kernels(ctx, hidden: torch.Tensor, weight: torch.Tensor, labels: to
     # Rows 128 bytes apart or a multiple of it: the kernel's 128-bit accesses
     # and the products' operand loads stay aligned for any vocabulary.
     ld = -(-v // 64) * 64
-    transposed = _transposed_hidden_pays(step, hidden, v)
+    own = step == n and _own_weight_grad(n, hidden)
+    transposed = own or _transposed_hidden_pays(step, hidden, v)
     # a chunk's rows, as many as the weight gradient's product sums over
     height = (lambda m: -(-m // 64) * 64) if transposed else (lambda m: m)
     buf = torch.empty((height(step), ld), dtype=hidden.dtype, device=dev)
     hidden_t = torch.empty(h * height(step), dtype=hidden.dtype, device=dev) if transposed else None
+    grad_weight = None if own else torch.empty((v, h), dtype=torch.float32, device=dev)
     wt = weight.t()
     f32_out = {} if hidden.dtype == torch.float32 else dict(out_dtype=torch.float32)
     for s in range(0, n, step):
@@ -158,19 +174,25 @@ def _forward_kernels(ctx, hidden: torch.Tensor, weight: torch.Tensor, labels: to
         kernels.ce_rows_(g, labels[s:e], ignore_index, row_loss[s:e])
         # the weight gradient's memory is free until its first product
         _grad_hidden(g, ld, weight, grad_hidden[s:e],
-                     lambda k: (grad_weight.view(-1)[:k] if s == 0 and k <= grad_weight.numel()
+                     lambda k: (grad_weight.view(-1)[:k] if s == 0 and not own and k <= grad_weight.numel()
                                 else torch.empty(k, dtype=torch.float32, device=dev)))
         if transposed:
             pad = height(e - s)
             ht = hidden_t[:h * pad].view(h, pad)
             kernels.ce_hidden(hc, ht, buf[:pad])
             g, hc = buf[:pad, :v], ht.t()
+        if own:
+            break
         if s == 0:
             torch.mm(g.t(), hc, **f32_out, out=grad_weight)
         else:
             torch.addmm(grad_weight, g.t(), hc, **f32_out, out=grad_weight)
     kernels.ce_loss(row_loss, labels, ignore_index, loss, n_valid)
-    ctx.save_for_backward(grad_hidden, grad_weight, n_valid)
+    if own:
+        ctx.vocab = v
+        ctx.save_for_backward(grad_hidden, buf, hidden_t.view(h, -1), n_valid)
+    else:
+        ctx.save_for_backward(grad_hidden, grad_weight, n_valid)
     return loss
 
 
@@ -223,20 +245,30 @@ class ChunkedLinearCrossEntropy(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_loss: torch.Tensor):
-        grad_hidden, grad_weight, n_valid = ctx.saved_tensors
-        # The kernel takes what the forward saved, unless hooks brought it back
+        grad_hidden, *weight_parts, n_valid = ctx.saved_tensors
+        saved = (grad_hidden, *weight_parts, n_valid)
+        # The kernels take what the forward saved, unless hooks brought it back
         # otherwise or the backward itself is differentiated.
-        if (grad_hidden.device.type == "cuda" and grad_weight.device == grad_hidden.device == n_valid.device
-                and grad_hidden.dtype == ctx.weight_dtype and grad_hidden.numel() > 0 and grad_weight.numel() > 0
-                and grad_hidden.is_contiguous() and grad_weight.is_contiguous()
+        if (grad_hidden.device.type == "cuda" and all(t.device == grad_hidden.device for t in saved)
+                and grad_hidden.dtype == ctx.weight_dtype and all(t.numel() > 0 for t in saved)
+                and all(t.is_contiguous() for t in saved)
                 and grad_loss.device == n_valid.device and grad_loss.dtype == torch.float32
                 and not (torch.is_grad_enabled() and grad_loss.requires_grad)
                 and not torch.compiler.is_compiling()
-                and all(type(t) is torch.Tensor for t in (grad_loss, grad_hidden, grad_weight, n_valid))
+                and all(type(t) is torch.Tensor for t in (grad_loss, *saved))
                 and grad_hidden.dtype in _DTYPES
-                and grad_hidden.data_ptr() % 16 == 0 and grad_weight.data_ptr() % 16 == 0):
+                and all(t.data_ptr() % 16 == 0 for t in saved[:-1])):
             with torch.cuda.device(grad_hidden.device):
-                return (*kernels.ce_scale(grad_loss, n_valid, grad_hidden, grad_weight), None, None, None)
+                if len(weight_parts) == 2:
+                    g, hidden_t = weight_parts
+                    return (*kernels.ce_weight_grad(grad_loss, n_valid, grad_hidden, g, ctx.vocab, hidden_t),
+                            None, None, None)
+                return (*kernels.ce_scale(grad_loss, n_valid, grad_hidden, weight_parts[0]), None, None, None)
+        if len(weight_parts) == 2:
+            g, hidden_t = weight_parts
+            grad_weight = g[:, :ctx.vocab].t().float() @ hidden_t.t().float()
+        else:
+            grad_weight = weight_parts[0]
         scale = (grad_loss.to(torch.float32) / n_valid)
         gh = (grad_hidden.to(torch.float32) * scale).to(grad_hidden.dtype)
         gw = (grad_weight * scale).to(ctx.weight_dtype)

@@ -430,6 +430,32 @@ def ce_scale(grad_loss: torch.Tensor, n_valid: torch.Tensor, grad_h: torch.Tenso
     return gh, gw
 
 
+def ce_weight_grad(grad_loss: torch.Tensor, n_valid: torch.Tensor, grad_h: torch.Tensor, g: torch.Tensor, vocab: int,
+                   hidden_t: torch.Tensor, stream: Optional[torch.cuda.Stream] = None) -> Tuple[torch.Tensor, torch.Tensor]:
+    """``grad_h`` and the weight gradient ``g[:, :vocab].T @ hidden_t.T`` times
+    ``grad_loss / n_valid``, both rounded once into their 16-bit type.  ``g``
+    [P, ld] and ``hidden_t`` [H, P] as ``ce_hidden`` leaves them, P <= 256."""
+    tokens, ld = g.shape
+    hidden = hidden_t.shape[0]
+    if (grad_h.dtype not in _CE_DTYPES or grad_h.element_size() != 2 or g.dtype != grad_h.dtype
+            or hidden_t.dtype != grad_h.dtype or grad_loss.dtype != torch.float32 or n_valid.dtype != torch.float32):
+        raise TypeError("ce_weight_grad: need 16-bit tensors of one type and float32 grad_loss and n_valid")
+    if (grad_loss.numel() != 1 or n_valid.numel() != 1 or hidden_t.shape[1] != tokens or not 0 < vocab <= ld):
+        raise ValueError("ce_weight_grad: one-element grad_loss and n_valid, g [P, ld >= vocab] and hidden_t [H, P] "
+                         "expected")
+    for t, what in ((grad_loss, "grad_loss"), (n_valid, "n_valid"), (grad_h, "grad_h"), (g, "g"),
+                    (hidden_t, "hidden_t")):
+        _require_cuda(t, what)
+        _require_contig(t, what)
+    gh = torch.empty_like(grad_h)
+    gw = torch.empty((vocab, hidden), dtype=grad_h.dtype, device=g.device)
+    _native.check(_native.hip().sf_ce_weight_grad(grad_loss.data_ptr(), n_valid.data_ptr(), g.data_ptr(), ld, vocab,
+                                                  hidden_t.data_ptr(), tokens, hidden, gw.data_ptr(),
+                                                  grad_h.data_ptr(), gh.data_ptr(), gh.numel(),
+                                                  _CE_DTYPES[g.dtype], _stream_ptr(stream)), "sf_ce_weight_grad")
+    return gh, gw
+
+
 def memcpy_async(dst: torch.Tensor, src: torch.Tensor, stream: Optional[torch.cuda.Stream] = None,
                  nbytes: Optional[int] = None) -> None:
     """Asynchronous byte copy between contiguous tensors on ``stream``.

@@ -1,5 +1,6 @@
 """What the fused output unit does around its products: the transposed,
-padded hidden rows, and the sum over the vocabulary in parts."""
+padded hidden rows, the sum over the vocabulary in parts, and the weight
+gradient of few tokens."""
 
 import pytest
 import torch
@@ -40,6 +41,8 @@ def both(dev, monkeypatch, dtype, n, h, v, chunk, name, on, off):
     y = torch.randint(0, v, (n,), generator=gen, device=dev)
     y[n - n // 8:] = -100
     out = []
+    if name != "_own_weight_grad":   # it would take the place of what is compared
+        monkeypatch.setattr(fused_ce, "_own_weight_grad", lambda *a: False)
     for answer in (on, off):
         monkeypatch.setattr(fused_ce, name, lambda *a: answer)
         a, b = hid.clone().requires_grad_(True), wgt.clone().requires_grad_(True)
@@ -89,6 +92,59 @@ def test_hidden_gradient_summed_in_parts(dev, monkeypatch, n, h, v, chunk, npart
     got, plain, ref = both(dev, monkeypatch, dtype, n, h, v, chunk, "_vocabulary_parts", nparts, 1)
     assert torch.equal(got[0], plain[0]) and torch.equal(got[2], plain[2])
     assert rel(got[1], ref[1]) <= 1.1 * rel(plain[1], ref[1]) + 1e-6
+
+
+# one and more tiles of 256 columns, 32 hidden rows at a time, 64 to 256 tokens
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 128, 129, 192, 193, 256])
+@pytest.mark.parametrize("h,v", [(8, 1), (72, 257), (264, 130), (1024, 2000)])
+def test_weight_gradient_from_its_factors(dev, n, h, v, dtype):
+    """Products of exact small integers: every sum is exact in fp32, so only the
+    scaling and the last rounding are left, and they are torch's."""
+    gen = torch.Generator(device=dev).manual_seed(n + v)
+    pad, ld = -(-n // 64) * 64, -(-v // 64) * 64
+    hid = torch.randint(-8, 9, (n, h), generator=gen, device=dev).to(dtype)
+    g = torch.full((pad, ld), float("nan"), dtype=dtype, device=dev)
+    g[:n, :v] = torch.randint(-8, 9, (n, v), generator=gen, device=dev).to(dtype)
+    hidden_t = torch.empty(h, pad, dtype=dtype, device=dev)
+    kernels.ce_hidden(hid, hidden_t, g)
+    gh = torch.randn(n, h, generator=gen, device=dev).to(dtype)
+    up, count = torch.tensor(3.0, device=dev), torch.tensor(7.0, device=dev)
+    gh_out, gw = kernels.ce_weight_grad(up, count, gh, g, v, hidden_t)
+    want = (g[:n, :v].double().t() @ hid.double()).float() * (up / count)
+    assert torch.equal(gw, want.to(dtype))
+    assert torch.equal(gh_out, (gh.float() * (up / count)).to(dtype))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n,h,v", [(1, 64, 1003), (100, 72, 5001), (250, 256, 32_000)])
+def test_loss_with_the_weight_gradient_in_the_backward(dev, monkeypatch, n, h, v, dtype):
+    """No further from float64 than through an fp32 gradient, once and again."""
+    got, plain, ref = both(dev, monkeypatch, dtype, n, h, v, 0, "_own_weight_grad", True, False)
+    assert torch.equal(got[0], plain[0]) and torch.equal(got[1], plain[1])
+    assert rel(got[2], ref[2]) <= 1.1 * rel(plain[2], ref[2]) + 1e-6
+
+
+def test_weight_gradient_in_the_backward_with_hooks_and_twice(dev):
+    """Saved tensors brought back from the host, a repeated backward, and a
+    backward that is itself differentiated give the same gradients."""
+    gen = torch.Generator(device=dev).manual_seed(9)
+    hid = torch.randn(100, 64, generator=gen, device=dev).bfloat16().requires_grad_(True)
+    wgt = (torch.randn(700, 64, generator=gen, device=dev) * 0.05).bfloat16().requires_grad_(True)
+    y = torch.randint(0, 700, (100,), generator=gen, device=dev)
+    loss = chunked_linear_cross_entropy(hid, wgt, y)
+    first = torch.autograd.grad(loss, (hid, wgt), retain_graph=True)
+    again = torch.autograd.grad(loss, (hid, wgt), retain_graph=True)
+    up = torch.ones((), device=dev, requires_grad=True)
+    double = torch.autograd.grad(loss, (hid, wgt), grad_outputs=up, create_graph=True)
+    with torch.autograd.graph.save_on_cpu():
+        loss = chunked_linear_cross_entropy(hid, wgt, y)
+    hooked = torch.autograd.grad(loss, (hid, wgt))
+    for a, b, c, d in zip(first, again, double, hooked):
+        assert torch.equal(a, b) and torch.equal(a, d)
+        assert rel(c.detach(), a.double()) <= 2.0 ** -7   # one rounding of sums in another order
+    slope = torch.autograd.grad(double[1].float().sum(), up)[0]
+    torch.testing.assert_close(slope, first[1].float().sum(), rtol=0.05, atol=0.05)
 
 
 def test_parts_and_transposed_rows_in_a_captured_graph(dev, monkeypatch):
