@@ -14,7 +14,7 @@
 // as torch operations took 7.2 ms, and adding the chunks' weight gradients
 // into the fp32 sum 8.1 ms more; loss with both gradients 35.1 -> 11.3 ms.  With
 // the hidden rows transposed for the weight gradient's product
-// (ce_hidden_kernel) 10.3, of which 9.4 are the products.  At 510 rows of 4096
+// (ce_hidden_kernel) 10.3, of which 9.7 are the products.  At 510 rows of 4096
 // (hidden 512): 453 -> 230 us, 57 of them on the GPU, the rest host time of the
 // launches.
 //
@@ -370,7 +370,7 @@ __global__ __launch_bounds__(kScaleThreads) void ce_scale32_kernel(
 // 1217, 777 x 1024 x 32000 79.9 | 68.6, 127 x 4096 x 128256 708 | 474.  (The
 // gradient of the logits transposed too: 3355, which its 0.4 ms does not pay.)
 //
-// Bound by HBM: 4 bytes per element, 67 MB at the first of these sizes.  A
+// Bound by HBM: 4 bytes per element, 67 MB and 17 us at the first of these sizes.  A
 // workgroup takes a tile of 64 x 64 through LDS, 128-bit accesses on both
 // sides.  Rows of 66 elements in LDS put the 8 lanes that read 8 rows each, and
 // the 8 columns beside each other in a wave, into banks of their own.  The
