@@ -3,7 +3,10 @@ plain PyTorch cross entropy on the same bf16 GEMM outputs, in fp32."""
 
 import pytest
 import torch
+from torch.fx.experimental.proxy_tensor import make_fx
+from torch.utils.checkpoint import checkpoint
 
+from test1_amd import fused_ce
 from test1_amd.fused_ce import chunked_linear_cross_entropy
 
 
@@ -53,3 +56,23 @@ def test_shape_errors():
         chunked_linear_cross_entropy(torch.zeros(4, 8), torch.zeros(10, 9), torch.zeros(4, dtype=torch.long))
     with pytest.raises(ValueError):
         chunked_linear_cross_entropy(torch.zeros(4, 8), torch.zeros(10, 8), torch.zeros(5, dtype=torch.long))
+
+
+def test_a_recorded_call_is_seen_as_one():
+    """The kernels are called through pointers, which no record of operations
+    holds: every kind of tracing has to be noticed, with plain tensors too."""
+    seen = []
+
+    def f(x):
+        seen.append(fused_ce._traced())
+        return x * 2
+
+    x = torch.randn(3)
+    f(x)
+    checkpoint(f, x.clone().requires_grad_(True), use_reentrant=False).sum().backward()
+    assert not any(seen)
+    for trace in (lambda: make_fx(f)(x), lambda: make_fx(f, pre_dispatch=True)(x),
+                  lambda: make_fx(f, tracing_mode="fake")(x), lambda: torch.jit.trace(f, x, check_trace=False)):
+        seen.clear()
+        trace()
+        assert seen and all(seen)

@@ -2,6 +2,7 @@
 
 import pytest
 import torch
+from torch.fx.experimental.proxy_tensor import make_fx
 
 from test1_amd import fused_ce, kernels
 from test1_amd.fused_ce import chunked_linear_cross_entropy
@@ -143,6 +144,27 @@ def test_strided_inputs_side_stream_and_repeated_backward(dev):
     assert rel(loss, ref[0]) < 1e-3
     for x1, x2, r in zip(g1, g2, ref[1:]):
         assert torch.equal(x1, x2) and rel(x1, r) < 1e-2
+
+
+@pytest.mark.parametrize("n,chunk", [(40, 0), (300, 128)])   # weight gradient in the backward, in the forward
+@pytest.mark.parametrize("pre_dispatch", [False, True])
+def test_a_traced_graph_computes_on_its_own_inputs(dev, n, chunk, pre_dispatch):
+    """Forward and backward recorded by ``make_fx`` on real tensors and run on
+    other inputs: what these give eagerly, to the type's rounding."""
+    def inputs(seed):
+        gen = torch.Generator(device=dev).manual_seed(seed)
+        return (torch.randn(n, 64, generator=gen, device=dev).bfloat16().requires_grad_(True),
+                (torch.randn(500, 64, generator=gen, device=dev) * 0.05).bfloat16().requires_grad_(True),
+                torch.randint(0, 500, (n,), generator=gen, device=dev))
+
+    def step(h, w, y):
+        loss = chunked_linear_cross_entropy(h, w, y, chunk_rows=chunk)
+        return (loss, *torch.autograd.grad(loss, (h, w)))
+
+    graph = make_fx(step, pre_dispatch=pre_dispatch)(*inputs(1))
+    h, w, y = inputs(2)
+    for got, want in zip(graph(h.detach(), w.detach(), y), exact(h, w, y, 1.0)):
+        assert rel(got, want) < 1e-2
 
 
 def test_all_rows_ignored_is_nan(dev):
