@@ -46,6 +46,19 @@ def _traced() -> bool:
             or torch._ops._len_torch_dispatch_stack_pre_dispatch() > 0)
 
 
+_PLAIN_KEYS = 0
+for _key in ("CPU", "CUDA", "ADInplaceOrView", "AutogradCPU", "AutogradCUDA", "AutocastCPU", "AutocastCUDA"):
+    _PLAIN_KEYS |= torch._C.DispatchKeySet(getattr(torch._C.DispatchKey, _key)).raw_repr()
+
+
+def _memory_is_value(t: torch.Tensor) -> bool:
+    """Whether a kernel that reads ``t``'s memory gets all of it: no batch of a
+    vmap, no wrapper of a function transform, no pending negation (such tensors
+    are of the plain type and differ in their dispatch keys), and no
+    forward-mode derivative beside it."""
+    return torch._C._dispatch_keys(t).raw_repr() & ~_PLAIN_KEYS == 0 and torch.autograd.forward_ad._current_level < 0
+
+
 def _kernels_take(hidden: torch.Tensor, weight: torch.Tensor, labels: torch.Tensor) -> bool:
     """Inputs the HIP kernels run on: one GPU, one float type, int64 labels, at
     least one row.  Left to torch: what its operations refuse by themselves
@@ -258,12 +271,13 @@ class ChunkedLinearCrossEntropy(torch.autograd.Function):
         grad_hidden, *weight_parts, n_valid = ctx.saved_tensors
         saved = (grad_hidden, *weight_parts, n_valid)
         # The kernels take what the forward saved, unless hooks brought it back
-        # otherwise or the backward itself is differentiated or traced.
+        # otherwise or the backward itself is differentiated, batched or traced.
         if (grad_hidden.device.type == "cuda" and all(t.device == grad_hidden.device for t in saved)
                 and grad_hidden.dtype == ctx.weight_dtype and all(t.numel() > 0 for t in saved)
                 and all(t.is_contiguous() for t in saved)
                 and grad_loss.device == n_valid.device and grad_loss.dtype == torch.float32
                 and not (torch.is_grad_enabled() and grad_loss.requires_grad)
+                and _memory_is_value(grad_loss)
                 and not _traced()
                 and all(type(t) is torch.Tensor for t in (grad_loss, *saved))
                 and grad_hidden.dtype in _DTYPES

@@ -76,3 +76,27 @@ def test_a_recorded_call_is_seen_as_one():
         seen.clear()
         trace()
         assert seen and all(seen)
+
+
+def test_gradients_that_are_more_than_their_memory():
+    """Wrapped, batched, negated and dual tensors are of the plain type; the
+    kernels, which read memory, must not take them."""
+    x = torch.tensor(1.0)
+    assert fused_ce._memory_is_value(x) and fused_ce._memory_is_value(torch.nn.Parameter(x))
+    with torch.inference_mode():
+        assert fused_ce._memory_is_value(torch.tensor(1.0))
+    seen = []
+
+    def f(t):
+        seen.append(fused_ce._memory_is_value(t))
+        return t * 2
+
+    torch.func.vmap(f)(torch.ones(3))
+    torch._vmap_internals._vmap(f)(torch.ones(3))          # what is_grads_batched=True runs
+    torch.func.jvp(f, (x,), (x,))
+    torch.func.grad(f)(x)
+    with torch.autograd.forward_ad.dual_level():
+        f(torch.autograd.forward_ad.make_dual(x, x))
+    f(torch.tensor(1 + 2j).conj().imag)
+    f(torch._efficientzerotensor(()))
+    assert len(seen) == 7 and not any(seen)

@@ -167,6 +167,36 @@ def test_a_traced_graph_computes_on_its_own_inputs(dev, n, chunk, pre_dispatch):
         assert rel(got, want) < 1e-2
 
 
+@pytest.mark.parametrize("n,chunk", [(40, 0), (300, 128)])   # weight gradient in the backward, in the forward
+def test_backward_of_a_batch_of_gradients_forward_mode_and_a_negated_one(dev, n, chunk):
+    """What the backward is called with can be more than its memory: a batch
+    (``is_grads_batched``, ``torch.func.vmap``), a dual tensor, a negated view."""
+    gen = torch.Generator(device=dev).manual_seed(4)
+    h = torch.randn(n, 64, generator=gen, device=dev).bfloat16().requires_grad_(True)
+    w = (torch.randn(500, 64, generator=gen, device=dev) * 0.05).bfloat16().requires_grad_(True)
+    y = torch.randint(0, 500, (n,), generator=gen, device=dev)
+    loss = chunked_linear_cross_entropy(h, w, y, chunk_rows=chunk)
+
+    def back(up, **kw):
+        return torch.autograd.grad(loss, (h, w), grad_outputs=up, retain_graph=True, **kw)
+
+    one = back(torch.ones((), device=dev))
+    ups = torch.tensor([1.0, 2.0, -4.0], device=dev)
+    for batch in (back(ups, is_grads_batched=True), torch.func.vmap(back)(ups)):
+        for got, want in zip(batch, one):
+            for k, up in enumerate(ups.tolist()):   # powers of two: the same sums, perhaps in another order
+                assert rel(got[k], up * want.double()) <= 2.0 ** -7
+    with torch.autograd.forward_ad.dual_level():
+        dual = back(torch.autograd.forward_ad.make_dual(ups[0], ups[1]))
+        for got, want in zip(dual, one):
+            primal, tangent = torch.autograd.forward_ad.unpack_dual(got)
+            assert rel(primal, want.double()) <= 2.0 ** -7 and rel(tangent, 2.0 * want.double()) <= 2.0 ** -7
+    negated = torch.tensor(0 + 1j, device=dev).conj().imag
+    assert negated.is_neg() and negated.item() == -1.0
+    for got, want in zip(back(negated), one):
+        assert rel(got, -want.double()) <= 2.0 ** -7
+
+
 def test_all_rows_ignored_is_nan(dev):
     w = torch.randn(32, 16, device=dev).bfloat16()
     loss = chunked_linear_cross_entropy(torch.randn(4, 16, device=dev).bfloat16(), w,
