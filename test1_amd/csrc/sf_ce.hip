@@ -8,8 +8,8 @@
 // one-hot update, the mask and the rounding back moved some 25 bytes per
 // logit and launched about 20 kernels per chunk.  ce_rows_kernel reads every
 // logit once and writes its gradient over it: 4 bytes per 16-bit logit.
-// Measured at 4092 rows of 128256 bf16 logits: ce_rows_kernel 0.389 ms (5.4
-// TB/s; a device copy reaches 5.1), ce_scale16_kernel for the 128256 x 4096
+// Measured at 4092 rows of 128256 bf16 logits: ce_rows_kernel 0.442 ms (4.7
+// TB/s, held back by the exponentials; a device copy reaches 5.1), ce_scale16_kernel for the 128256 x 4096
 // weight and 4092 x 4096 hidden gradients 0.521 ms (6.1 TB/s).  The same steps
 // as torch operations took 7.2 ms, and adding the chunks' weight gradients
 // into the fp32 sum 8.1 ms more; loss with both gradients 35.1 -> 11.3 ms.  With
@@ -34,6 +34,7 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 
 constexpr float kLog2e = 1.44269504088896340736f;
+constexpr float kLog2eLo = 1.92596299e-8f;   // log2(e) - kLog2e
 constexpr int kGroup = 8;   // 16-bit elements per 128-bit access
 
 // 16-bit formats: a pair in a 32-bit word <-> two floats.  The conversions
@@ -61,10 +62,26 @@ struct F16 {
     }
 };
 
-// exp(t) for t <= 0 or so, as 2^(t log2 e): v_exp_f32 has no range reduction
-// to pay for.  The product's rounding costs |t| 2^-24 relative, far below the
-// 16-bit rounding of what it feeds and, in the sum, below fp32 addition's.
-__device__ __forceinline__ float exp_fast(float t) { return __builtin_amdgcn_exp2f(t * kLog2e); }
+// exp(t) for t <= 0 as 2^(t log2 e), the product rounded: relative error up to
+// |t| 2^-24 and no subnormal results.  For the terms of a row's sum alone:
+// against the lane's own maximum |t| is small, and the sum's logarithm comes
+// out as close to 64 bits as with expf (mean relative error of the row losses
+// 3.3e-8 | 3.9e-8 at 4092 x 128256, 3.8e-8 | 4.2e-8 at 510 x 4096).
+__device__ __forceinline__ float exp_term(float t) { return __builtin_amdgcn_exp2f(t * kLog2e); }
+
+// exp(t) for finite t <= 0 or so and t = -inf, to an ulp or two, subnormal
+// results included: 2^n times 2^f, f the rest of t log2 e in two parts.  What
+// becomes a probability takes this one: with exp_term 1.1e-4 of the bf16
+// results at 4092 x 128256 were not the nearest to the exact ones, with it
+// 0.6e-4, as with expf.  It needs 6 instructions more than exp_term and expf
+// 11, which shows where the row is short: us with exp_term | this | expf, bf16
+// rows: 4092 x 128256 403 | 442 | 469, 4092 x 32000 80 | 113 | 121, 1023 x
+// 50257 47 | 60 | 63, 510 x 4096 5.9 | 6.2 | 6.9.
+__device__ __forceinline__ float exp_full(float t) {
+    t = fmaxf(t, -200.0f);   // 2^f of an infinite t would be NaN
+    const float n = rintf(t * kLog2e);
+    return __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(fmaf(t, kLog2eLo, fmaf(t, kLog2e, -n))), int(n));
+}
 
 // A partial logsumexp: the maximum so far and the sum of exp(x - base(max)).
 // base() is the maximum itself, or 0 where that is infinite, so that rows
@@ -78,8 +95,8 @@ __device__ __forceinline__ Lse merge(Lse a, Lse b) {
     const float m = fmaxf(a.m, b.m);
     const float c = base(m);
     // an empty part stays empty whatever the bases are; a NaN sum stays NaN
-    const float sa = a.s == 0.0f ? 0.0f : a.s * exp_fast(base(a.m) - c);
-    const float sb = b.s == 0.0f ? 0.0f : b.s * exp_fast(base(b.m) - c);
+    const float sa = a.s == 0.0f ? 0.0f : a.s * expf(base(a.m) - c);
+    const float sb = b.s == 0.0f ? 0.0f : b.s * expf(base(b.m) - c);
     return {m, sa + sb};
 }
 
@@ -105,7 +122,7 @@ __device__ __forceinline__ float block_lse(Lse p, Lse* parts) {
         float s = 0.0f;
 #pragma unroll
         for (int w = 0; w < kT / 64; ++w)
-            s += parts[w].s == 0.0f ? 0.0f : parts[w].s * exp_fast(base(parts[w].m) - c);
+            s += parts[w].s == 0.0f ? 0.0f : parts[w].s * expf(base(parts[w].m) - c);
         p = {m, s};
     }
     return base(p.m) + logf(p.s);
@@ -197,24 +214,36 @@ __global__ __launch_bounds__(kT) void ce_rows_kernel(uint16_t* __restrict__ logi
     for (int k = 0; k < kG; ++k)
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            s0 += exp_fast(Fmt::lo(v[k][j]) - c);
-            s1 += exp_fast(Fmt::hi(v[k][j]) - c);
+            s0 += exp_term(Fmt::lo(v[k][j]) - c);
+            s1 += exp_term(Fmt::hi(v[k][j]) - c);
         }
     keep_packed<kG>(v);
     const float lse = block_lse<kT>({m, s0 + s1}, parts);
     if (threadIdx.x == 0) row_loss[row] = lse - target;
+    if (!__builtin_isfinite(lse)) {
+        // a row with NaN or infinities: what softmax gives, from memory again
+        for (uint32_t g = threadIdx.x; g < groups; g += kT) {
+            const u32x4 r = xv[g];
+            u32x4 o;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) o[j] = Fmt::pack(expf(Fmt::lo(r[j]) - lse), expf(Fmt::hi(r[j]) - lse));
+            xv[g] = o;
+        }
+        if (threadIdx.x == uint32_t(y) / kGroup % kT) x[y] = uint16_t(Fmt::pack(expf(target - lse) - 1.0f, 0.0f));
+        return;
+    }
 #pragma unroll
     for (int k = 0; k < kG; ++k) {
         const uint32_t g = uint32_t(k) * kT + threadIdx.x;
         u32x4 o;
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-            o[j] = Fmt::pack(exp_fast(Fmt::lo(v[k][j]) - lse), exp_fast(Fmt::hi(v[k][j]) - lse));
+            o[j] = Fmt::pack(exp_full(Fmt::lo(v[k][j]) - lse), exp_full(Fmt::hi(v[k][j]) - lse));
         if (k < kFull || g < groups) xv[g] = o;
     }
     // The label's element, over what the same lane has just stored with its group.
     if (threadIdx.x == uint32_t(y) / kGroup % kT)
-        x[y] = uint16_t(Fmt::pack(exp_fast(target - lse) - 1.0f, 0.0f));
+        x[y] = uint16_t(Fmt::pack(exp_full(target - lse) - 1.0f, 0.0f));
 }
 
 // Element access of the streaming kernel below.
@@ -222,14 +251,12 @@ struct Elem32 {
     using S = float;
     __device__ static float load(const S* p) { return *p; }
     __device__ static void store(S* p, float f) { *p = f; }
-    __device__ static float exp(float t) { return expf(t); }   // results kept in fp32
 };
 template <typename Fmt>
 struct Elem16 {
     using S = uint16_t;
     __device__ static float load(const S* p) { return Fmt::lo(*p); }
     __device__ static void store(S* p, float f) { *p = uint16_t(Fmt::pack(f, 0.0f)); }
-    __device__ static float exp(float t) { return exp_fast(t); }
 };
 
 // Rows that do not fit the registers (16-bit rows of more than 155,648
@@ -262,15 +289,15 @@ __global__ __launch_bounds__(kT) void ce_rows_stream_kernel(typename El::S* __re
 #pragma unroll
         for (int k = 0; k < kU; ++k) m = fmaxf(m, f[k]);
         const float c = base(m);
-        float s = p.s == 0.0f ? 0.0f : p.s * El::exp(base(p.m) - c);
+        float s = p.s == 0.0f ? 0.0f : p.s * expf(base(p.m) - c);
 #pragma unroll
-        for (int k = 0; k < kU; ++k) s += El::exp(f[k] - c);
+        for (int k = 0; k < kU; ++k) s += expf(f[k] - c);
         p = {m, s};
     }
     const float lse = block_lse<kT>(p, parts);
     if (threadIdx.x == 0) row_loss[row] = lse - target;
     for (uint32_t i = threadIdx.x; i < vocab; i += kT) {
-        const float q = El::exp(El::load(x + i) - lse);
+        const float q = expf(El::load(x + i) - lse);
         El::store(x + i, int64_t(i) == y ? q - 1.0f : q);
     }
 }

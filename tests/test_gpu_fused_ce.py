@@ -84,6 +84,27 @@ def test_rows_special_values(dev, vocab, dtype):
     torch.testing.assert_close(got.double(), ref_g, rtol=1e-2, atol=1e-5, equal_nan=True)
 
 
+@pytest.mark.parametrize("vocab", [40, 4096, 160_001])
+def test_rows_keep_probabilities_down_to_the_smallest(dev, vocab):
+    """logsumexp is 0 exactly, so a probability is exp of its logit: the nearest
+    bf16 value, or its neighbour where two ulps of fp32 decide it, down to bf16's
+    subnormals (the smallest is 2^-133, exp(-92.2))."""
+    x = torch.full((1, vocab), -200.0, device=dev)
+    x[0, 0] = 0.0
+    x[0, 1:25] = torch.tensor([-30, -40.25, -55.5, -60.75, -70.5, -80, -85, -86, -87, -87.5, -88, -88.5, -89, -89.5, -90,
+                               -90.5, -91, -91.5, -92, -92.5, -93, -94, -110, float("-inf")], device=dev)
+    x = x.bfloat16()
+    want = torch.exp(x[0, 1:25].double())
+    got = strided(1, vocab, torch.bfloat16, dev)
+    got.copy_(x)
+    loss = torch.empty(1, device=dev)
+    kernels.ce_rows_(got, torch.zeros(1, dtype=torch.int64, device=dev), -100, loss)
+    assert loss.item() == 0.0
+    half_ulp = torch.clamp(2.0 ** (torch.floor(torch.log2(want)) - 8), min=2.0 ** -134)
+    err = (got[0, 1:25].double() - want).abs()
+    assert (err <= half_ulp + 2.0 ** -22 * want).all(), (got[0, 1:25], want)
+
+
 def exact(h, w, y, scale):
     h, w = h.detach().double().requires_grad_(True), w.detach().double().requires_grad_(True)
     loss = torch.nn.functional.cross_entropy(h @ w.t(), y)
