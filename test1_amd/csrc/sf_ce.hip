@@ -625,11 +625,22 @@ inline int status() {
 
 inline bool misaligned(const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) != 0; }
 
-template <typename Fmt, int kT, int kG, int kFull>
-void launch_rows(uint16_t* x, uint64_t ld, uint64_t rows, uint32_t vocab, const int64_t* labels, int64_t ignore,
-                 float* row_loss, hipStream_t st) {
-    hipLaunchKernelGGL((ce_rows_kernel<Fmt, kT, kG, kFull>), dim3(uint32_t(rows)), dim3(kT), 0, st, x, ld, vocab, labels,
-                       ignore, row_loss);
+// Lanes of one launch: a dispatch takes fewer than 2^32 along a dimension.
+constexpr uint64_t kMaxLanes = uint64_t(1) << 31;
+
+// A kernel with one workgroup of kT lanes per row, over as many launches as
+// the rows need.
+template <int kT, typename Kernel, typename S>
+int launch_rows(Kernel kernel, S* x, uint64_t ld, uint64_t rows, uint32_t vocab, const int64_t* labels, int64_t ignore,
+                float* row_loss, hipStream_t st) {
+    for (uint64_t r = 0; r < rows; r += kMaxLanes / kT) {
+        const uint64_t n = rows - r < kMaxLanes / kT ? rows - r : kMaxLanes / kT;
+        hipLaunchKernelGGL(kernel, dim3(uint32_t(n)), dim3(kT), 0, st, x + r * ld, ld, vocab, labels + r, ignore,
+                           row_loss + r);
+        const int e = status();
+        if (e != SF_OK) return e;
+    }
+    return SF_OK;
 }
 
 template <typename Fmt>
@@ -670,15 +681,13 @@ int launch_weight_grad(const float* grad_loss, const float* n_valid, const void*
 // groups per lane, so that short rows keep many workgroups per CU and long
 // ones all their loads in flight at once.
 template <typename Fmt>
-void dispatch_rows16(uint16_t* x, uint64_t ld, uint64_t rows, uint32_t vocab, const int64_t* labels, int64_t ignore,
-                     float* row_loss, hipStream_t st) {
+int dispatch_rows16(uint16_t* x, uint64_t ld, uint64_t rows, uint32_t vocab, const int64_t* labels, int64_t ignore,
+                    float* row_loss, hipStream_t st) {
     const uint32_t groups = (vocab + kGroup - 1) / kGroup;
     // (lanes, groups per lane, of them full: what the line above could not hold)
-#define SF_ROWS(T, G, FULL)                                                                 \
-    if (groups <= uint32_t(T) * G) {                                                        \
-        launch_rows<Fmt, T, G, FULL>(x, ld, rows, vocab, labels, ignore, row_loss, st);     \
-        return;                                                                             \
-    }
+#define SF_ROWS(T, G, FULL)         \
+    if (groups <= uint32_t(T) * G) \
+        return launch_rows<T>(ce_rows_kernel<Fmt, T, G, FULL>, x, ld, rows, vocab, labels, ignore, row_loss, st);
     SF_ROWS(64, 2, 0)
     SF_ROWS(256, 2, 0)
     SF_ROWS(256, 4, 2)
@@ -689,8 +698,7 @@ void dispatch_rows16(uint16_t* x, uint64_t ld, uint64_t rows, uint32_t vocab, co
     SF_ROWS(1024, 16, 12)
     SF_ROWS(1024, 19, 16)
 #undef SF_ROWS
-    hipLaunchKernelGGL((ce_rows_stream_kernel<Elem16<Fmt>, 1024>), dim3(uint32_t(rows)), dim3(1024), 0, st, x, ld,
-                       vocab, labels, ignore, row_loss);
+    return launch_rows<1024>(ce_rows_stream_kernel<Elem16<Fmt>, 1024>, x, ld, rows, vocab, labels, ignore, row_loss, st);
 }
 
 }  // namespace
@@ -705,20 +713,16 @@ int sf_ce_rows(void* logits, int dtype, size_t ld, size_t rows, size_t vocab, co
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     if (dtype == SF_DTYPE_F32) {
         if (misaligned(logits, 4)) return SF_EINVAL;
-        hipLaunchKernelGGL((ce_rows_stream_kernel<Elem32, 1024>), dim3(uint32_t(rows)), dim3(1024), 0, st,
-                           static_cast<float*>(logits), uint64_t(ld), uint32_t(vocab), labels, ignore_index,
-                           row_loss);
-        return status();
+        return launch_rows<1024>(ce_rows_stream_kernel<Elem32, 1024>, static_cast<float*>(logits), uint64_t(ld),
+                                 uint64_t(rows), uint32_t(vocab), labels, ignore_index, row_loss, st);
     }
     if (dtype != SF_DTYPE_BF16 && dtype != SF_DTYPE_F16) return SF_EDTYPE;
     // whole 128-bit groups: every row starts on one and its last one is inside the row's ld elements
     if (misaligned(logits, 16) || ld % kGroup != 0) return SF_EALIGN;
     uint16_t* x = static_cast<uint16_t*>(logits);
-    if (dtype == SF_DTYPE_BF16)
-        dispatch_rows16<Bf16>(x, ld, rows, uint32_t(vocab), labels, ignore_index, row_loss, st);
-    else
-        dispatch_rows16<F16>(x, ld, rows, uint32_t(vocab), labels, ignore_index, row_loss, st);
-    return status();
+    return dtype == SF_DTYPE_BF16
+               ? dispatch_rows16<Bf16>(x, ld, rows, uint32_t(vocab), labels, ignore_index, row_loss, st)
+               : dispatch_rows16<F16>(x, ld, rows, uint32_t(vocab), labels, ignore_index, row_loss, st);
 }
 
 int sf_ce_hidden(const void* hidden, size_t ldh, size_t rows, size_t cols, void* hidden_t, size_t ldt, void* tail,

@@ -105,6 +105,24 @@ def test_rows_keep_probabilities_down_to_the_smallest(dev, vocab):
     assert (err <= half_ulp + 2.0 ** -22 * want).all(), (got[0, 1:25], want)
 
 
+def test_more_rows_than_one_launch_takes(dev):
+    """fp32 rows take a workgroup of 1024 lanes each, and a launch fewer than
+    2^32 lanes: 2^22 rows and more are launched in parts."""
+    n, v = (1 << 22) + 5, 4
+    gen = torch.Generator(device=dev).manual_seed(6)
+    x = torch.randn(n, v, generator=gen, device=dev)
+    y = torch.randint(0, v, (n,), generator=gen, device=dev)
+    y[::1000] = -100
+    ref_loss, ref_g, p = rows_reference(x, y)
+    loss = torch.full((n + 1,), 7.0, device=dev)
+    kernels.ce_rows_(x, y, -100, loss[:n])
+    torch.cuda.synchronize()
+    # as in test_rows_match_float64
+    assert ((loss[:n].double() - ref_loss).abs() <= 1e-6 * (4 + ref_loss.abs())).all() and loss[n] == 7.0
+    half_ulp, tiny = EPS[torch.float32]
+    assert ((x.double() - ref_g).abs() <= half_ulp * ref_g.abs() + 6e-6 * p + tiny).all()
+
+
 def exact(h, w, y, scale):
     h, w = h.detach().double().requires_grad_(True), w.detach().double().requires_grad_(True)
     loss = torch.nn.functional.cross_entropy(h @ w.t(), y)
