@@ -349,10 +349,11 @@ template <typename Fmt>
 __global__ __launch_bounds__(kScaleThreads) void ce_scale16_kernel(
     const float* __restrict__ grad_loss, const float* __restrict__ n_valid, const uint16_t* __restrict__ h,
     uint16_t* __restrict__ h_out, uint64_t n_h, const float* __restrict__ w, uint16_t* __restrict__ w_out,
-    uint64_t n_w, uint64_t w_blocks) {
+    uint64_t n_w, uint64_t w_blocks, uint64_t first_block) {
     const float scale = *grad_loss / *n_valid;
-    if (blockIdx.x < w_blocks) {
-        const uint64_t i = (uint64_t(blockIdx.x) * kScaleThreads + threadIdx.x) * kGroup;
+    const uint64_t block = first_block + blockIdx.x;
+    if (block < w_blocks) {
+        const uint64_t i = (block * kScaleThreads + threadIdx.x) * kGroup;
         if (i + kGroup <= n_w) {
             const f32x4* p = reinterpret_cast<const f32x4*>(w + i);
             const f32x4 a = __builtin_nontemporal_load(p), b = __builtin_nontemporal_load(p + 1);
@@ -362,7 +363,7 @@ __global__ __launch_bounds__(kScaleThreads) void ce_scale16_kernel(
         }
         return;
     }
-    const uint64_t i = ((uint64_t(blockIdx.x) - w_blocks) * kScaleThreads + threadIdx.x) * kGroup;
+    const uint64_t i = ((block - w_blocks) * kScaleThreads + threadIdx.x) * kGroup;
     if (i + kGroup <= n_h) {
         const u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(h + i));
         u32x4 o;
@@ -377,13 +378,14 @@ __global__ __launch_bounds__(kScaleThreads) void ce_scale16_kernel(
 __global__ __launch_bounds__(kScaleThreads) void ce_scale32_kernel(
     const float* __restrict__ grad_loss, const float* __restrict__ n_valid, const float* __restrict__ h,
     float* __restrict__ h_out, uint64_t n_h, const float* __restrict__ w, float* __restrict__ w_out, uint64_t n_w,
-    uint64_t w_blocks) {
+    uint64_t w_blocks, uint64_t first_block) {
     const float scale = *grad_loss / *n_valid;
-    const bool is_w = blockIdx.x < w_blocks;
+    const uint64_t block = first_block + blockIdx.x;
+    const bool is_w = block < w_blocks;
     const float* src = is_w ? w : h;
     float* dst = is_w ? w_out : h_out;
     const uint64_t n = is_w ? n_w : n_h;
-    const uint64_t b = is_w ? blockIdx.x : uint64_t(blockIdx.x) - w_blocks;
+    const uint64_t b = is_w ? block : block - w_blocks;
     const uint64_t i = (b * kScaleThreads + threadIdx.x) * kGroup;
     for (uint64_t j = i; j < n && j < i + kGroup; ++j) dst[j] = src[j] * scale;
 }
@@ -643,6 +645,21 @@ int launch_rows(Kernel kernel, S* x, uint64_t ld, uint64_t rows, uint32_t vocab,
     return SF_OK;
 }
 
+// The scaling of both gradients, in as many launches as its blocks need.
+template <typename S, typename Kernel>
+int launch_scale(Kernel kernel, const float* grad_loss, const float* n_valid, const void* h, void* h_out, uint64_t n_h,
+                 const float* w, void* w_out, uint64_t n_w, uint64_t w_blocks, uint64_t blocks, hipStream_t st) {
+    constexpr uint64_t kMax = kMaxLanes / kScaleThreads;
+    for (uint64_t first = 0; first < blocks; first += kMax) {
+        hipLaunchKernelGGL(kernel, dim3(uint32_t(blocks - first < kMax ? blocks - first : kMax)), dim3(kScaleThreads), 0,
+                           st, grad_loss, n_valid, static_cast<const S*>(h), static_cast<S*>(h_out), n_h, w,
+                           static_cast<S*>(w_out), n_w, w_blocks, first);
+        const int e = status();
+        if (e != SF_OK) return e;
+    }
+    return SF_OK;
+}
+
 template <typename Fmt>
 int launch_sum(int nparts, const float* parts, uint32_t count, uint32_t cols, void* out, const void* g, size_t ld,
                const void* w, uint32_t tail, hipStream_t st) {
@@ -786,25 +803,19 @@ int sf_ce_scale(const float* grad_loss, const float* n_valid, const void* grad_h
         return SF_EALIGN;
     constexpr uint64_t kPer = uint64_t(kScaleThreads) * kGroup;
     const uint64_t wb = (n_w + kPer - 1) / kPer, hb = (n_h + kPer - 1) / kPer;
-    if (wb + hb > ((uint64_t(1) << 31) / kScaleThreads)) return SF_EINVAL;
-    const dim3 grid(uint32_t(wb + hb)), block(kScaleThreads);
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    if (dtype == SF_DTYPE_F32) {
-        hipLaunchKernelGGL(ce_scale32_kernel, grid, block, 0, st, grad_loss, n_valid,
-                           static_cast<const float*>(grad_h), static_cast<float*>(grad_h_out), uint64_t(n_h), grad_w,
-                           static_cast<float*>(grad_w_out), uint64_t(n_w), wb);
-    } else if (dtype == SF_DTYPE_BF16) {
-        hipLaunchKernelGGL(ce_scale16_kernel<Bf16>, grid, block, 0, st, grad_loss, n_valid,
-                           static_cast<const uint16_t*>(grad_h), static_cast<uint16_t*>(grad_h_out), uint64_t(n_h),
-                           grad_w, static_cast<uint16_t*>(grad_w_out), uint64_t(n_w), wb);
-    } else if (dtype == SF_DTYPE_F16) {
-        hipLaunchKernelGGL(ce_scale16_kernel<F16>, grid, block, 0, st, grad_loss, n_valid,
-                           static_cast<const uint16_t*>(grad_h), static_cast<uint16_t*>(grad_h_out), uint64_t(n_h),
-                           grad_w, static_cast<uint16_t*>(grad_w_out), uint64_t(n_w), wb);
-    } else {
-        return SF_EDTYPE;
+    switch (dtype) {
+        case SF_DTYPE_F32:
+            return launch_scale<float>(ce_scale32_kernel, grad_loss, n_valid, grad_h, grad_h_out, n_h, grad_w,
+                                       grad_w_out, n_w, wb, wb + hb, st);
+        case SF_DTYPE_BF16:
+            return launch_scale<uint16_t>(ce_scale16_kernel<Bf16>, grad_loss, n_valid, grad_h, grad_h_out, n_h, grad_w,
+                                          grad_w_out, n_w, wb, wb + hb, st);
+        case SF_DTYPE_F16:
+            return launch_scale<uint16_t>(ce_scale16_kernel<F16>, grad_loss, n_valid, grad_h, grad_h_out, n_h, grad_w,
+                                          grad_w_out, n_w, wb, wb + hb, st);
+        default: return SF_EDTYPE;
     }
-    return status();
 }
 
 int sf_ce_weight_grad(const float* grad_loss, const float* n_valid, const void* g, size_t ld, size_t vocab,

@@ -123,6 +123,21 @@ def test_more_rows_than_one_launch_takes(dev):
     assert ((x.double() - ref_g).abs() <= half_ulp * ref_g.abs() + 6e-6 * p + tiny).all()
 
 
+def test_more_gradients_than_one_launch_scales(dev):
+    """A launch scales 2^34 elements; here the hidden gradient alone has more,
+    and a little weight gradient stands before it."""
+    n = (1 << 34) + 3 * 1024 + 5
+    if torch.cuda.mem_get_info(dev)[0] < 5 * n:
+        pytest.skip("needs 80 GiB of free GPU memory")
+    grad_h = torch.ones(n, dtype=torch.bfloat16, device=dev)
+    grad_h[-4000:] = torch.arange(4000, device=dev).bfloat16()
+    grad_w = torch.arange(1000, device=dev, dtype=torch.float32)
+    gh, gw = kernels.ce_scale(torch.tensor(3.0, device=dev), torch.tensor(2.0, device=dev), grad_h, grad_w)
+    assert torch.equal(gw, (grad_w * 1.5).bfloat16())
+    assert torch.equal(gh[-4000:], (grad_h[-4000:].float() * 1.5).bfloat16())
+    assert all(bool((part == 1.5).all()) for part in gh[:-4000].split(1 << 31))
+
+
 def exact(h, w, y, scale):
     h, w = h.detach().double().requires_grad_(True), w.detach().double().requires_grad_(True)
     loss = torch.nn.functional.cross_entropy(h @ w.t(), y)
