@@ -871,8 +871,10 @@ int cast_launch(const float* src, uint16_t* dst, size_t n, hipStream_t st, hipEv
     if (s < d + 2 * n && d < s + 4 * n) return SF_EOVERLAP;
     const uint32_t lead = lead_elems(d);
     const uint64_t blocks = ceil_div(n + lead, uint64_t(kCastThreads) * kCastUnroll * kGroup);
-    if (blocks > kMaxBlocks && ((s | d) & 15) == 0) return SF_EINVAL;  // > 8.6e9 elements: not a real unit
-    if ((s & 3) == 0 && (d & 1) == 0 && blocks <= kMaxBlocks) {
+    // > 8.6e9 elements: not a real unit; the limit counts whole groups, so up to
+    // 7 elements more need one workgroup more
+    if (((s | d) & 15) == 0 && ceil_div(n / kGroup, uint64_t(kCastThreads) * kCastUnroll) > kMaxBlocks) return SF_EINVAL;
+    if ((s & 3) == 0 && (d & 1) == 0 && blocks <= kMaxBlocks + 1) {
         hipExtLaunchKernelGGL(to_f16 ? cast_flat_f16_kernel : cast_flat_kernel, dim3(uint32_t(blocks)),
                               dim3(kCastThreads), 0, st, start, stop, 0, src, dst, lead, uint64_t(n));
     } else {
