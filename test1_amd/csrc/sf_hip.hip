@@ -542,7 +542,14 @@ __global__ __launch_bounds__(kThreads) void gather_rows_kernel(const void* __res
 // repeat_gather_rows_kernel copies it to the others inside HBM.  Both find
 // the first token by a hash table of the window's ids in LDS, which every
 // workgroup makes for itself (some 5 us; no memory beside the operands).
+//
+// Rows of a table in HBM come here with a cap of at most kFewBlocks, for the
+// loads in flight: a workgroup walks over all windows for its share of each, so
+// many workgroups pay that walk for a few rows (us at a cap of 4096, here |
+// gather_rows_kernel: 1 M 16-bit rows of 64 1269 | 27, 200,000 of 1024 269 |
+// 101, 65,536 of 4096 129 | 122).
 constexpr uint32_t kLinkBlocks = 32;
+constexpr uint64_t kFewBlocks = 256;
 constexpr size_t kLinkRow = 2560;
 constexpr uint32_t kWindow = 8192;
 constexpr uint32_t kSlots = 2 * kWindow;   // of the hash table, at most half full
@@ -806,12 +813,13 @@ int launch_gather_rows(const void* src, const int64_t* ids, size_t ntok, size_t 
     s.nrows = nrows;
     s.per_row = mode == kEdges ? (uint64_t(row_len) + 2 * kGroup - 2) / kGroup : ceil_div(row_len, kGroup);
     s.recip = uint32_t(ceil_div(uint64_t(1) << 31, s.per_row));
-    uint64_t cap = max_workgroups > 0 ? uint64_t(max_workgroups) : kMaxBlocks;
+    uint64_t cap = max_workgroups > 0 && uint64_t(max_workgroups) < kMaxBlocks ? uint64_t(max_workgroups) : kMaxBlocks;
     const bool from_host = memory_type(src) == int(hipMemoryTypeHost);
     const bool once = from_host && mode != kElements && cap > kLinkBlocks && ntok >= kLinkBlocks &&
                       nrows < kOnceRows && repeated_bytes(ntok, nrows, row_len * src_elem) >= kOnceBytes &&
                       memory_type(dst) == int(hipMemoryTypeDevice);
-    const bool link = (once || max_workgroups > 0 || (from_host && row_len * src_elem >= kLinkRow)) &&
+    const bool link = (once || (max_workgroups > 0 && (from_host || cap <= kFewBlocks)) ||
+                       (from_host && row_len * src_elem >= kLinkRow)) &&
                       nrows < (uint64_t(1) << 31);
     if (link && from_host && cap > kLinkBlocks) cap = kLinkBlocks;
     switch (mode) {

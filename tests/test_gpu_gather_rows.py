@@ -76,3 +76,16 @@ def test_repeated_rows_cross_the_link_once(dev, f32, row_len, nrows, ntok):
     check(dev, nrows, row_len, ids, f32, True, False)
     ids[:] = nrows - 1   # all the same
     check(dev, nrows, row_len, ids, f32, True, False)
+
+
+@pytest.mark.parametrize("cap", [256, 257, (1 << 31) - 1])
+def test_few_and_many_workgroups_for_a_table_in_hbm(dev, cap):
+    """Up to 256 workgroups walk over windows of tokens, more over tiles; and
+    2^24 of them would be more lanes than a launch takes."""
+    n = (1 << 24) + 1000
+    table = torch.arange(80, dtype=torch.int16, device=dev).view(10, 8)
+    ids = torch.arange(n, device=dev) % 10
+    out = torch.full((n, 8), -1, dtype=torch.int16, device=dev)
+    kernels.gather_rows(table, ids, out, max_workgroups=cap)
+    torch.cuda.synchronize()
+    assert torch.equal(out, table[ids])
