@@ -763,12 +763,15 @@ inline double repeated_bytes(size_t ntok, size_t nrows, size_t row_bytes) {
     return (read - met) * double(row_bytes);
 }
 
-// Reading rows once pays from here on: 2 MiB are 37 us on the link; the hash
-// tables and the second kernel cost 5 (1,024 tokens) to 25 us (8,192).  fp32
+// Reading rows once pays from here on: 2 MiB are 37 us on the link; a window's
+// hash tables and the second kernel cost 5 (1,024 tokens) to 25 us (8,192), so
+// every full window has to save that much.  65,536 tokens of 30,000 16-bit rows
+// of 160, 2.7 MB to save in 8 windows, 393 -> 499 us; 16,384 of 1,000 fp32 rows
+// of 160, 3.8 MB in 2, 88 -> 57.  fp32
 // rows of 4096: 4,096 tokens of 32,000 rows 1168 -> 1125 us, of 2,000 rows
 // 1076 -> 533; 1,024 of 32,000 rows, 0.3 MiB to save, 298 -> 306.  8,192
 // tokens of 256 rows of 1024 160 -> 45 us, of 256 rows of 64, 0.4 MiB, 15 -> 24.
-constexpr double kOnceBytes = 2 << 20;
+constexpr double kOnceBytes = 2 << 20, kOnceWindowBytes = 3 << 19;
 
 template <bool kCast, RowMode kMode>
 int launch_gather(const void* src, const int64_t* ids, uint64_t ntok, const RowShape& s, uint16_t* dst, uint32_t* bad,
@@ -816,7 +819,9 @@ int launch_gather_rows(const void* src, const int64_t* ids, size_t ntok, size_t 
     uint64_t cap = max_workgroups > 0 && uint64_t(max_workgroups) < kMaxBlocks ? uint64_t(max_workgroups) : kMaxBlocks;
     const bool from_host = memory_type(src) == int(hipMemoryTypeHost);
     const bool once = from_host && mode != kElements && cap > kLinkBlocks && ntok >= kLinkBlocks &&
-                      nrows < kOnceRows && repeated_bytes(ntok, nrows, row_len * src_elem) >= kOnceBytes &&
+                      nrows < kOnceRows &&
+                      repeated_bytes(ntok, nrows, row_len * src_elem) >=
+                          fmax(kOnceBytes, kOnceWindowBytes * double(ntok / kWindow)) &&
                       memory_type(dst) == int(hipMemoryTypeDevice);
     const bool link = (once || (max_workgroups > 0 && (from_host || cap <= kFewBlocks)) ||
                        (from_host && row_len * src_elem >= kLinkRow)) &&

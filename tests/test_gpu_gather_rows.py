@@ -65,10 +65,11 @@ def test_no_rows_asked_for_and_no_rows_to_have(dev, ids):
     (True, 515, 4000, 8192),     # a whole window of rows that start anywhere
     (True, 512, 4001, 8193),     # and one token more
     (False, 1024, 2003, 20_000),
-    (True, 2048, 1, 500),        # one row alone
+    (True, 1 << 19, 1, 40),      # one row alone
 ])
 def test_repeated_rows_cross_the_link_once(dev, f32, row_len, nrows, ntok):
-    """Sizes at which the two-kernel path runs (2 MiB of repeated rows)."""
+    """Sizes at which the two-kernel path runs (2 MiB of repeated rows a window,
+    where a table of few rows counts as read 8 times)."""
     ids = torch.randint(0, nrows, (ntok,), generator=torch.Generator().manual_seed(ntok))
     check(dev, nrows, row_len, ids, f32, True, False)
     ids[5::7] = -1
