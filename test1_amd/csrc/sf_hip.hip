@@ -535,7 +535,9 @@ __global__ __launch_bounds__(kThreads) void gather_rows_kernel(const void* __res
 // from LDS, so that no second latency stands before the rows' own.  Host rows
 // shorter than kLinkRow bytes go one per workgroup instead, as fast or faster
 // (us, link | one per workgroup: 3,000 fp32 rows of 320 77.3 | 71.7, of 500
-// 120.8 | 116.3, of 640 140.2 | 139.9, of 1000 221 | 225).
+// 120.8 | 116.3, of 640 140.2 | 139.9, of 1000 221 | 225), unless they are at
+// most kShortRow bytes and there are many (65,536 16-bit rows of 8 21 | 43, of 64
+// 42 | 57, fp32 59 | 76, of 160 81 | 78).
 //
 // kOnce: a row that several tokens ask for crosses the link once.  The first
 // token of each window of kWindow that asks for it gathers it, and
@@ -543,14 +545,17 @@ __global__ __launch_bounds__(kThreads) void gather_rows_kernel(const void* __res
 // the first token by a hash table of the window's ids in LDS, which every
 // workgroup makes for itself (some 5 us; no memory beside the operands).
 //
-// Rows of a table in HBM come here with a cap of at most kFewBlocks, for the
-// loads in flight: a workgroup walks over all windows for its share of each, so
-// many workgroups pay that walk for a few rows (us at a cap of 4096, here |
-// gather_rows_kernel: 1 M 16-bit rows of 64 1269 | 27, 200,000 of 1024 269 |
-// 101, 65,536 of 4096 129 | 122).
+// A cap decides where it leaves few workgroups: below kManyBlocks for a table in
+// host memory, up to kLinkBlocks for rows into host memory (us, here |
+// gather_rows_kernel: 20,000 16-bit rows of 1024 with 16 workgroups 762 | 846,
+// with 64 795 | 757) and up to kFewBlocks inside HBM, for the loads in flight:
+// a workgroup walks over all windows for its share of each, so many workgroups
+// pay that walk for a few rows (at a cap of 4096: 1 M 16-bit rows of 64 1269 |
+// 27, 200,000 of 1024 269 | 101, 65,536 of 4096 129 | 122).
 constexpr uint32_t kLinkBlocks = 32;
-constexpr uint64_t kFewBlocks = 256;
-constexpr size_t kLinkRow = 2560;
+constexpr uint64_t kFewBlocks = 256, kManyBlocks = 4096;
+constexpr size_t kLinkRow = 2560, kShortRow = 256;
+constexpr size_t kManyTokens = 8192;
 constexpr uint32_t kWindow = 8192;
 constexpr uint32_t kSlots = 2 * kWindow;   // of the hash table, at most half full
 constexpr uint32_t kEmpty = ~0u;
@@ -818,14 +823,17 @@ int launch_gather_rows(const void* src, const int64_t* ids, size_t ntok, size_t 
     s.recip = uint32_t(ceil_div(uint64_t(1) << 31, s.per_row));
     uint64_t cap = max_workgroups > 0 && uint64_t(max_workgroups) < kMaxBlocks ? uint64_t(max_workgroups) : kMaxBlocks;
     const bool from_host = memory_type(src) == int(hipMemoryTypeHost);
+    const size_t row_bytes = row_len * src_elem;
     const bool once = from_host && mode != kElements && cap > kLinkBlocks && ntok >= kLinkBlocks &&
                       nrows < kOnceRows &&
-                      repeated_bytes(ntok, nrows, row_len * src_elem) >=
+                      repeated_bytes(ntok, nrows, row_bytes) >=
                           fmax(kOnceBytes, kOnceWindowBytes * double(ntok / kWindow)) &&
                       memory_type(dst) == int(hipMemoryTypeDevice);
-    const bool link = (once || (max_workgroups > 0 && (from_host || cap <= kFewBlocks)) ||
-                       (from_host && row_len * src_elem >= kLinkRow)) &&
-                      nrows < (uint64_t(1) << 31);
+    const bool few = from_host ? cap < kManyBlocks || row_bytes >= kLinkRow ||
+                                     (row_bytes <= kShortRow && ntok >= kManyTokens)
+                               : cap <= kLinkBlocks ||
+                                     (cap <= kFewBlocks && memory_type(dst) == int(hipMemoryTypeDevice));
+    const bool link = (once || few) && nrows < (uint64_t(1) << 31);
     if (link && from_host && cap > kLinkBlocks) cap = kLinkBlocks;
     switch (mode) {
         case kWhole: return launch_gather<kCast, kWhole>(src, ids, ntok, s, dst, bad, cap, from_host, link, once, st);

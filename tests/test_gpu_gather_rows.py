@@ -79,6 +79,18 @@ def test_repeated_rows_cross_the_link_once(dev, f32, row_len, nrows, ntok):
     check(dev, nrows, row_len, ids, f32, True, False)
 
 
+@pytest.mark.parametrize("src_host,dst_host,row_len,ntok,wg", [
+    (True, False, 8, 8192, 0), (True, False, 8, 8191, 0),             # short rows, many or few of them
+    (True, False, 64, 20_000, 4095), (True, False, 64, 20_000, 4096), (True, False, 72, 20_000, 0),
+    (False, True, 72, 3000, 32), (False, True, 72, 3000, 33),         # few or more workgroups into host memory
+])
+def test_both_sides_of_the_lines_between_the_kernels(dev, src_host, dst_host, row_len, ntok, wg):
+    ids = torch.randint(0, 500, (ntok,), generator=torch.Generator().manual_seed(ntok + wg))
+    ids[::17] = 500
+    for f32 in (True, False):
+        check(dev, 500, row_len, ids, f32, src_host, dst_host, wg)
+
+
 @pytest.mark.parametrize("cap", [256, 257, (1 << 31) - 1])
 def test_few_and_many_workgroups_for_a_table_in_hbm(dev, cap):
     """Up to 256 workgroups walk over windows of tokens, more over tiles; and
