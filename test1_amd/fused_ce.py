@@ -12,8 +12,9 @@ place, into ``softmax - onehot``, and since the step's backward follows at
 once, the gradients with respect to the hidden rows and the weight are formed
 right away (as the fused kernel does) and only scaled in the backward; the
 weight's of few tokens is formed there, where its scaling costs nothing.  Peak
-extra memory is one chunk of logits plus an fp32 weight gradient, instead of
-the [N, V] logits in bf16 and fp32 and their gradient.
+extra memory is one chunk of logits with its hidden rows transposed and up to
+128 MiB of partial sums, plus an fp32 weight gradient, instead of the [N, V]
+logits in bf16 and fp32 and their gradient.
 
 Numerics: logsumexp, softmax and the loss are fp32; the logits are the bf16
 GEMM's output widened, as ``nn.CrossEntropyLoss`` on bf16 logits sees them;
@@ -74,17 +75,47 @@ def _kernels_take(hidden: torch.Tensor, weight: torch.Tensor, labels: torch.Tens
             and all(type(t) in (torch.Tensor, torch.nn.Parameter) for t in (hidden, weight, labels)))
 
 
-def auto_chunk_rows(vocab: int, hidden_size: int, element_size: int) -> int:
+_PARTS_VOCAB = 16384   # the shortest vocabulary that ``_vocabulary_parts`` divides
+_PARTS_TILES = 64      # and the most tiles of a product
+
+
+def _tiles(rows: int, hidden_size: int) -> int:
+    return -(-rows // 256) * -(-hidden_size // 256)
+
+
+def auto_chunk_rows(tokens: int, vocab: int, hidden_size: int, element_size: int) -> int:
     """Rows per chunk when the caller names none.  One chunk where possible:
     the products run at 0.80-1.47 PFLOP/s on 523 rows against 4092 (hidden
     4096, vocabulary 128256), and every chunk after the first reads and writes
-    the whole fp32 weight gradient again.  The chunk of logits may take what a
-    16-bit product of the weight gradient's size would (``hidden_size`` rows
-    of it), and at least 384 MiB (fp32: 256 MiB): with that the call's peak is
-    no higher than with chunks of 256 MiB of fp32 logits, their 16-bit copy
-    and that product beside the accumulator."""
-    least = (384 << 20) // (2 * vocab) if element_size == 2 else (256 << 20) // (4 * vocab)
-    return max(1, hidden_size, least)
+    the whole fp32 weight gradient again.  What a chunk may take beside that
+    gradient is what the torch operations take at their peak with chunks of 256
+    MiB of fp32 logits.  16-bit: the next chunk's logits, a temporary of
+    ``logsumexp`` and the 16-bit gradient of the chunk before, 640 MiB, or that
+    gradient and a 16-bit product of the weight gradient's size; here a chunk
+    has its logits, its hidden rows transposed, and partial sums of at most 128
+    MiB (``_vocabulary_parts``), which the first chunk finds in the weight
+    gradient's memory and a short last one behind its logits.  fp32: logits, and
+    a product that is not made here."""
+    if element_size == 4:
+        return max(1, hidden_size, (256 << 20) // (4 * vocab))
+    peak = max(640 << 20, (128 << 20) + 2 * vocab * hidden_size)
+    ld = -(-vocab // 64) * 64
+    rows = peak // (2 * (ld + hidden_size))
+    # the fewest rows of a chunk whose partial sums have to be allocated
+    least = tokens if tokens <= rows else rows - (64 << 20) // ld
+    if (vocab >= _PARTS_VOCAB and _tiles(max(1, least), hidden_size) <= _PARTS_TILES
+            and not (tokens <= rows and 16 * tokens <= vocab)):
+        rows = (peak - (128 << 20)) // (2 * (ld + hidden_size))
+    # equal chunks, whole tiles of 256 rows if that fits, else whole 64s, to
+    # which the transposed rows are padded (8192 x 4096 x 128256 in 4096 + 4096
+    # 20.8 ms, in 4416 + 3776 26.1)
+    if rows < 64:
+        return max(1, rows)
+    rows = rows // 64 * 64
+    if tokens > rows:
+        equal = -(-tokens // -(-tokens // rows))
+        rows = next(r for r in (-(-equal // 256) * 256, -(-equal // 64) * 64) if r <= rows)
+    return rows
 
 
 def _transposed_hidden_pays(rows: int, hidden: torch.Tensor, vocab: int) -> bool:
@@ -96,9 +127,12 @@ def _transposed_hidden_pays(rows: int, hidden: torch.Tensor, vocab: int) -> bool
     tokens x hidden x vocabulary, as they are | transposed and padded: 777 x
     1024 x 32000 80 | 69, 127 x 4096 x 128256 708 | 474, 4092 x 4096 x 128256
     4198 | 3490; below, 510 x 512 x 4096 21.8 | 22.2.  Only rows that lie one
-    behind the other: what is laid out along the sum already needs nothing."""
-    return (hidden.element_size() == 2 and hidden.stride(1) == 1 and hidden.stride(0) >= hidden.shape[1]
-            and 2 * rows * hidden.shape[1] * vocab >= 1 << 35)
+    behind the other: what is laid out along the sum already needs nothing.
+    And only where the transposed rows take no more than the torch operations'
+    fp32 logits with their temporary, or 16-bit product, beside the logits."""
+    h = hidden.shape[1]
+    return (hidden.element_size() == 2 and hidden.stride(1) == 1 and hidden.stride(0) >= h
+            and 2 * rows * h * vocab >= 1 << 35 and rows * h <= max(3 * rows * vocab, vocab * h))
 
 
 def _vocabulary_parts(rows: int, weight: torch.Tensor) -> int:
@@ -121,8 +155,8 @@ def _vocabulary_parts(rows: int, weight: torch.Tensor) -> int:
     380 | 286; 4092 x 1024 x 50257 in chunks of 256 6073 | 3654).  Operands that
     start on 16-byte boundaries only."""
     v, h = weight.shape
-    tiles = -(-rows // 256) * -(-h // 256)
-    if (weight.element_size() != 2 or tiles > 64 or v < 16384 or h % 8 != 0 or not weight.is_contiguous()
+    tiles = _tiles(rows, h)
+    if (weight.element_size() != 2 or tiles > _PARTS_TILES or v < _PARTS_VOCAB or h % 8 != 0 or not weight.is_contiguous()
             or weight.data_ptr() % 16 != 0):
         return 1
     # the weight read twice, its gradient written in fp32 and rounded; the
@@ -195,10 +229,18 @@ def _forward_kernels(ctx, hidden: torch.Tensor, weight: torch.Tensor, labels: to
         g = buf[:e - s, :v]
         torch.mm(hc, wt, out=g)
         kernels.ce_rows_(g, labels[s:e], ignore_index, row_loss[s:e])
-        # the weight gradient's memory is free until its first product
-        _grad_hidden(g, ld, weight, grad_hidden[s:e],
-                     lambda k: (grad_weight.view(-1)[:k] if s == 0 and not own and k <= grad_weight.numel()
-                                else torch.empty(k, dtype=torch.float32, device=dev)))
+
+        def scratch(k: int) -> torch.Tensor:
+            # the weight gradient's memory is free until its first product, the
+            # logits' behind a chunk shorter than the others
+            if s == 0 and not own and k <= grad_weight.numel():
+                return grad_weight.view(-1)[:k]
+            behind = buf[height(e - s):].view(-1)
+            if 2 * k <= behind.numel():
+                return behind[:2 * k].view(torch.float32)
+            return torch.empty(k, dtype=torch.float32, device=dev)
+
+        _grad_hidden(g, ld, weight, grad_hidden[s:e], scratch)
         if transposed:
             pad = height(e - s)
             ht = hidden_t[:h * pad].view(h, pad)
@@ -306,7 +348,7 @@ def chunked_linear_cross_entropy(hidden: torch.Tensor, weight: torch.Tensor, lab
     ~256 MiB of fp32 logits)."""
     if chunk_rows <= 0:
         if hidden.dim() == 2 and _kernels_take(hidden, weight, labels):
-            chunk_rows = auto_chunk_rows(weight.shape[0], weight.shape[-1], hidden.element_size())
+            chunk_rows = auto_chunk_rows(hidden.shape[0], weight.shape[0], weight.shape[-1], hidden.element_size())
         else:
             chunk_rows = max(1, (256 << 20) // (4 * weight.shape[0]))
     return ChunkedLinearCrossEntropy.apply(hidden, weight, labels, int(ignore_index), int(chunk_rows))

@@ -100,3 +100,25 @@ def test_gradients_that_are_more_than_their_memory():
     f(torch.tensor(1 + 2j).conj().imag)
     f(torch._efficientzerotensor(()))
     assert len(seen) == 7 and not any(seen)
+
+
+@pytest.mark.parametrize("vocab", [1, 30, 1000, 4096, 16_383, 16_384, 32_000, 128_256, 152_064])
+@pytest.mark.parametrize("hidden", [64, 768, 1536, 4096, 8192])
+def test_a_chunk_takes_no_more_than_the_torch_operations_did(vocab, hidden):
+    """Logits, transposed hidden rows and partial sums against the fp32 chunks
+    of 256 MiB: their logits, logsumexp's temporary and a 16-bit chunk, or that
+    and the 16-bit product."""
+    former = max(640 << 20, (128 << 20) + 2 * vocab * hidden)
+    weight = torch.empty(vocab, hidden, dtype=torch.bfloat16, device="meta")
+    ld = -(-vocab // 64) * 64
+    for tokens in (1, 64, 1000, 4092, 4400, *range(5000, 50_000, 999), 1_000_000):
+        step = min(tokens, fused_ce.auto_chunk_rows(tokens, vocab, hidden, 2))
+        buffers = 2 * -(-step // 64) * 64 * (ld + hidden)
+        for first in (0, tokens - tokens % step):
+            rows = min(step, tokens - first)
+            parts = fused_ce._vocabulary_parts(rows, weight)
+            sums = 4 * parts * rows * hidden if 0 < rows and parts > 1 else 0
+            if (first == 0 and parts * rows <= vocab) or sums <= 2 * (step - -(-rows // 64) * 64) * ld:
+                sums = 0
+            assert buffers + sums <= former
+    assert fused_ce.auto_chunk_rows(4092, 128_256, 4096, 2) >= 4092

@@ -86,6 +86,7 @@ def test_parts_are_added_up_with_what_they_leave(dev, nparts, n, h, v, dtype):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("n,h,v,chunk,nparts", [(1, 64, 1003, 0, 16), (127, 72, 5001, 0, 8), (300, 64, 1003, 128, 4),
+                                                (330, 64, 5000, 300, 4),   # the second chunk's behind its logits
                                                 (300, 256, 32_000, 70, 2)])
 def test_hidden_gradient_summed_in_parts(dev, monkeypatch, n, h, v, chunk, nparts, dtype):
     """No further from float64 than one sum: parts of it in fp32, rounded once."""
@@ -179,3 +180,25 @@ def test_parts_and_transposed_rows_in_a_captured_graph(dev, monkeypatch):
         torch.cuda.synchronize()
         for t, w in zip(out, want):
             assert torch.equal(t.detach(), w), rep
+
+
+@pytest.mark.parametrize("n,h,v,chunk", [(100_000, 4096, 1000, 0), (40_000, 4096, 100, 40_000), (3000, 768, 152_064, 0),
+                                         (1800, 768, 152_064, 0)])
+def test_peak_memory_of_the_forward(dev, n, h, v, chunk):
+    """Beside the gradients it keeps, the forward takes no more than the torch
+    operations do: at most 640 MiB or, with chunks named by the caller, as much
+    as their fp32 logits, a temporary and a 16-bit copy; and a 16-bit product."""
+    hid = torch.randn(n, h, device=dev).bfloat16().requires_grad_(True)
+    wgt = (torch.randn(v, h, device=dev) * 0.05).bfloat16().requires_grad_(True)
+    y = torch.randint(0, v, (n,), device=dev)
+    chunked_linear_cross_entropy(hid, wgt, y, chunk_rows=chunk)   # the library's workspaces
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    loss = chunked_linear_cross_entropy(hid, wgt, y, chunk_rows=chunk)
+    torch.cuda.synchronize()
+    took = torch.cuda.max_memory_allocated() - before - 2 * n * h - 4 * v * h
+    named = 10 * min(n, chunk) * v
+    most = max(named if chunk else 640 << 20, (2 * min(n, chunk) * v if chunk else 128 << 20) + 2 * v * h)
+    # and row losses, labels, scalars, and the rows padded to 64 columns
+    assert loss.isfinite() and took <= most + 16 * n + 128 * min(n, chunk) + (1 << 20), (took, most)
