@@ -1052,7 +1052,10 @@ int stage_launch(const float* host, uint16_t* dst, size_t n, hipStream_t st) {
     // pinned host memory, which a kernel can read; the cast writes device memory
     if (pointer_attributes(host, &a) != int(hipMemoryTypeHost) || memory_type(dst) != int(hipMemoryTypeDevice))
         return SF_EINVAL;
-    const sf_seg seg = {reinterpret_cast<uint64_t>(a.devicePointer), reinterpret_cast<uint64_t>(dst), n};
+    // Whether the runtime reports the addresses of the pointer or of its
+    // allocation is not documented: the two belong together either way.
+    const ptrdiff_t inside = reinterpret_cast<const char*>(host) - static_cast<const char*>(a.hostPointer);
+    const sf_seg seg = {reinterpret_cast<uint64_t>(a.devicePointer) + uint64_t(inside), reinterpret_cast<uint64_t>(dst), n};
     return launch_segs<OpCast>(&seg, 1, kStageBlocks, st);
 }
 
