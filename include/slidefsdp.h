@@ -12,7 +12,11 @@
  *     the SF_E* codes below; sf_error_string() turns any of them into text.
  *   - Device entry points are asynchronous on the caller's stream, allocate
  *     nothing and keep no global mutable state, so any host thread may call
- *     them concurrently on different streams.
+ *     them concurrently on different streams.  The one exception is
+ *     sf_stage_f32_bf16_noalloc, whose device scratch buffer is shared by its
+ *     larger calls on a device: the library orders each such call after the
+ *     previous one on that device (an event it records), whatever stream
+ *     each runs on.
  *   - Sizes are element counts unless the name says bytes.
  *
  * Each declaration names the reference interface (file:line in the
@@ -42,7 +46,7 @@ typedef void* sf_event_t;
 #define SF_EOVERLAP 9005    /* source and destination ranges overlap */
 #define SF_ENOREQ 9006      /* unknown or already released I/O ticket */
 #define SF_EALIGN 9007      /* O_DIRECT transfer not aligned to SF_IO_ALIGN */
-#define SF_ETOOBIG 9008     /* larger than SF_STAGE_SCRATCH_ELEMS */
+#define SF_ETOOBIG 9008     /* larger than the library's device scratch */
 #define SF_ETIMEDOUT 9009   /* a bounded wait ended before the work completed */
 #define SF_EDMA_BASE 10000  /* + (hsa_status_t & 0xFFF): a ROCr DMA call failed */
 #define SF_EIO_BASE 20000   /* + errno: a file operation failed */
@@ -108,11 +112,15 @@ int sf_cast_f32_f16_timed(const float* src, uint16_t* dst, size_t n,
                           sf_event_t stop);
 
 /* Stage n fp32 values from pinned host memory into a bf16 device array:
- * dst[i] = rne(host_src[i]) (the rounding of sf_cast_f32_bf16), by one kernel
- * on `stream` that reads the host array over the link.  host_src must be
- * pinned host memory (SF_EINVAL otherwise: a kernel reads no other), dst and
- * workspace device memory.  `workspace`, of at least 8 elements, is not
- * touched; it is required as it was when the values travelled through it.
+ * dst[i] = rne(host_src[i]) (the rounding of sf_cast_f32_bf16).  Up to 4 Mi
+ * values are read over the link by one kernel on `stream`; more travel in
+ * pieces of workspace_elems (rounded down to a multiple of 8) through the
+ * caller's device fp32 `workspace`: each piece is copied into it by DMA and
+ * cast from it into dst, all in order on `stream`, so the workspace may be
+ * reused once the stream has passed the call.  A workspace of fewer than 1 Mi
+ * elements (at least 8 are required) is not used: the kernel reads any number.
+ * host_src must be pinned host memory (SF_EINVAL otherwise: kernels and
+ * asynchronous copies read no other), dst and workspace device memory.
  * Replaces the reference's staging of one unit, layer_state.py:299-314 (host
  * cast of the flat master into the pinned convert buffer, then a
  * non_blocking bf16 copy on the H2D stream), with the cast moved to the
@@ -121,16 +129,25 @@ int sf_stage_f32_bf16(const float* host_src, uint16_t* dst, size_t n,
                       float* workspace, size_t workspace_elems,
                       sf_stream_t stream);
 
-/* The largest chunk_elems that sf_stage_f32_bf16_noalloc takes. */
+/* Elements (fp32) of the device scratch buffer of
+ * sf_stage_f32_bf16_noalloc: 64 MiB on every device the library runs on,
+ * held until the process ends. */
 #define SF_STAGE_SCRATCH_ELEMS ((size_t)16 << 20)
 
-/* sf_stage_f32_bf16 without a workspace argument; it allocates nothing and
- * shares nothing between calls.  chunk_elems, 0 or 8 to
- * SF_STAGE_SCRATCH_ELEMS (more is refused with SF_ETOOBIG before anything is
- * enqueued), has no effect: the values are not staged in pieces.  `stream`
- * must belong to the current device.  No counterpart in the reference; for
- * callers that cannot allocate device memory (tight serving loops, harnesses
- * that forbid allocation). */
+/* sf_stage_f32_bf16 that allocates nothing: what goes in pieces (chunk_elems
+ * fp32 elements; 0 selects SF_STAGE_SCRATCH_ELEMS, more is refused with
+ * SF_ETOOBIG before anything is enqueued) goes through a device buffer of the
+ * library's own, one static array per device, whose address is looked up
+ * (and one ordering event created) on the first such call on each device.
+ * `stream` must belong to the current device.  No hipMalloc, hipFree or
+ * other allocating call is made after that.  The calls in pieces on a device
+ * use that device's one buffer, so the library orders them: each one's stream
+ * first waits for the last cast of the previous one on that device (an event
+ * recorded after it), then the call records the event after its own last
+ * cast.  On different streams they are therefore serialised on the device, in
+ * the order their host calls enter the library.  No counterpart in the
+ * reference; for callers that cannot allocate device memory (tight serving
+ * loops, harnesses that forbid allocation). */
 int sf_stage_f32_bf16_noalloc(const float* host_src, uint16_t* dst, size_t n,
                               size_t chunk_elems, sf_stream_t stream);
 

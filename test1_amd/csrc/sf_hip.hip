@@ -1036,27 +1036,56 @@ int sf_fill_b16(uint16_t* dst, size_t n, uint16_t value, sf_stream_t stream) {
 }  // extern "C"
 
 // ---------------------------------------------------------------------
-// Staging: pinned fp32 host array -> bf16 device array, by the segment cast
-// reading the host array over the link: one kernel, which the link bounds.
-// With kStageBlocks workgroups of kHostUnroll groups per lane it reads as
-// fast as a DMA copy, starts sooner and leaves no cast to follow: 147,712
-// elements 30.1 -> 14.3 us, 600,000 61 -> 48, 8 M 587 -> 572, 32 M 2287 ->
-// 2251.  One workgroup per tile reads 2 M elements in 181 us, 64 of 4 groups
-// per lane in 146, 16 to 96 of 8 in 146 to 153.
+// Staging: pinned fp32 host array -> bf16 device array.
+//
+// Up to kStageDirect elements the segment cast reads the host array over the
+// link: one kernel, which the link bounds.  With kStageBlocks workgroups of
+// kHostUnroll groups per lane it reads as fast as a DMA copy, starts sooner and
+// leaves no cast to follow: 147,712 elements 30.1 -> 14.3 us, 600,000 61 -> 48,
+// 8 M 587 -> 572.  One workgroup per tile reads 2 M elements in 181 us, 64 of 4
+// groups per lane in 146, 16 to 96 of 8 in 146 to 153.
+//
+// Larger arrays go piece by piece through a device fp32 buffer, all on one
+// stream: each piece is copied into the buffer by DMA and cast from it by the
+// flat cast; the next piece's copy into the same buffer follows that cast in
+// stream order.  There the kernel's head start is 2 % and less, and it holds
+// its compute units for the whole transfer, which a caller wants beside other
+// work: 12 x 32 M elements beside 40 products of 8192^3 ended after 40.4 ms
+// (products 36.0 of 34.7 alone) by DMA and after 45.2 by the kernel (45.2, the
+// staging 31).  Pieces under kStagePiece elements, whose copies no longer reach
+// the link's rate, leave the kernel the faster way at any size.
 // ---------------------------------------------------------------------
 namespace {
 
-int stage_launch(const float* host, uint16_t* dst, size_t n, hipStream_t st) {
+constexpr size_t kStageDirect = size_t(4) << 20;
+constexpr size_t kStagePiece = size_t(1) << 20;
+
+// Whether n elements are read by one kernel, with pieces of `chunk` otherwise.
+inline bool stage_direct(size_t n, size_t chunk) { return n <= kStageDirect || chunk < kStagePiece; }
+
+int stage_launch(const float* host, uint16_t* dst, size_t n, float* buf, size_t chunk, hipStream_t st) {
     if (n == 0) return SF_OK;
     hipPointerAttribute_t a;
-    // pinned host memory, which a kernel can read; the cast writes device memory
+    // pinned host memory, which a kernel and an asynchronous copy can read; the cast writes device memory
     if (pointer_attributes(host, &a) != int(hipMemoryTypeHost) || memory_type(dst) != int(hipMemoryTypeDevice))
         return SF_EINVAL;
-    // Whether the runtime reports the addresses of the pointer or of its
-    // allocation is not documented: the two belong together either way.
-    const ptrdiff_t inside = reinterpret_cast<const char*>(host) - static_cast<const char*>(a.hostPointer);
-    const sf_seg seg = {reinterpret_cast<uint64_t>(a.devicePointer) + uint64_t(inside), reinterpret_cast<uint64_t>(dst), n};
-    return launch_segs<OpCast>(&seg, 1, kStageBlocks, st);
+    if (stage_direct(n, chunk)) {
+        // Whether the runtime reports the addresses of the pointer or of its
+        // allocation is not documented: the two belong together either way.
+        const ptrdiff_t inside = reinterpret_cast<const char*>(host) - static_cast<const char*>(a.hostPointer);
+        const sf_seg seg = {reinterpret_cast<uint64_t>(a.devicePointer) + uint64_t(inside),
+                            reinterpret_cast<uint64_t>(dst), n};
+        return launch_segs<OpCast>(&seg, 1, kStageBlocks, st);
+    }
+    chunk -= chunk % kGroup;  // every piece starts 16-byte aligned in dst if dst does
+    for (size_t off = 0; off < n; off += chunk) {
+        const size_t c = n - off < chunk ? n - off : chunk;
+        const hipError_t e = hipMemcpyAsync(buf, host + off, c * sizeof(float), hipMemcpyHostToDevice, st);
+        if (e != hipSuccess) return hip_status(e);
+        const int rc = cast_launch(buf, dst + off, c, st, nullptr, nullptr);
+        if (rc != SF_OK) return rc;
+    }
+    return SF_OK;
 }
 
 }  // namespace
@@ -1069,8 +1098,75 @@ int sf_stage_f32_bf16(const float* host_src, uint16_t* dst, size_t n, float* wor
     if (host_src == nullptr || dst == nullptr || workspace == nullptr || workspace_elems < size_t(kGroup) ||
         memory_type(workspace) != int(hipMemoryTypeDevice))
         return SF_EINVAL;
-    return stage_launch(host_src, dst, n, reinterpret_cast<hipStream_t>(stream));
+    return stage_launch(host_src, dst, n, workspace, workspace_elems, reinterpret_cast<hipStream_t>(stream));
 }
+
+}  // extern "C"
+
+// ---------------------------------------------------------------------
+// Staging without allocating: the pieces go through the library's own
+// device buffer instead of a caller workspace.  `scratch` is a static
+// device array, so every device the library's code object is loaded on
+// holds one for the life of the process.  In host code its name is not a
+// device address: the address comes from hipGetSymbolAddress, looked up
+// once per device with that device current, and only that address is
+// passed to the copies and the cast.
+// ---------------------------------------------------------------------
+namespace {
+
+__device__ __align__(256) float scratch[SF_STAGE_SCRATCH_ELEMS];
+
+constexpr int kMaxDevices = 64;
+// Per device: the address of `scratch`, and an event recorded after the last
+// cast of the previous call (the next call's stream waits on it).  The
+// mutex is held from the wait to the record, so the calls of several host
+// threads are ordered one after the other.
+struct ScratchState {
+    float* ptr = nullptr;
+    hipEvent_t last = nullptr;
+    bool recorded = false;
+};
+std::mutex g_scratch_mu;
+ScratchState g_scratch[kMaxDevices];
+
+// The current device, which must be the device of `st` (the null stream:
+// the current device).
+int device_for_stream(hipStream_t st, int* dev) {
+    int cur = 0;
+    hipError_t e = hipGetDevice(&cur);
+    if (e != hipSuccess) return hip_status(e);
+    if (st != nullptr) {
+        hipDevice_t sd = 0;
+        e = hipStreamGetDevice(st, &sd);
+        if (e != hipSuccess) return hip_status(e);
+        if (int(sd) != cur) return SF_EINVAL;
+    }
+    *dev = cur;
+    return SF_OK;
+}
+
+// The device's scratch state, set up on its first use; g_scratch_mu is held.
+int scratch_state(int dev, ScratchState** out) {
+    if (dev < 0 || dev >= kMaxDevices) return SF_EINVAL;
+    ScratchState& s = g_scratch[dev];
+    if (s.ptr == nullptr) {
+        void* p = nullptr;
+        hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
+        if (e != hipSuccess) return hip_status(e);
+        if (p == nullptr) return SF_EINVAL;
+        if (s.last == nullptr) {
+            e = hipEventCreateWithFlags(&s.last, hipEventDisableTiming);
+            if (e != hipSuccess) return hip_status(e);
+        }
+        s.ptr = static_cast<float*>(p);
+    }
+    *out = &s;
+    return SF_OK;
+}
+
+}  // namespace
+
+extern "C" {
 
 int sf_stage_f32_bf16_noalloc(const float* host_src, uint16_t* dst, size_t n, size_t chunk_elems,
                               sf_stream_t stream) {
@@ -1078,16 +1174,26 @@ int sf_stage_f32_bf16_noalloc(const float* host_src, uint16_t* dst, size_t n, si
     if (n == 0) return SF_OK;
     if (host_src == nullptr || dst == nullptr || (chunk_elems != 0 && chunk_elems < size_t(kGroup))) return SF_EINVAL;
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    // the stream must be the current device's
-    if (st != nullptr) {
-        int cur = 0;
-        hipDevice_t sd = 0;
-        hipError_t e = hipGetDevice(&cur);
-        if (e == hipSuccess) e = hipStreamGetDevice(st, &sd);
+    int dev = 0;
+    int rc = device_for_stream(st, &dev);
+    if (rc != SF_OK) return rc;
+    const size_t chunk = chunk_elems == 0 ? SF_STAGE_SCRATCH_ELEMS : chunk_elems;
+    if (stage_direct(n, chunk)) return stage_launch(host_src, dst, n, nullptr, chunk, st);
+    std::lock_guard<std::mutex> lk(g_scratch_mu);
+    ScratchState* s = nullptr;
+    rc = scratch_state(dev, &s);
+    if (rc != SF_OK) return rc;
+    if (s->recorded) {
+        const hipError_t e = hipStreamWaitEvent(st, s->last, 0);
         if (e != hipSuccess) return hip_status(e);
-        if (int(sd) != cur) return SF_EINVAL;
     }
-    return stage_launch(host_src, dst, n, st);
+    rc = stage_launch(host_src, dst, n, s->ptr, chunk, st);
+    // Recorded also after a failed launch: whatever was enqueued before the
+    // failure still uses the scratch buffer and must precede the next call.
+    const hipError_t e = hipEventRecord(s->last, st);
+    if (e == hipSuccess) s->recorded = true;
+    if (rc != SF_OK) return rc;
+    return hip_status(e);
 }
 
 int sf_memcpy_async(void* dst, const void* src, size_t bytes, int kind, sf_stream_t stream) {

@@ -120,9 +120,11 @@ def _check_stage_args(dst: torch.Tensor, host_src: torch.Tensor) -> None:
 def stage_f32_bf16_(dst: torch.Tensor, host_src: torch.Tensor, workspace: torch.Tensor,
                     stream: Optional[torch.cuda.Stream] = None) -> torch.Tensor:
     """dst[:] = RNE-bf16(host_src) for a pinned fp32 host tensor and a bf16 GPU
-    tensor, by one kernel on ``stream`` that reads the host tensor over the
-    link.  ``workspace`` must be an fp32 GPU tensor of at least 8 elements; it
-    is not touched."""
+    tensor: up to 4 Mi elements by one kernel that reads the host tensor over
+    the link, more piece by piece through the fp32 GPU tensor ``workspace``
+    (pieces of its size rounded down to 8 elements; one of fewer than 1 Mi is
+    not used), all in order on ``stream``; ``workspace`` is free again once the
+    stream has passed the call."""
     _check_stage_args(dst, host_src)
     if workspace.dtype != torch.float32 or workspace.numel() < 8:
         raise ValueError("stage_f32_bf16_: the workspace must be a float32 GPU tensor of at least 8 elements")
@@ -136,8 +138,10 @@ def stage_f32_bf16_(dst: torch.Tensor, host_src: torch.Tensor, workspace: torch.
 
 def stage_f32_bf16_noalloc_(dst: torch.Tensor, host_src: torch.Tensor, chunk_elems: int = 0,
                             stream: Optional[torch.cuda.Stream] = None) -> torch.Tensor:
-    """``stage_f32_bf16_`` without a workspace, allocating nothing.
-    ``chunk_elems`` (at most ``_native.SF_STAGE_SCRATCH_ELEMS``) has no effect."""
+    """``stage_f32_bf16_`` through the library's own device scratch buffer
+    (pieces of ``chunk_elems``, at most ``_native.SF_STAGE_SCRATCH_ELEMS``;
+    0: that size), allocating nothing.  Calls that go in pieces on one device
+    share the buffer and run one after the other."""
     _check_stage_args(dst, host_src)
     _native.check(_native.hip().sf_stage_f32_bf16_noalloc(host_src.data_ptr(), dst.data_ptr(), host_src.numel(),
                                                           int(chunk_elems), _stream_ptr(stream)),
