@@ -16,6 +16,7 @@ import ctypes
 import importlib.util
 import os
 import threading
+import warnings
 
 import torch  # noqa: F401  (loads torch's HIP runtime first; see above)
 
@@ -147,16 +148,12 @@ _segs = None
 _RESTYPES = {"sf_error_string": ctypes.c_char_p, "sf_dma_choose_engines": ctypes.c_uint32}
 
 
-def _require_built(path: str) -> None:
+def _bind(path: str, sigs: dict) -> ctypes.CDLL:
     if not os.path.exists(path):
         raise RuntimeError(
             f"native library not built: {path}. Build it with `python -c \"import "
             f"__graft_entry__ as g; g.build()\"` (or `python -m test1_amd.build`)."
         )
-
-
-def _bind(path: str, sigs: dict) -> ctypes.CDLL:
-    _require_built(path)
     lib = ctypes.CDLL(path)
     for name, args in sigs.items():
         fn = getattr(lib, name)
@@ -184,19 +181,29 @@ def cpu() -> ctypes.CDLL:
 
 
 def segs():
-    """The module that reads segment tables from lists of tensors."""
+    """The module that reads segment tables from lists of tensors, or None
+    where it is missing, does not load or was built against another torch
+    (whose tensors it would misread): Python then makes the same tables."""
     global _segs
     if _segs is None:
         with _lock:
             if _segs is None:
-                import torch  # noqa: F401  (its libraries are what the module links against)
+                _segs = _load_segs() or False
+    return _segs or None
 
-                _require_built(SEGS_LIB)
-                spec = importlib.util.spec_from_file_location("_sf_segs", SEGS_LIB)
-                module = importlib.util.module_from_spec(spec)
-                spec.loader.exec_module(module)
-                _segs = module
-    return _segs
+
+def _load_segs():
+    try:
+        spec = importlib.util.spec_from_file_location("_sf_segs", SEGS_LIB)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        if module.TORCH_VERSION != torch.__version__:
+            raise ImportError(f"built against torch {module.TORCH_VERSION}, this is {torch.__version__}")
+        return module
+    except ImportError as e:
+        warnings.warn(f"{SEGS_LIB}: {e}; segment tables are made in Python, some 0.5 us a tensor slower "
+                      f"(`python -m test1_amd.build` builds it)", RuntimeWarning)
+        return None
 
 
 class NativeError(RuntimeError):

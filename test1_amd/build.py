@@ -75,7 +75,8 @@ def build_segs(verbose: bool = False) -> str:
     tmp = _atomic_out(out)
     base = os.path.dirname(torch.__file__)
     _run([CXX, "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-fvisibility=hidden",
-          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}", "-I", INCLUDE,
+          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
+          f'-DSF_TORCH_VERSION="{torch.__version__}"', "-I", INCLUDE,
           "-I", sysconfig.get_paths()["include"], "-isystem", os.path.join(base, "include"), "-o", tmp,
           os.path.join(CSRC, "sf_segs.cpp"), "-L", os.path.join(base, "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10"],
          verbose)

@@ -120,4 +120,12 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_sf_segs", nullptr, -1, methods, n
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__sf_segs(void) { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__sf_segs(void) {
+    PyObject* m = PyModule_Create(&module);
+    // the layout of the tensors read here is this torch's alone
+    if (m != nullptr && PyModule_AddStringConstant(m, "TORCH_VERSION", SF_TORCH_VERSION) != 0) {
+        Py_DECREF(m);
+        return nullptr;
+    }
+    return m;
+}

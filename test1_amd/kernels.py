@@ -159,7 +159,8 @@ def _seg_array(segs: Sequence[Tuple[int, int, int]]):
 def cast_scatter_f32_bf16(pairs: Sequence[Tuple[torch.Tensor, torch.Tensor]],
                           stream: Optional[torch.cuda.Stream] = None) -> None:
     """For each (src fp32, dst bf16) pair of contiguous GPU tensors: dst = RNE(src)."""
-    fast = _native.segs().pair_table(pairs, True)
+    native = _native.segs()
+    fast = native.pair_table(pairs, True) if native is not None else None
     if fast is not None:
         table, count = fast
         _native.check(_native.hip().sf_cast_scatter_f32_bf16(table, count, _stream_ptr(stream)),
@@ -195,7 +196,8 @@ def _check_b16(t: torch.Tensor, what: str, host_ok: bool = False) -> None:
 def _list_table(tensors: Sequence[torch.Tensor], name: str, as_dst: bool):
     """Segment table of 16-bit GPU tensors (their addresses as destinations
     or sources), the number of its entries and of its elements."""
-    fast = _native.segs().list_table(tensors, as_dst)
+    native = _native.segs()
+    fast = native.list_table(tensors, as_dst) if native is not None else None
     if fast is not None:
         return fast
     total = 0
@@ -238,7 +240,8 @@ def copy_segs_b16(pairs: Sequence[Tuple[torch.Tensor, torch.Tensor]],
     """For each (src, dst) pair of contiguous 16-bit tensors of equal numel,
     dst = src, all in one launch.  Sources are GPU tensors; destinations are
     GPU tensors or pinned host tensors."""
-    fast = _native.segs().pair_table(pairs, False)
+    native = _native.segs()
+    fast = native.pair_table(pairs, False) if native is not None else None
     if fast is not None:
         table, count = fast
         if count:

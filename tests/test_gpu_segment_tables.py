@@ -56,3 +56,23 @@ def test_the_rest_is_left_to_the_python_checks(dev):
     inside = []
     torch.func.vmap(lambda x: inside.append(_native.segs().list_table([x], False)) or x)(ok.view(2, 32))
     assert inside == [None]
+
+
+def test_the_same_results_without_the_module(dev, monkeypatch):
+    sizes = [3, 64, 1000, 1]
+    parts = [torch.randn(n, device=dev).bfloat16() for n in sizes]
+    wide = [p.float() for p in parts]
+
+    def results():
+        packed = torch.empty(sum(sizes), dtype=torch.bfloat16, device=dev)
+        back, copies, cast = ([torch.zeros_like(p) for p in parts] for _ in range(3))
+        kernels.pack_b16(parts, packed)
+        kernels.unpack_b16(packed, back)
+        kernels.copy_segs_b16(list(zip(parts, copies)))
+        kernels.cast_scatter_f32_bf16(list(zip(wide, cast)))
+        return [packed, *back, *copies, *cast]
+
+    want = results()
+    monkeypatch.setattr(_native, "segs", lambda: None)
+    assert all(torch.equal(a, b) for a, b in zip(results(), want))
+    assert torch.equal(want[0], torch.cat(parts))
