@@ -135,7 +135,7 @@ def _transposed_hidden_pays(rows: int, hidden: torch.Tensor, vocab: int) -> bool
             and 2 * rows * h * vocab >= 1 << 35 and rows * h <= max(3 * rows * vocab, vocab * h))
 
 
-def _vocabulary_parts(rows: int, weight: torch.Tensor) -> int:
+def _vocabulary_parts(rows: int, weight: torch.Tensor, own: bool = False) -> int:
     """Parts in which the hidden gradient's product of a chunk of ``rows`` sums
     over the vocabulary (1: the product as it is).  The library sums each of
     its 256 x 256 tiles in one workgroup; with as many parts as give every
@@ -148,21 +148,28 @@ def _vocabulary_parts(rows: int, weight: torch.Tensor) -> int:
     3500 x 1536 x 152064, 84 tiles, 6617 | 7454), as it does with short sums
     (the product alone, 510 x 512 x 4096 19.2 | 17.9).  The parts are at most
     512 tiles of fp32.  Adding them up is a launch more, which makes a call that
-    the host's 240 us bound 20 us slower (300 x 1024 x 17000, 64 x 1024 x
-    30000, 250 x 1024 x 32000); so only where the call moves 800 MB or its
+    the host's 240 us bound 20 to 35 us slower (300 x 1024 x 17000, 64 x 1024 x
+    30000, 250 x 1024 x 32000); so only where the call moves 800 MiB or its
     products take 34 GFLOP each (whole calls: 4000 x 64 x 30522, 1.2 GB, 386 |
-    312; 100 x 2560 x 32000, 1.2 GB, 348 | 274; 777 x 1024 x 32000, 51 GFLOP,
-    380 | 286; 4092 x 1024 x 50257 in chunks of 256 6073 | 3654).  Operands that
-    start on 16-byte boundaries only."""
+    312; 777 x 1024 x 32000, 51 GFLOP, 380 | 286; 4092 x 1024 x 50257 in chunks
+    of 256 6073 | 3654).  ``own``: the weight gradient is formed from its factors
+    in the backward (``_own_weight_grad``) and moves less, which leaves the sum
+    itself as the larger part: one element of it takes the time of 6 kB, and the
+    line is at 700 MB (whole calls on a host that needs 180 us for one, and on
+    one that needs 265; below, 64 x 5120 x 16384 196 | 192, 272 | 300, 250 x 4096
+    x 16384 217 | 196, 260 | 295; above, 100 x 2560 x 32000 258 | 191, 271 | 297,
+    200 x 1024 x 60000 351 | 225, 356 | 294, 100 x 512 x 100000 369 | 273, 371 |
+    292, 200 x 256 x 152064 460 | 217, 463 | 299).  Operands that start on
+    16-byte boundaries only."""
     v, h = weight.shape
     tiles = _tiles(rows, h)
     if (weight.element_size() != 2 or tiles > _PARTS_TILES or v < _PARTS_VOCAB or h % 8 != 0 or not weight.is_contiguous()
             or weight.data_ptr() % 16 != 0):
         return 1
-    # the weight read twice, its gradient written in fp32 and rounded; the
-    # logits written, turned into their gradient in place and read twice
-    moved = (14 * h + 10 * rows) * v
-    if moved < 800 << 20 and 2 * rows * h * v < 1 << 35:
+    # the weight read twice, its gradient written (in fp32 and rounded, or once);
+    # the logits written, turned into their gradient in place and read twice
+    moved = ((6 * h if own else 14 * h) + 10 * rows) * v
+    if moved + 6000 * v < 700_000_000 if own else moved < 800 << 20 and 2 * rows * h * v < 1 << 35:
         return 1
     parts = 2
     while parts < 16 and parts * tiles < 256:
@@ -170,12 +177,13 @@ def _vocabulary_parts(rows: int, weight: torch.Tensor) -> int:
     return parts
 
 
-def _grad_hidden(g: torch.Tensor, ld: int, weight: torch.Tensor, out: torch.Tensor, scratch) -> None:
+def _grad_hidden(g: torch.Tensor, ld: int, weight: torch.Tensor, own: bool, out: torch.Tensor, scratch) -> None:
     """out = g @ weight for the gradient of a chunk's logits, ``ld`` elements
-    from row to row.  ``scratch(elements)``: fp32 memory for the parts."""
+    from row to row.  ``own``: see ``_vocabulary_parts``.  ``scratch(elements)``:
+    fp32 memory for the parts."""
     n, v = g.shape
     h = weight.shape[1]
-    nparts = _vocabulary_parts(n, weight)
+    nparts = _vocabulary_parts(n, weight, own)
     if nparts == 1:
         torch.mm(g, weight, out=out)
         return
@@ -240,7 +248,7 @@ def _forward_kernels(ctx, hidden: torch.Tensor, weight: torch.Tensor, labels: to
                 return behind[:2 * k].view(torch.float32)
             return torch.empty(k, dtype=torch.float32, device=dev)
 
-        _grad_hidden(g, ld, weight, grad_hidden[s:e], scratch)
+        _grad_hidden(g, ld, weight, own, grad_hidden[s:e], scratch)
         if transposed:
             pad = height(e - s)
             ht = hidden_t[:h * pad].view(h, pad)

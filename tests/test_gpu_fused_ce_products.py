@@ -126,6 +126,43 @@ def test_loss_with_the_weight_gradient_in_the_backward(dev, monkeypatch, n, h, v
     assert rel(got[2], ref[2]) <= 1.1 * rel(plain[2], ref[2]) + 1e-6
 
 
+@pytest.mark.parametrize("nparts", [2, 16])
+@pytest.mark.parametrize("n,h,v", [(1, 64, 1003), (100, 72, 5001)])
+def test_few_tokens_with_the_sum_in_parts(dev, monkeypatch, n, h, v, nparts):
+    """The weight gradient from its factors and the hidden gradient in parts,
+    whose memory is then an allocation of its own."""
+    monkeypatch.setattr(fused_ce, "_vocabulary_parts", lambda *a: nparts)
+    got, plain, ref = both(dev, monkeypatch, torch.bfloat16, n, h, v, 0, "_own_weight_grad", True, False)
+    assert torch.equal(got[0], plain[0]) and torch.equal(got[1], plain[1])
+    for a, r in zip(got, ref):
+        assert rel(a, r) <= 1e-2
+
+
+@pytest.mark.parametrize("n,h,v,chunk,own,split", [
+    (100, 512, 100_000, 0, True, True),      # from its factors, and in parts
+    (100, 2560, 32_000, 0, True, True),
+    (100, 512, 30_000, 0, True, False),
+    (777, 1024, 32_000, 0, False, True),     # in the weight gradient's memory
+    (1240, 1024, 32_000, 620, False, True),  # there, and for the second chunk allocated
+    (777, 1025, 32_000, 0, False, False),    # rows that start anywhere
+])
+def test_routes_by_the_rules_own_decision(dev, n, h, v, chunk, own, split):
+    gen = torch.Generator(device=dev).manual_seed(n + v)
+    hid = torch.randn(n, h, generator=gen, device=dev).bfloat16().requires_grad_(True)
+    wgt = (torch.randn(v, h, generator=gen, device=dev) * 0.05).bfloat16().requires_grad_(True)
+    y = torch.randint(0, v, (n,), generator=gen, device=dev)
+    rows = min(n, chunk or n)
+    assert fused_ce._own_weight_grad(n, hid) == own
+    assert (fused_ce._vocabulary_parts(rows, wgt, own) > 1) == split
+    assert own or fused_ce._transposed_hidden_pays(rows, hid, v) == (2 * rows * h * v >= 1 << 35)
+    loss = chunked_linear_cross_entropy(hid, wgt, y, chunk_rows=chunk)
+    got = (loss.detach(), *torch.autograd.grad(loss, (hid, wgt)))
+    a, b = hid.detach().double().requires_grad_(True), wgt.detach().double().requires_grad_(True)
+    ref = torch.nn.functional.cross_entropy(a @ b.t(), y)
+    for x, r in zip(got, (ref.detach(), *torch.autograd.grad(ref, (a, b)))):
+        assert rel(x, r) <= 1e-2   # the type's rounding of the logits' gradient and of the results
+
+
 def test_weight_gradient_in_the_backward_with_hooks_and_twice(dev):
     """Saved tensors brought back from the host, a repeated backward, and a
     backward that is itself differentiated give the same gradients."""
