@@ -245,7 +245,10 @@ __global__ __launch_bounds__(kThreads) void fill_b16_kernel(
 // x 4 142.5 | 4.6 | 10.2.  Small tiles: few elements still fill the chip.  A
 // capped grid instead has few workgroups, each with kHostUnroll groups per
 // lane in flight: one layer into host memory with 16 workgroups of 256 x 8
-// 7802 us, 256 x 4 7926, 256 x 2 8062, 512 x 1 8145.
+// 7802 us, 256 x 4 7926, 256 x 2 8062, 512 x 1 8145.  A capped unpack of host
+// memory takes kReadUnroll, whose requests fill the link already and whose
+// smaller tiles end together (us, 8 | 4 groups with 16 workgroups: 2 M elements
+// 77.9 | 74.6, one layer 7705 | 7583; with 8, 2 M 82.8 | 75.7).
 // ---------------------------------------------------------------------
 struct SegTable {
     uint64_t src[SF_MAX_SEGS];
@@ -310,6 +313,7 @@ __device__ __forceinline__ void move_group(const typename Op::S* src, uint16_t* 
 
 constexpr int kSegUnroll = 1;   // groups per lane and tile: one workgroup per tile
 constexpr int kHostUnroll = 8;  // the same for a capped grid
+constexpr int kReadUnroll = 4;  // and for one that unpacks host memory
 constexpr int kStageBlocks = 48;   // workgroups that read one array over the host link
 
 template <typename Op, int kU>
@@ -692,10 +696,14 @@ inline uint64_t ceil_div(uint64_t a, uint64_t b) { return (a + b - 1) / b; }
 constexpr uint64_t kMaxBlocks = (uint64_t(1) << 31) / kThreads;
 
 template <typename Op>
-int launch_segs(const sf_seg* segs, int nsegs, int max_workgroups, hipStream_t stream) {
+int launch_segs(const sf_seg* segs, int nsegs, int max_workgroups, hipStream_t stream, int host_unroll = kHostUnroll) {
     if (nsegs < 0 || (nsegs > 0 && segs == nullptr)) return SF_EINVAL;
     const bool capped = max_workgroups > 0;
-    const uint64_t tile_elems = uint64_t(kThreads) * kGroup * (capped ? kHostUnroll : kSegUnroll);
+    const int unroll = capped ? host_unroll : kSegUnroll;
+    const auto kernel = unroll == kHostUnroll ? seg_kernel<Op, kHostUnroll>
+                        : unroll == kReadUnroll ? seg_kernel<Op, kReadUnroll>
+                                                : seg_kernel<Op, kSegUnroll>;
+    const uint64_t tile_elems = uint64_t(kThreads) * kGroup * uint64_t(unroll);
     // Tables longer than SF_MAX_SEGS are split into several launches.
     for (int base = 0; base < nsegs; base += SF_MAX_SEGS) {
         const int cnt = (nsegs - base < SF_MAX_SEGS) ? (nsegs - base) : SF_MAX_SEGS;
@@ -721,8 +729,7 @@ int launch_segs(const sf_seg* segs, int nsegs, int max_workgroups, hipStream_t s
         if (size_units > kMaxBlocks) return SF_EINVAL;  // > 68e9 elements: not a real layer
         uint64_t grid = tiles < kMaxBlocks ? tiles : kMaxBlocks;
         if (capped && grid > uint64_t(max_workgroups)) grid = uint64_t(max_workgroups);
-        hipLaunchKernelGGL((capped ? seg_kernel<Op, kHostUnroll> : seg_kernel<Op, kSegUnroll>), dim3(uint32_t(grid)),
-                           dim3(kThreads), 0, stream, t);
+        hipLaunchKernelGGL(kernel, dim3(uint32_t(grid)), dim3(kThreads), 0, stream, t);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return int(e);
     }
@@ -980,6 +987,7 @@ int sf_pack_b16(const sf_seg* segs, int nsegs, uint16_t* dst, int max_workgroups
 int sf_unpack_b16(const uint16_t* src, const sf_seg* segs, int nsegs, int max_workgroups,
                   sf_stream_t stream) {
     if (nsegs < 0 || (nsegs > 0 && (segs == nullptr || src == nullptr))) return SF_EINVAL;
+    const int unroll = max_workgroups > 0 && memory_type(src) == int(hipMemoryTypeHost) ? kReadUnroll : kHostUnroll;
     sf_seg local[SF_MAX_SEGS];
     uint64_t off = 0;
     for (int base = 0; base < nsegs; base += SF_MAX_SEGS) {
@@ -990,7 +998,7 @@ int sf_unpack_b16(const uint16_t* src, const sf_seg* segs, int nsegs, int max_wo
             local[i].n = segs[base + i].n;
             off += segs[base + i].n;
         }
-        int rc = launch_segs<OpCopy16>(local, cnt, max_workgroups, reinterpret_cast<hipStream_t>(stream));
+        int rc = launch_segs<OpCopy16>(local, cnt, max_workgroups, reinterpret_cast<hipStream_t>(stream), unroll);
         if (rc != SF_OK) return rc;
     }
     return SF_OK;

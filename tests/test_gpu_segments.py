@@ -61,3 +61,17 @@ def test_pack_and_unpack_of_neighbours(dev, wg):
     torch.cuda.synchronize()
     assert torch.equal(out, flat)
     assert all(torch.equal(a, b) for a, b in zip(back, parts))
+
+
+@pytest.mark.parametrize("wg", [0, 1, 5])
+def test_unpack_of_host_memory(dev, wg):
+    """Tiles of 8192 elements of a capped grid, of 2048 otherwise."""
+    sizes = [*SIZES, 8191, 8192, 8193, 3 * 8192 + 5]
+    flat = pinned_empty(sum(sizes) + 3, torch.int16)
+    flat.copy_(torch.arange(flat.numel(), dtype=torch.int32).to(torch.int16))
+    for skew in (0, 3):
+        back = [torch.full((n + 2,), -1, dtype=torch.int16, device=dev) for n in sizes]
+        kernels.unpack_b16(flat[skew:], [b[1:-1] for b in back], max_workgroups=wg)
+        torch.cuda.synchronize()
+        for b, want in zip(back, flat[skew:skew + sum(sizes)].split(sizes)):
+            assert torch.equal(b[1:-1].cpu(), want) and int(b[0]) == int(b[-1]) == -1
