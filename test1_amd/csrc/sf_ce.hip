@@ -2,21 +2,21 @@
 // of its gradients, for MI355X (gfx950).
 //
 // The three products around these kernels (logits, hidden and weight
-// gradient) are library GEMMs; what lies between them is bound by HBM, and as
+// gradient) are library GEMMs; what lies between them moves bytes, and as
 // separate elementwise and reduction passes it cost more than the products
 // themselves: widening, logsumexp (three passes), gather, subtract, exp, the
 // one-hot update, the mask and the rounding back moved some 25 bytes per
 // logit and launched about 20 kernels per chunk.  ce_rows_kernel reads every
 // logit once and writes its gradient over it: 4 bytes per 16-bit logit.
-// Measured at 4092 rows of 128256 bf16 logits: ce_rows_kernel 0.442 ms (4.7
-// TB/s, held back by the exponentials; a device copy reaches 5.1), ce_scale16_kernel for the 128256 x 4096
-// weight and 4092 x 4096 hidden gradients 0.521 ms (6.1 TB/s).  The same steps
-// as torch operations took 7.2 ms, and adding the chunks' weight gradients
-// into the fp32 sum 8.1 ms more; loss with both gradients 35.1 -> 11.3 ms.  With
-// the hidden rows transposed for the weight gradient's product
-// (ce_hidden_kernel) 10.3, of which 9.7 are the products.  At 510 rows of 4096
-// (hidden 512): 453 -> 230 us, 57 of them on the GPU, the rest host time of the
-// launches.
+// Measured at 4092 rows of 128256 bf16 logits: ce_rows_kernel 0.44-0.47 ms (4.7
+// to 4.5 TB/s, held back by the exponentials; a device copy reaches 5.1),
+// ce_scale16_kernel for the 128256 x 4096 weight and 4092 x 4096 hidden
+// gradients 0.52 ms (6.0 TB/s).  The same steps as torch operations took 7.2 ms,
+// and adding the chunks' weight gradients into the fp32 sum 8.1 ms more; loss
+// with both gradients 35.1 -> 11.3 ms.  With the hidden rows transposed for the
+// weight gradient's product (ce_hidden_kernel) 10.3, of which 9.6 are the
+// products.  At 510 rows of 4096 (hidden 512): 450 -> 195 to 248 us with the
+// host, 61 of them on the GPU, the rest host time of the launches.
 //
 // The C ABI is declared in include/slidefsdp.h.
 

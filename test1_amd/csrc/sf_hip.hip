@@ -4,10 +4,12 @@
 // written once, so the bound is HBM bandwidth (or the host link, for the
 // copies), never the matrix cores.  The kernels therefore use
 //   - 128-bit global loads and stores, 8 elements per lane per group,
-//   - several independent groups per lane to keep enough bytes in flight,
-//   - 128- or 256-lane workgroups (2 or 4 wave64s) and an exact grid of
-//     many thousands of workgroups so all 256 CUs over the 8 XCDs stay busy,
-//   - no LDS and no MFMA.
+//   - several independent groups per lane, or many workgroups of one group per
+//     lane, to keep enough bytes in flight,
+//   - 128- or 256-lane workgroups (2 or 4 wave64s): over HBM many thousands of
+//     them, so that all 256 CUs over the 8 XCDs stay busy, over the host link a
+//     few dozen, which fill it,
+//   - no MFMA, and LDS only for the ids of the row gathers.
 //
 // The C ABI is declared in include/slidefsdp.h.
 

@@ -1,9 +1,9 @@
 """The staging entry point that allocates nothing (sf_stage_f32_bf16_noalloc,
 its pieces through the library's static device scratch buffer) against the
-one with a caller workspace (sf_stage_f32_bf16), through the C ABI: two
-calls in a row, the second with a smaller input, bit for bit, and both equal
-to the oracle's cast; once the runtime's pools are warm, repeating the two
-calls leaves the free device memory unchanged;
+one with a caller workspace (sf_stage_f32_bf16), through the C ABI: calls in
+a row with ever smaller inputs, bit for bit, and all equal to the oracle's
+cast; once the runtime's pools are warm, repeating them leaves the free device
+memory unchanged;
 a piece larger than the scratch is refused with its own status before
 anything is enqueued."""
 
@@ -26,8 +26,9 @@ def test_noalloc_stage_matches_workspace_stage(dev):
     lib = _native.hip()
     scratch = _native.SF_STAGE_SCRATCH_ELEMS
     # (elements, piece): three pieces of the whole scratch with a ragged last
-    # one, then a smaller input in pieces of an odd size
-    cases = [(2 * scratch + 100_003, 0), (1_000_003, 4099)]
+    # one, a smaller input in pieces of an odd size, and one that a kernel
+    # reads without them
+    cases = [(2 * scratch + 100_003, 0), (5_300_003, 1_050_001), (1_000_003, 4099)]
     g = torch.Generator().manual_seed(11)
     bufs = []
     for n, chunk in cases:
@@ -40,7 +41,7 @@ def test_noalloc_stage_matches_workspace_stage(dev):
         bufs.append((x, a, b, work, chunk))
     st = torch.cuda.current_stream()
 
-    def two_calls():
+    def all_calls():
         for k, (x, a, b, work, chunk) in enumerate(bufs):
             print(f"call {k}: {x.numel()} elements, pieces of {chunk or scratch}", flush=True)
             assert lib.sf_stage_f32_bf16_noalloc(x.data_ptr(), a.data_ptr(), x.numel(), chunk,
@@ -53,11 +54,11 @@ def test_noalloc_stage_matches_workspace_stage(dev):
     # and the event waits between calls (in a fresh process its pools still
     # grew by 2 MiB in the second round); two further identical rounds, with
     # nothing else in between, leave the free device memory unchanged.
-    two_calls()
-    two_calls()
+    all_calls()
+    all_calls()
     free_before = torch.cuda.mem_get_info(dev)[0]
-    two_calls()
-    two_calls()
+    all_calls()
+    all_calls()
     free_after = torch.cuda.mem_get_info(dev)[0]
     # the same stagings through the workspace entry point
     for x, a, b, work, chunk in bufs:
