@@ -204,8 +204,8 @@ def _own_weight_grad(n: int, hidden: torch.Tensor) -> bool:
     658), and where they are no larger than the fp32 gradient that would be
     kept instead."""
     h = hidden.shape[1]
-    return (hidden.element_size() == 2 and n <= 256 and n <= 2 * h and h % 8 == 0 and hidden.stride(1) == 1
-            and hidden.stride(0) >= h)
+    return (hidden.element_size() == 2 and n <= 256 and -(-n // 64) * 64 <= 2 * h and h % 8 == 0
+            and hidden.stride(1) == 1 and hidden.stride(0) >= h)
 
 
 def _forward_kernels(ctx, hidden: torch.Tensor, weight: torch.Tensor, labels: torch.Tensor, ignore_index: int,

@@ -122,3 +122,16 @@ def test_a_chunk_takes_no_more_than_the_torch_operations_did(vocab, hidden):
                 sums = 0
             assert buffers + sums <= former
     assert fused_ce.auto_chunk_rows(4092, 128_256, 4096, 2) >= 4092
+
+
+@pytest.mark.parametrize("hidden", [8, 16, 32, 64, 128, 256])
+def test_factors_kept_for_the_backward_are_no_larger_than_the_gradient(hidden):
+    """They are padded to 64 tokens; beside them stands the fp32 gradient."""
+    vocab = 1 << 20
+    for n in (1, 16, 63, 64, 65, 128, 129, 256, 257):
+        hid = torch.empty(n, hidden, dtype=torch.bfloat16, device="meta")
+        padded = -(-n // 64) * 64
+        if fused_ce._own_weight_grad(n, hid):
+            assert n <= 256 and 2 * padded * vocab <= 4 * vocab * hidden
+        else:
+            assert n > 256 or 2 * padded * vocab > 4 * vocab * hidden
