@@ -83,6 +83,15 @@ def _tiles(rows: int, hidden_size: int) -> int:
     return -(-rows // 256) * -(-hidden_size // 256)
 
 
+def _row_elements(vocab: int, element_size: int) -> int:
+    """Elements from a row of logits to the next: rows 128 bytes apart or a
+    multiple of it keep the kernel's 128-bit accesses and the products' operand
+    loads aligned for any vocabulary.  Vocabularies under 64 are not padded
+    beyond what the kernel needs, 16 bytes (fp32: nothing)."""
+    unit = 64 if vocab >= 64 else 8 if element_size == 2 else 1
+    return -(-vocab // unit) * unit
+
+
 def auto_chunk_rows(tokens: int, vocab: int, hidden_size: int, element_size: int) -> int:
     """Rows per chunk when the caller names none.  One chunk where possible:
     the products run at 0.80-1.47 PFLOP/s on 523 rows against 4092 (hidden
@@ -99,7 +108,7 @@ def auto_chunk_rows(tokens: int, vocab: int, hidden_size: int, element_size: int
     if element_size == 4:
         return max(1, hidden_size, (256 << 20) // (4 * vocab))
     peak = max(640 << 20, (128 << 20) + 2 * vocab * hidden_size)
-    ld = -(-vocab // 64) * 64
+    ld = _row_elements(vocab, 2)
     rows = peak // (2 * (ld + hidden_size))
     # the fewest rows of a chunk whose partial sums have to be allocated
     least = tokens if tokens <= rows else rows - (64 << 20) // ld
@@ -219,9 +228,7 @@ def _forward_kernels(ctx, hidden: torch.Tensor, weight: torch.Tensor, labels: to
     loss = torch.empty((), dtype=torch.float32, device=dev)
     n_valid = torch.empty((), dtype=torch.float32, device=dev)
     step = max(1, min(n, int(chunk_rows)))
-    # Rows 128 bytes apart or a multiple of it: the kernel's 128-bit accesses
-    # and the products' operand loads stay aligned for any vocabulary.
-    ld = -(-v // 64) * 64
+    ld = _row_elements(v, hidden.element_size())
     own = step == n and _own_weight_grad(n, hidden)
     transposed = own or _transposed_hidden_pays(step, hidden, v)
     # a chunk's rows, as many as the weight gradient's product sums over

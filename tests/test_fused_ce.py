@@ -110,7 +110,7 @@ def test_a_chunk_takes_no_more_than_the_torch_operations_did(vocab, hidden):
     and the 16-bit product."""
     former = max(640 << 20, (128 << 20) + 2 * vocab * hidden)
     weight = torch.empty(vocab, hidden, dtype=torch.bfloat16, device="meta")
-    ld = -(-vocab // 64) * 64
+    ld = fused_ce._row_elements(vocab, 2)
     for tokens in (1, 64, 1000, 4092, 4400, *range(5000, 50_000, 999), 1_000_000):
         step = min(tokens, fused_ce.auto_chunk_rows(tokens, vocab, hidden, 2))
         buffers = 2 * -(-step // 64) * 64 * (ld + hidden)

@@ -239,3 +239,29 @@ def test_peak_memory_of_the_forward(dev, n, h, v, chunk):
     most = max(named if chunk else 640 << 20, (2 * min(n, chunk) * v if chunk else 128 << 20) + 2 * v * h)
     # and row losses, labels, scalars, and the rows padded to 64 columns
     assert loss.isfinite() and took <= most + 16 * n + 128 * min(n, chunk) + (1 << 20), (took, most)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("v", [1, 4, 9, 63, 64, 65])
+def test_short_vocabularies(dev, v, dtype):
+    """Rows of logits that are not padded: the loss and its gradients, and the
+    memory (64 elements a row would be 256 MB in bf16 at 2 M tokens, fp32 512)."""
+    n, h = 2_000_003 if v == 4 else 3001, 8
+    gen = torch.Generator(device=dev).manual_seed(v)
+    hid = torch.randn(n, h, generator=gen, device=dev).to(dtype).requires_grad_(True)
+    wgt = (torch.randn(v, h, generator=gen, device=dev) * 0.5).to(dtype).requires_grad_(True)
+    y = torch.randint(0, v, (n,), generator=gen, device=dev)
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    loss = chunked_linear_cross_entropy(hid, wgt, y)
+    torch.cuda.synchronize()
+    took = torch.cuda.max_memory_allocated() - before
+    if v == 4:
+        assert took <= 10 * n * v + n * (h * hid.element_size() + 16) + (64 << 20), took
+    a, b = hid.detach().double().requires_grad_(True), wgt.detach().double().requires_grad_(True)
+    ref = torch.nn.functional.cross_entropy(a @ b.t(), y)
+    tol = 1e-2 if dtype == torch.bfloat16 else 1e-5
+    for x, r in zip((loss.detach(), *torch.autograd.grad(loss, (hid, wgt))),
+                    (ref.detach(), *torch.autograd.grad(ref, (a, b)))):
+        assert (x.double() - r).norm() <= tol * r.norm() + 1e-7
