@@ -8,8 +8,8 @@
 // one-hot update, the mask and the rounding back moved some 25 bytes per
 // logit and launched about 20 kernels per chunk.  ce_rows_kernel reads every
 // logit once and writes its gradient over it: 4 bytes per 16-bit logit.
-// Measured at 4092 rows of 128256 bf16 logits: ce_rows_kernel 0.44-0.47 ms (4.7
-// to 4.5 TB/s, held back by the exponentials; a device copy reaches 5.1),
+// Measured at 4092 rows of 128256 bf16 logits: ce_rows_kernel 0.43 ms (4.9
+// TB/s; a device copy reaches 5.1),
 // ce_scale16_kernel for the 128256 x 4096 weight and 4092 x 4096 hidden
 // gradients 0.52 ms (6.0 TB/s).  The same steps as torch operations took 7.2 ms,
 // and adding the chunks' weight gradients into the fp32 sum 8.1 ms more; loss
@@ -73,10 +73,9 @@ __device__ __forceinline__ float exp_term(float t) { return __builtin_amdgcn_exp
 // results included: 2^n times 2^f, f the rest of t log2 e in two parts.  What
 // becomes a probability takes this one: with exp_term 1.1e-4 of the bf16
 // results at 4092 x 128256 were not the nearest to the exact ones, with it
-// 0.6e-4, as with expf.  It needs 6 instructions more than exp_term and expf
-// 11, which shows where the row is short: us with exp_term | this | expf, bf16
-// rows: 4092 x 128256 403 | 442 | 469, 4092 x 32000 80 | 113 | 121, 1023 x
-// 50257 47 | 60 | 63, 510 x 4096 5.9 | 6.2 | 6.9.
+// 0.4e-4 to 0.9e-4, as with expf, which needs 5 instructions more.  us with
+// exp_term | this, bf16 rows: 4092 x 128256 403 | 427, 4092 x 32000 80 | 83,
+// 1023 x 50257 47 | 51, 20000 x 4096 49 | 54.
 __device__ __forceinline__ float exp_full(float t) {
     t = fmaxf(t, -200.0f);   // 2^f of an infinite t would be NaN
     const float n = rintf(t * kLog2e);
@@ -91,42 +90,38 @@ struct Lse {
 };
 __device__ __forceinline__ float base(float m) { return __builtin_isinf(m) ? 0.0f : m; }
 
-__device__ __forceinline__ Lse merge(Lse a, Lse b) {
-    const float m = fmaxf(a.m, b.m);
-    const float c = base(m);
+// The same over groups of kN neighbouring lanes of a wave, in every lane: the
+// maximum first, so that each lane rescales its part once (merging pairs costs
+// two exponentials a step: 300,000 rows of 2000 bf16 1,030 us, so 694), then the
+// sums.
+template <int kN>
+__device__ __forceinline__ Lse lane_lse(Lse p) {
+    float m = p.m;
+#pragma unroll
+    for (int d = kN / 2; d > 0; d >>= 1) m = fmaxf(m, __shfl_xor(m, d));
     // an empty part stays empty whatever the bases are; a NaN sum stays NaN
-    const float sa = a.s == 0.0f ? 0.0f : a.s * expf(base(a.m) - c);
-    const float sb = b.s == 0.0f ? 0.0f : b.s * expf(base(b.m) - c);
-    return {m, sa + sb};
+    float s = p.s == 0.0f ? 0.0f : p.s * expf(base(p.m) - base(m));
+#pragma unroll
+    for (int d = kN / 2; d > 0; d >>= 1) s += __shfl_xor(s, d);
+    return {m, s};
 }
 
-// logsumexp over the workgroup, the same value in every lane.  Wave by
-// shuffles, then the waves' parts through LDS, merged by every lane in the
-// same order.
+// logsumexp over a row's kT lanes, the same value in every one: in one wave
+// without a barrier, else through LDS.
 template <int kT>
 __device__ __forceinline__ float block_lse(Lse p, Lse* parts) {
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) {
-        const Lse o = {__shfl_xor(p.m, d), __shfl_xor(p.s, d)};
-        p = merge(p, o);
-    }
-    if (kT > 64) {
+    p = lane_lse<(kT < 64 ? kT : 64)>(p);
+    if constexpr (kT > 64) {
         if ((threadIdx.x & 63) == 0) parts[threadIdx.x >> 6] = p;
-    }
-    __syncthreads();
-    if (kT > 64) {
-        float m = parts[0].m;
-#pragma unroll
-        for (int w = 1; w < kT / 64; ++w) m = fmaxf(m, parts[w].m);
-        const float c = base(m);
-        float s = 0.0f;
-#pragma unroll
-        for (int w = 0; w < kT / 64; ++w)
-            s += parts[w].s == 0.0f ? 0.0f : parts[w].s * expf(base(parts[w].m) - c);
-        p = {m, s};
+        __syncthreads();
+        p = lane_lse<kT / 64>(parts[threadIdx.x % (kT / 64)]);
     }
     return base(p.m) + logf(p.s);
 }
+
+// Rows of one workgroup: rows that one wave or less reads share it.
+template <int kT>
+constexpr int kRowsOf = kT <= 64 ? 256 / kT : 1;
 
 // What a row's label asks for.
 enum RowKind { kValid, kIgnored, kBadLabel };
@@ -151,7 +146,7 @@ __device__ __forceinline__ void keep_packed(u32x4 (&v)[kG]) {
 }
 
 // ---------------------------------------------------------------------
-// One workgroup per row, the whole row in registers as packed 16-bit pairs:
+// kT lanes per row, the whole row in registers as packed 16-bit pairs:
 // kG groups of 8 per lane, so 4 kG VGPRs, up to 76 of the 128 a lane of a
 // 1024-lane workgroup has.  Read once, written once; between the two only
 // one barrier, since each lane sums against its own maximum and the parts
@@ -161,12 +156,15 @@ __device__ __forceinline__ void keep_packed(u32x4 (&v)[kG]) {
 // groups of every lane need no check.
 // ---------------------------------------------------------------------
 template <typename Fmt, int kT, int kG, int kFull>
-__global__ __launch_bounds__(kT) void ce_rows_kernel(uint16_t* __restrict__ logits, uint64_t ld, uint32_t vocab,
-                                                     const int64_t* __restrict__ labels, int64_t ignore_index,
-                                                     float* __restrict__ row_loss) {
-    __shared__ Lse parts[kT / 64];
-    __shared__ float target;
-    const uint64_t row = blockIdx.x;
+__global__ __launch_bounds__(kT * kRowsOf<kT>) void ce_rows_kernel(uint16_t* __restrict__ logits, uint64_t ld,
+                                                                   uint64_t rows, uint32_t vocab,
+                                                                   const int64_t* __restrict__ labels,
+                                                                   int64_t ignore_index, float* __restrict__ row_loss) {
+    __shared__ Lse parts[kT > 64 ? kT / 64 : 1];
+    __shared__ float first;
+    const uint32_t lane = threadIdx.x % kT;
+    const uint64_t row = uint64_t(blockIdx.x) * kRowsOf<kT> + threadIdx.x / kT;
+    if (kRowsOf<kT> > 1 && row >= rows) return;   // no barrier below for these
     uint16_t* x = logits + row * ld;
     u32x4* xv = reinterpret_cast<u32x4*>(x);
     const int64_t y = labels[row];
@@ -175,22 +173,29 @@ __global__ __launch_bounds__(kT) void ce_rows_kernel(uint16_t* __restrict__ logi
     if (kind != kValid) {
         const uint32_t w = kind == kIgnored ? 0u : Fmt::kNan2;
         const u32x4 fill = {w, w, w, w};
-        for (uint32_t g = threadIdx.x; g < groups; g += kT) xv[g] = fill;
-        if (threadIdx.x == 0) row_loss[row] = kind == kIgnored ? 0.0f : __builtin_nanf("");
+        for (uint32_t g = lane; g < groups; g += kT) xv[g] = fill;
+        if (lane == 0) row_loss[row] = kind == kIgnored ? 0.0f : __builtin_nanf("");
         return;
     }
     u32x4 v[kG];
 #pragma unroll
     for (int k = 0; k < kG; ++k) {
-        const uint32_t g = uint32_t(k) * kT + threadIdx.x;
+        const uint32_t g = uint32_t(k) * kT + lane;
         v[k] = xv[k < kFull || g < groups ? g : groups - 1];
     }
-    // Read before any lane writes: the barrier in block_lse stands between.
-    if (threadIdx.x == 0) target = Fmt::lo(x[y]);
+    // Read before any lane writes: the barrier in block_lse stands between, or
+    // the row's lanes are one wave's.
+    float target = 0.0f;
+    if (lane == 0) target = Fmt::lo(x[y]);
+    if (kT > 64) {
+        if (lane == 0) first = target;
+    } else {
+        target = __shfl(target, 0, kT < 64 ? kT : 64);
+    }
     const uint32_t rem = vocab % kGroup;
 #pragma unroll
     for (int k = kFull; k < kG; ++k) {
-        const uint32_t g = uint32_t(k) * kT + threadIdx.x;
+        const uint32_t g = uint32_t(k) * kT + lane;
         if (g >= groups) {
             v[k] = u32x4{Fmt::kNegInf2, Fmt::kNegInf2, Fmt::kNegInf2, Fmt::kNegInf2};
         } else if (rem != 0 && g == groups - 1) {
@@ -219,22 +224,23 @@ __global__ __launch_bounds__(kT) void ce_rows_kernel(uint16_t* __restrict__ logi
         }
     keep_packed<kG>(v);
     const float lse = block_lse<kT>({m, s0 + s1}, parts);
-    if (threadIdx.x == 0) row_loss[row] = lse - target;
+    if (kT > 64) target = first;
+    if (lane == 0) row_loss[row] = lse - target;
     if (!__builtin_isfinite(lse)) {
         // a row with NaN or infinities: what softmax gives, from memory again
-        for (uint32_t g = threadIdx.x; g < groups; g += kT) {
+        for (uint32_t g = lane; g < groups; g += kT) {
             const u32x4 r = xv[g];
             u32x4 o;
 #pragma unroll
             for (int j = 0; j < 4; ++j) o[j] = Fmt::pack(expf(Fmt::lo(r[j]) - lse), expf(Fmt::hi(r[j]) - lse));
             xv[g] = o;
         }
-        if (threadIdx.x == uint32_t(y) / kGroup % kT) x[y] = uint16_t(Fmt::pack(expf(target - lse) - 1.0f, 0.0f));
+        if (lane == uint32_t(y) / kGroup % kT) x[y] = uint16_t(Fmt::pack(expf(target - lse) - 1.0f, 0.0f));
         return;
     }
 #pragma unroll
     for (int k = 0; k < kG; ++k) {
-        const uint32_t g = uint32_t(k) * kT + threadIdx.x;
+        const uint32_t g = uint32_t(k) * kT + lane;
         u32x4 o;
 #pragma unroll
         for (int j = 0; j < 4; ++j)
@@ -242,7 +248,7 @@ __global__ __launch_bounds__(kT) void ce_rows_kernel(uint16_t* __restrict__ logi
         if (k < kFull || g < groups) xv[g] = o;
     }
     // The label's element, over what the same lane has just stored with its group.
-    if (threadIdx.x == uint32_t(y) / kGroup % kT)
+    if (lane == uint32_t(y) / kGroup % kT)
         x[y] = uint16_t(Fmt::pack(exp_full(target - lse) - 1.0f, 0.0f));
 }
 
@@ -260,28 +266,38 @@ struct Elem16 {
 };
 
 // Rows that do not fit the registers (16-bit rows of more than 155,648
-// elements) and fp32 rows: one workgroup per row, two passes, the second one
-// over what the caches still hold.
+// elements) and fp32 rows: kT lanes per row, two passes, the second one over
+// what the caches still hold.
 template <typename El, int kT>
-__global__ __launch_bounds__(kT) void ce_rows_stream_kernel(typename El::S* __restrict__ logits, uint64_t ld,
-                                                            uint32_t vocab, const int64_t* __restrict__ labels,
-                                                            int64_t ignore_index, float* __restrict__ row_loss) {
-    __shared__ Lse parts[kT / 64];
-    __shared__ float target;
-    const uint64_t row = blockIdx.x;
+__global__ __launch_bounds__(kT * kRowsOf<kT>) void ce_rows_stream_kernel(typename El::S* __restrict__ logits,
+                                                                          uint64_t ld, uint64_t rows, uint32_t vocab,
+                                                                          const int64_t* __restrict__ labels,
+                                                                          int64_t ignore_index,
+                                                                          float* __restrict__ row_loss) {
+    __shared__ Lse parts[kT > 64 ? kT / 64 : 1];
+    __shared__ float first;
+    const uint32_t lane = threadIdx.x % kT;
+    const uint64_t row = uint64_t(blockIdx.x) * kRowsOf<kT> + threadIdx.x / kT;
+    if (kRowsOf<kT> > 1 && row >= rows) return;   // no barrier below for these
     typename El::S* x = logits + row * ld;
     const int64_t y = labels[row];
     const RowKind kind = row_kind(y, ignore_index, vocab);
     if (kind != kValid) {
         const float f = kind == kIgnored ? 0.0f : __builtin_nanf("");
-        for (uint32_t i = threadIdx.x; i < vocab; i += kT) El::store(x + i, f);
-        if (threadIdx.x == 0) row_loss[row] = f;
+        for (uint32_t i = lane; i < vocab; i += kT) El::store(x + i, f);
+        if (lane == 0) row_loss[row] = f;
         return;
     }
-    if (threadIdx.x == 0) target = El::load(x + y);
+    float target = 0.0f;
+    if (lane == 0) target = El::load(x + y);
+    if (kT > 64) {
+        if (lane == 0) first = target;
+    } else {
+        target = __shfl(target, 0, kT < 64 ? kT : 64);
+    }
     constexpr int kU = 4;
     Lse p = {-__builtin_inff(), 0.0f};
-    for (uint32_t i = threadIdx.x; i < vocab; i += kT * kU) {
+    for (uint32_t i = lane; i < vocab; i += kT * kU) {
         float f[kU];
 #pragma unroll
         for (int k = 0; k < kU; ++k) f[k] = i + k * kT < vocab ? El::load(x + i + k * kT) : -__builtin_inff();
@@ -295,8 +311,9 @@ __global__ __launch_bounds__(kT) void ce_rows_stream_kernel(typename El::S* __re
         p = {m, s};
     }
     const float lse = block_lse<kT>(p, parts);
-    if (threadIdx.x == 0) row_loss[row] = lse - target;
-    for (uint32_t i = threadIdx.x; i < vocab; i += kT) {
+    if (kT > 64) target = first;
+    if (lane == 0) row_loss[row] = lse - target;
+    for (uint32_t i = lane; i < vocab; i += kT) {
         const float q = expf(El::load(x + i) - lse);
         El::store(x + i, int64_t(i) == y ? q - 1.0f : q);
     }
@@ -630,15 +647,15 @@ inline bool misaligned(const void* p, uintptr_t a) { return (reinterpret_cast<ui
 // Lanes of one launch: a dispatch takes fewer than 2^32 along a dimension.
 constexpr uint64_t kMaxLanes = uint64_t(1) << 31;
 
-// A kernel with one workgroup of kT lanes per row, over as many launches as
-// the rows need.
+// A kernel of kT lanes per row, over as many launches as the rows need.
 template <int kT, typename Kernel, typename S>
 int launch_rows(Kernel kernel, S* x, uint64_t ld, uint64_t rows, uint32_t vocab, const int64_t* labels, int64_t ignore,
                 float* row_loss, hipStream_t st) {
-    for (uint64_t r = 0; r < rows; r += kMaxLanes / kT) {
-        const uint64_t n = rows - r < kMaxLanes / kT ? rows - r : kMaxLanes / kT;
-        hipLaunchKernelGGL(kernel, dim3(uint32_t(n)), dim3(kT), 0, st, x + r * ld, ld, vocab, labels + r, ignore,
-                           row_loss + r);
+    constexpr uint64_t kMax = kMaxLanes / kT;
+    for (uint64_t r = 0; r < rows; r += kMax) {
+        const uint64_t n = rows - r < kMax ? rows - r : kMax;
+        hipLaunchKernelGGL(kernel, dim3(uint32_t((n + kRowsOf<kT> - 1) / kRowsOf<kT>)), dim3(kT * kRowsOf<kT>), 0, st,
+                           x + r * ld, ld, n, vocab, labels + r, ignore, row_loss + r);
         const int e = status();
         if (e != SF_OK) return e;
     }
@@ -694,9 +711,9 @@ int launch_weight_grad(const float* grad_loss, const float* n_valid, const void*
     return status();
 }
 
-// The smallest workgroup that holds the row: lanes first (up to 1024), then
-// groups per lane, so that short rows keep many workgroups per CU and long
-// ones all their loads in flight at once.
+// The fewest lanes that hold the row (up to 1024), then groups per lane, so
+// that short rows keep many of them on a CU and long ones all their loads in
+// flight at once.
 template <typename Fmt>
 int dispatch_rows16(uint16_t* x, uint64_t ld, uint64_t rows, uint32_t vocab, const int64_t* labels, int64_t ignore,
                     float* row_loss, hipStream_t st) {
@@ -705,6 +722,8 @@ int dispatch_rows16(uint16_t* x, uint64_t ld, uint64_t rows, uint32_t vocab, con
 #define SF_ROWS(T, G, FULL)         \
     if (groups <= uint32_t(T) * G) \
         return launch_rows<T>(ce_rows_kernel<Fmt, T, G, FULL>, x, ld, rows, vocab, labels, ignore, row_loss, st);
+    // (16 lanes: 2 M rows of 64 932 -> 216 us, rows of a wave each before)
+    SF_ROWS(16, 1, 0)
     SF_ROWS(64, 2, 0)
     SF_ROWS(256, 2, 0)
     SF_ROWS(256, 4, 2)
@@ -716,6 +735,20 @@ int dispatch_rows16(uint16_t* x, uint64_t ld, uint64_t rows, uint32_t vocab, con
     SF_ROWS(1024, 19, 16)
 #undef SF_ROWS
     return launch_rows<1024>(ce_rows_stream_kernel<Elem16<Fmt>, 1024>, x, ld, rows, vocab, labels, ignore, row_loss, st);
+}
+
+// fp32 rows: as many lanes as have a whole step of the loop to do.  us, 1024
+// lanes for every row | so: 2 M rows of 4 15,325 | 160, 500,000 of 512 4,205 |
+// 557, 65,536 of 512 555 | 69.
+int dispatch_rows32(float* x, uint64_t ld, uint64_t rows, uint32_t vocab, const int64_t* labels, int64_t ignore,
+                    float* row_loss, hipStream_t st) {
+    if (vocab <= 64)
+        return launch_rows<16>(ce_rows_stream_kernel<Elem32, 16>, x, ld, rows, vocab, labels, ignore, row_loss, st);
+    if (vocab <= 512)
+        return launch_rows<64>(ce_rows_stream_kernel<Elem32, 64>, x, ld, rows, vocab, labels, ignore, row_loss, st);
+    if (vocab <= 8192)
+        return launch_rows<256>(ce_rows_stream_kernel<Elem32, 256>, x, ld, rows, vocab, labels, ignore, row_loss, st);
+    return launch_rows<1024>(ce_rows_stream_kernel<Elem32, 1024>, x, ld, rows, vocab, labels, ignore, row_loss, st);
 }
 
 }  // namespace
@@ -730,8 +763,8 @@ int sf_ce_rows(void* logits, int dtype, size_t ld, size_t rows, size_t vocab, co
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     if (dtype == SF_DTYPE_F32) {
         if (misaligned(logits, 4)) return SF_EINVAL;
-        return launch_rows<1024>(ce_rows_stream_kernel<Elem32, 1024>, static_cast<float*>(logits), uint64_t(ld),
-                                 uint64_t(rows), uint32_t(vocab), labels, ignore_index, row_loss, st);
+        return dispatch_rows32(static_cast<float*>(logits), ld, rows, uint32_t(vocab), labels, ignore_index, row_loss,
+                               st);
     }
     if (dtype != SF_DTYPE_BF16 && dtype != SF_DTYPE_F16) return SF_EDTYPE;
     // whole 128-bit groups: every row starts on one and its last one is inside the row's ld elements

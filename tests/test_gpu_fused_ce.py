@@ -60,6 +60,35 @@ def test_rows_match_float64(dev, vocab, dtype):
     assert ((got.double() - ref_g).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+# 16, 64, 256 or 1024 lanes a row: 16-bit to 128, 1024, fp32 to 64, 512, 8192
+@pytest.mark.parametrize("vocab", [1, 8, 15, 64, 65, 128, 129, 512, 513])
+@pytest.mark.parametrize("rows", [1, 17, 333])
+def test_short_rows_share_a_workgroup(dev, rows, vocab, dtype):
+    """Rows of one wave, valid, ignored and bad ones side by side, the last
+    workgroup ragged; nothing behind the last row is touched."""
+    gen = torch.Generator(device=dev).manual_seed(rows * vocab)
+    x = (torch.randn(rows, vocab, generator=gen, device=dev) * 3).to(dtype)
+    y = torch.randint(0, vocab, (rows,), generator=gen, device=dev)
+    y[1::3], y[2::5] = -100, vocab
+    ref_loss, ref_g, p = rows_reference(x, y)
+    ref_loss[y == vocab] = float("nan")
+    ref_g[y == vocab] = float("nan")
+    ld = -(-vocab // 8) * 8
+    buf = torch.full((rows + 2, ld), 7.0, dtype=dtype, device=dev)
+    buf[:rows, :vocab] = x
+    loss = torch.full((rows + 1,), 7.0, device=dev)
+    kernels.ce_rows_(buf[:rows, :vocab], y, -100, loss[:rows])
+    half_ulp, tiny = EPS[dtype]
+    good = y != vocab
+    # as in test_rows_match_float64
+    assert ((loss[:rows].double() - ref_loss)[good].abs() <= 1e-6 * (4 + ref_loss[good].abs())).all()
+    bound = half_ulp * ref_g.abs() + 6e-6 * p + tiny
+    assert ((buf[:rows, :vocab].double() - ref_g).abs() <= bound)[good].all()
+    assert loss[:rows][~good].isnan().all() and buf[:rows, :vocab][~good].isnan().all()
+    assert (buf[rows:] == 7.0).all() and loss[rows] == 7.0
+
+
 @pytest.mark.parametrize("vocab", [40, 70_003])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_rows_special_values(dev, vocab, dtype):
