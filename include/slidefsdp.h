@@ -275,6 +275,13 @@ int sf_ce_loss(const float* row_loss, const int64_t* labels, size_t n,
                int64_t ignore_index, float* loss, float* n_valid,
                sf_stream_t stream);
 
+/* The same by many workgroups, for many rows: parts is device memory for
+ * 2 * SF_CE_LOSS_PARTS doubles. */
+#define SF_CE_LOSS_PARTS 256
+int sf_ce_loss_parts(const float* row_loss, const int64_t* labels, size_t n,
+                     int64_t ignore_index, void* parts, float* loss,
+                     float* n_valid, sf_stream_t stream);
+
 /* Both gradients times *grad_loss / *n_valid: grad_h (n_h elements of dtype)
  * into grad_h_out, grad_w (n_w fp32 elements) rounded once into grad_w_out
  * (dtype).  All four arrays start on 16-byte boundaries (SF_EALIGN). */

@@ -41,6 +41,7 @@ SF_EALIGN = 9007
 SF_ETOOBIG = 9008
 SF_ETIMEDOUT = 9009
 SF_STAGE_SCRATCH_ELEMS = 16 << 20
+SF_CE_LOSS_PARTS = 256
 # row_slot markers of the row-wise AdamW: a zero-gradient row, a row left as it is
 SF_ROW_ZERO = -1
 SF_ROW_SKIP = -2
@@ -91,6 +92,7 @@ HIP_SIGNATURES = {
     "sf_ce_rows": [_vp, _i, _sz, _sz, _sz, _vp, ctypes.c_int64, _vp, _vp],
     "sf_ce_hidden": [_vp, _sz, _sz, _sz, _vp, _sz, _vp, _sz, _vp],
     "sf_ce_sum": [_vp, _i, _sz, _sz, _vp, _i, _vp, _sz, _vp, _sz, _vp],
+    "sf_ce_loss_parts": [_vp, _vp, _sz, ctypes.c_int64, _vp, _vp, _vp, _vp],
     "sf_ce_loss": [_vp, _vp, _sz, ctypes.c_int64, _vp, _vp, _vp],
     "sf_ce_weight_grad": [_vp, _vp, _vp, _sz, _sz, _vp, _sz, _sz, _vp, _vp, _vp, _sz, _i, _vp],
     "sf_ce_scale": [_vp, _vp, _vp, _vp, _sz, _vp, _vp, _sz, _i, _vp],

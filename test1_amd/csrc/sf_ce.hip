@@ -319,37 +319,75 @@ __global__ __launch_bounds__(kT * kRowsOf<kT>) void ce_rows_stream_kernel(typena
     }
 }
 
-// Mean of the rows' losses and the number of rows it is taken over: one
-// workgroup, each row once, in an order fixed by n alone.
+// Mean of the rows' losses and the number of rows it is taken over, each row
+// once, in an order fixed by n alone: one workgroup, or, for many rows,
+// kLossParts of them into `parts` and one more over those (us, one | parts:
+// 32,768 rows 7.3 | 10.4, 65,536 12.0 | 10.4, 300,000 46 | 10.4, 2 M 633 | 10.1).
+struct LossSum {
+    double sum, count;
+};
+template <int kT>
+__device__ __forceinline__ LossSum block_sum(LossSum p, LossSum* waves) {
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) {
+        p.sum += __shfl_xor(p.sum, d);
+        p.count += __shfl_xor(p.count, d);
+    }
+    if ((threadIdx.x & 63) == 0) waves[threadIdx.x >> 6] = p;
+    __syncthreads();
+    if (threadIdx.x == 0)
+        for (int w = 1; w < kT / 64; ++w) {
+            p.sum += waves[w].sum;
+            p.count += waves[w].count;
+        }
+    return p;   // the whole sum in lane 0
+}
+
+__device__ __forceinline__ LossSum sum_rows(const float* __restrict__ row_loss, const int64_t* __restrict__ labels,
+                                            uint64_t n, int64_t ignore_index, uint64_t first, uint64_t step) {
+    LossSum p = {0.0, 0.0};
+#pragma unroll 4
+    for (uint64_t i = first; i < n; i += step) {
+        p.sum += double(row_loss[i]);
+        p.count += labels[i] != ignore_index ? 1.0 : 0.0;
+    }
+    return p;
+}
+
 constexpr int kLossThreads = 1024;
 __global__ __launch_bounds__(kLossThreads) void ce_loss_kernel(const float* __restrict__ row_loss,
                                                                const int64_t* __restrict__ labels, uint64_t n,
                                                                int64_t ignore_index, float* __restrict__ loss,
                                                                float* __restrict__ n_valid) {
-    __shared__ double ssum[kLossThreads / 64];
-    __shared__ double scnt[kLossThreads / 64];
-    double sum = 0.0, cnt = 0.0;
-    for (uint64_t i = threadIdx.x; i < n; i += kLossThreads) {
-        sum += double(row_loss[i]);
-        cnt += labels[i] != ignore_index ? 1.0 : 0.0;
-    }
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) {
-        sum += __shfl_xor(sum, d);
-        cnt += __shfl_xor(cnt, d);
-    }
-    if ((threadIdx.x & 63) == 0) {
-        ssum[threadIdx.x >> 6] = sum;
-        scnt[threadIdx.x >> 6] = cnt;
-    }
-    __syncthreads();
+    __shared__ LossSum waves[kLossThreads / 64];
+    const LossSum p = block_sum<kLossThreads>(
+        sum_rows(row_loss, labels, n, ignore_index, threadIdx.x, kLossThreads), waves);
     if (threadIdx.x != 0) return;
-    for (int w = 1; w < kLossThreads / 64; ++w) {
-        sum += ssum[w];
-        cnt += scnt[w];
-    }
-    *loss = float(sum / cnt);
-    *n_valid = float(cnt);
+    *loss = float(p.sum / p.count);
+    *n_valid = float(p.count);
+}
+
+constexpr int kLossParts = SF_CE_LOSS_PARTS;
+constexpr int kPartThreads = 256;
+__global__ __launch_bounds__(kPartThreads) void ce_loss_parts_kernel(const float* __restrict__ row_loss,
+                                                                     const int64_t* __restrict__ labels, uint64_t n,
+                                                                     int64_t ignore_index, LossSum* __restrict__ parts) {
+    __shared__ LossSum waves[kPartThreads / 64];
+    const LossSum p = block_sum<kPartThreads>(
+        sum_rows(row_loss, labels, n, ignore_index, blockIdx.x * kPartThreads + threadIdx.x,
+                               uint64_t(kLossParts) * kPartThreads),
+        waves);
+    if (threadIdx.x == 0) parts[blockIdx.x] = p;
+}
+
+__global__ __launch_bounds__(kLossParts) void ce_loss_total_kernel(const LossSum* __restrict__ parts,
+                                                                   float* __restrict__ loss,
+                                                                   float* __restrict__ n_valid) {
+    __shared__ LossSum waves[kLossParts / 64];
+    const LossSum p = block_sum<kLossParts>(parts[threadIdx.x], waves);
+    if (threadIdx.x != 0) return;
+    *loss = float(p.sum / p.count);
+    *n_valid = float(p.count);
 }
 
 // out = in * (grad_loss / n_valid) for both gradients in one launch: the
@@ -822,6 +860,22 @@ int sf_ce_loss(const float* row_loss, const int64_t* labels, size_t n, int64_t i
         return SF_EINVAL;
     hipLaunchKernelGGL(ce_loss_kernel, dim3(1), dim3(kLossThreads), 0, reinterpret_cast<hipStream_t>(stream),
                        row_loss, labels, uint64_t(n), ignore_index, loss, n_valid);
+    return status();
+}
+
+int sf_ce_loss_parts(const float* row_loss, const int64_t* labels, size_t n, int64_t ignore_index, void* parts,
+                     float* loss, float* n_valid, sf_stream_t stream) {
+    if (loss == nullptr || n_valid == nullptr || parts == nullptr ||
+        (n > 0 && (row_loss == nullptr || labels == nullptr)))
+        return SF_EINVAL;
+    if (misaligned(parts, sizeof(double))) return SF_EALIGN;
+    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    LossSum* p = static_cast<LossSum*>(parts);
+    hipLaunchKernelGGL(ce_loss_parts_kernel, dim3(kLossParts), dim3(kPartThreads), 0, st, row_loss, labels, uint64_t(n),
+                       ignore_index, p);
+    const int e = status();
+    if (e != SF_OK) return e;
+    hipLaunchKernelGGL(ce_loss_total_kernel, dim3(1), dim3(kLossParts), 0, st, p, loss, n_valid);
     return status();
 }
 

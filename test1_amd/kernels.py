@@ -403,6 +403,11 @@ def ce_grad_hidden(g: torch.Tensor, weight: torch.Tensor, parts: torch.Tensor, o
                                           _stream_ptr(stream)), "sf_ce_sum")
 
 
+# Up to here one workgroup sums the rows' losses, in less than the 10 us that the
+# two launches of more take.
+_LOSS_ROWS = 50_000
+
+
 def ce_loss(row_loss: torch.Tensor, labels: torch.Tensor, ignore_index: int, loss: torch.Tensor,
             n_valid: torch.Tensor, stream: Optional[torch.cuda.Stream] = None) -> None:
     """``n_valid`` = labels that are not ``ignore_index``, ``loss`` = sum of
@@ -414,6 +419,12 @@ def ce_loss(row_loss: torch.Tensor, labels: torch.Tensor, ignore_index: int, los
         raise TypeError("ce_loss: need int64 labels and float32 row_loss, loss and n_valid")
     if row_loss.numel() != labels.numel() or loss.numel() != 1 or n_valid.numel() != 1:
         raise ValueError("ce_loss: one row_loss per label and one-element results expected")
+    if labels.numel() > _LOSS_ROWS:
+        parts = torch.empty(2 * _native.SF_CE_LOSS_PARTS, dtype=torch.float64, device=row_loss.device)
+        _native.check(_native.hip().sf_ce_loss_parts(row_loss.data_ptr(), labels.data_ptr(), labels.numel(),
+                                                     int(ignore_index), parts.data_ptr(), loss.data_ptr(),
+                                                     n_valid.data_ptr(), _stream_ptr(stream)), "sf_ce_loss_parts")
+        return
     _native.check(_native.hip().sf_ce_loss(row_loss.data_ptr(), labels.data_ptr(), labels.numel(), int(ignore_index),
                                            loss.data_ptr(), n_valid.data_ptr(), _stream_ptr(stream)), "sf_ce_loss")
 

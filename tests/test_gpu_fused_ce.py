@@ -134,6 +134,21 @@ def test_rows_keep_probabilities_down_to_the_smallest(dev, vocab):
     assert (err <= half_ulp + 2.0 ** -22 * want).all(), (got[0, 1:25], want)
 
 
+# one workgroup up to 50,000 rows, then 256 of 256 lanes
+@pytest.mark.parametrize("n", [1, 63, 1025, 50_000, 50_001, 65_537, 1_000_003])
+def test_mean_of_the_rows(dev, n):
+    gen = torch.Generator(device=dev).manual_seed(n)
+    row_loss = torch.rand(n, generator=gen, device=dev) * 20
+    labels = torch.randint(0, 9, (n,), generator=gen, device=dev)
+    row_loss[labels == 3] = 0.0
+    loss, count = torch.full((3,), 7.0, device=dev), torch.full((3,), 7.0, device=dev)
+    kernels.ce_loss(row_loss, labels, 3, loss[1], count[1])
+    valid = int((labels != 3).sum())
+    assert count.tolist() == [7.0, float(valid), 7.0] and loss[0] == loss[2] == 7.0
+    want = row_loss.double().sum() / valid   # sums in 64 bits, rounded once
+    assert (loss[1].isnan() and valid == 0) or abs(loss[1].double() - want) <= 2.0 ** -23 * want
+
+
 def test_more_rows_than_one_launch_takes(dev):
     """fp32 rows take a workgroup of 1024 lanes each, and a launch fewer than
     2^32 lanes: 2^22 rows and more are launched in parts."""
