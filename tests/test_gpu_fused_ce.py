@@ -167,6 +167,19 @@ def test_more_rows_than_one_launch_takes(dev):
     assert ((x.double() - ref_g).abs() <= half_ulp * ref_g.abs() + 6e-6 * p + tiny).all()
 
 
+# a lane takes 8 elements, a workgroup 1024
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("n_h,n_w", [(1, 1), (7, 9), (8, 1023), (1024, 1025), (3001, 70_003)])
+def test_both_gradients_scaled(dev, n_h, n_w, dtype):
+    gen = torch.Generator(device=dev).manual_seed(n_h)
+    grad_h = torch.randn(n_h, generator=gen, device=dev).to(dtype)
+    grad_w = torch.randn(n_w, generator=gen, device=dev)
+    up, count = torch.tensor(3.0, device=dev), torch.tensor(7.0, device=dev)
+    gh, gw = kernels.ce_scale(up, count, grad_h, grad_w)
+    scale = up / count
+    assert torch.equal(gh, (grad_h.float() * scale).to(dtype)) and torch.equal(gw, (grad_w * scale).to(dtype))
+
+
 def test_more_gradients_than_one_launch_scales(dev):
     """A launch scales 2^34 elements; here the hidden gradient alone has more,
     and a little weight gradient stands before it."""
