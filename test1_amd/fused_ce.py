@@ -35,6 +35,7 @@ from . import kernels
 
 
 _DTYPES = (torch.bfloat16, torch.float16, torch.float32)
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
 
 
 def _traced() -> bool:
@@ -72,7 +73,7 @@ def _kernels_take(hidden: torch.Tensor, weight: torch.Tensor, labels: torch.Tens
             and hidden.shape[0] < 1 << 31
             and not (torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != hidden.dtype)
             and not _traced()
-            and all(type(t) in (torch.Tensor, torch.nn.Parameter) for t in (hidden, weight, labels)))
+            and type(hidden) in _PLAIN and type(weight) in _PLAIN and type(labels) in _PLAIN)
 
 
 _PARTS_VOCAB = 16384   # the shortest vocabulary that ``_vocabulary_parts`` divides
@@ -107,8 +108,10 @@ def auto_chunk_rows(tokens: int, vocab: int, hidden_size: int, element_size: int
     a product that is not made here."""
     if element_size == 4:
         return max(1, hidden_size, (256 << 20) // (4 * vocab))
-    peak = max(640 << 20, (128 << 20) + 2 * vocab * hidden_size)
     ld = _row_elements(vocab, 2)
+    if 2 * (ld + hidden_size) * (tokens + 63) <= 512 << 20:   # with any partial sums
+        return max(1, tokens)
+    peak = max(640 << 20, (128 << 20) + 2 * vocab * hidden_size)
     rows = peak // (2 * (ld + hidden_size))
     # the fewest rows of a chunk whose partial sums have to be allocated
     least = tokens if tokens <= rows else rows - (64 << 20) // ld
@@ -276,6 +279,10 @@ def _forward_kernels(ctx, hidden: torch.Tensor, weight: torch.Tensor, labels: to
     return loss
 
 
+def _torch_chunk_rows(vocab: int) -> int:
+    return max(1, (256 << 20) // (4 * vocab))
+
+
 def _forward_torch(ctx, hidden: torch.Tensor, weight: torch.Tensor, labels: torch.Tensor, ignore_index: int,
                    chunk_rows: int) -> torch.Tensor:
     n, h = hidden.shape
@@ -318,7 +325,11 @@ class ChunkedLinearCrossEntropy(torch.autograd.Function):
         if labels.shape != hidden.shape[:1]:
             raise ValueError("chunked linear cross entropy: one label per hidden row expected")
         ctx.weight_dtype = weight.dtype
-        if not _kernels_take(hidden, weight, labels):
+        take = _kernels_take(hidden, weight, labels)
+        if chunk_rows <= 0:
+            chunk_rows = (auto_chunk_rows(hidden.shape[0], weight.shape[0], weight.shape[1], hidden.element_size()) if take
+                          else _torch_chunk_rows(weight.shape[0]))
+        if not take:
             return _forward_torch(ctx, hidden, weight, labels, ignore_index, chunk_rows)
         with torch.cuda.device(hidden.device):
             return _forward_kernels(ctx, hidden, weight, labels, ignore_index, chunk_rows)
@@ -362,8 +373,5 @@ def chunked_linear_cross_entropy(hidden: torch.Tensor, weight: torch.Tensor, lab
     ``chunk_rows`` <= 0 picks the chunks (``auto_chunk_rows`` on a GPU, else
     ~256 MiB of fp32 logits)."""
     if chunk_rows <= 0:
-        if hidden.dim() == 2 and _kernels_take(hidden, weight, labels):
-            chunk_rows = auto_chunk_rows(hidden.shape[0], weight.shape[0], weight.shape[-1], hidden.element_size())
-        else:
-            chunk_rows = max(1, (256 << 20) // (4 * weight.shape[0]))
+        chunk_rows = 0 if hidden.is_cuda else _torch_chunk_rows(weight.shape[0])
     return ChunkedLinearCrossEntropy.apply(hidden, weight, labels, int(ignore_index), int(chunk_rows))
