@@ -8,15 +8,15 @@
 // one-hot update, the mask and the rounding back moved some 25 bytes per
 // logit and launched about 20 kernels per chunk.  ce_rows_kernel reads every
 // logit once and writes its gradient over it: 4 bytes per 16-bit logit.
-// Measured at 4092 rows of 128256 bf16 logits: ce_rows_kernel 0.43 ms (4.9
-// TB/s; a device copy reaches 5.1),
-// ce_scale16_kernel for the 128256 x 4096 weight and 4092 x 4096 hidden
-// gradients 0.52 ms (6.0 TB/s).  The same steps as torch operations took 7.2 ms,
-// and adding the chunks' weight gradients into the fp32 sum 8.1 ms more; loss
-// with both gradients 35.1 -> 11.3 ms.  With the hidden rows transposed for the
-// weight gradient's product (ce_hidden_kernel) 10.3, of which 9.6 are the
-// products.  At 510 rows of 4096 (hidden 512): 450 -> 195 to 248 us with the
-// host, 61 of them on the GPU, the rest host time of the launches.
+// Measured at 4092 rows of 128256 bf16 logits: ce_rows_kernel 0.43-0.45 ms
+// (4.7 to 4.9 TB/s; a device copy reaches 5.1), ce_scale16_kernel for the 128256 x 4096
+// weight and 4092 x 4096 hidden gradients 0.52 ms (6.0 TB/s).  The same steps as
+// torch operations took 7.2 ms, and adding the chunks' weight gradients into the
+// fp32 sum 8.1 ms more; loss with both gradients 35.1 -> 11.3 ms.  With the
+// hidden rows transposed for the weight gradient's product (ce_hidden_kernel)
+// 10.3, of which 9.5 are the products.  At 510 rows of 4096 (hidden 512) 450 ->
+// 165 to 260 us with the host, 60 of them on the GPU, the rest host time of the
+// launches.
 //
 // The C ABI is declared in include/slidefsdp.h.
 

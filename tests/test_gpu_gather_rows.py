@@ -102,3 +102,43 @@ def test_few_and_many_workgroups_for_a_table_in_hbm(dev, cap):
     kernels.gather_rows(table, ids, out, max_workgroups=cap)
     torch.cuda.synchronize()
     assert torch.equal(out, table[ids])
+
+
+@pytest.mark.parametrize("src_host,nrows,row_len,ntok", [(False, 500, 72, 900), (True, 500, 72, 900), (True, 100, 4096, 300)])
+def test_gathers_and_staging_in_a_captured_graph(dev, src_host, nrows, row_len, ntok):
+    """The routes look at the memory's type on the host: allowed under capture.
+    Replays with other ids and values, and eager work between them."""
+    flat = pinned_empty(nrows * row_len, torch.float32) if src_host else torch.empty(nrows * row_len, device=dev)
+    table = flat.view(nrows, row_len)
+    host = pinned_empty(50_000, torch.float32)
+    ids = torch.zeros(ntok, dtype=torch.int64, device=dev)
+    rows = torch.zeros(ntok, row_len, dtype=torch.int16, device=dev)
+    staged = torch.zeros(50_000, dtype=torch.bfloat16, device=dev)
+    work = torch.empty(8, dtype=torch.float32, device=dev)
+
+    def step():
+        kernels.gather_rows(table, ids, rows)
+        kernels.stage_f32_bf16_(staged, host, work)
+
+    flat.zero_()
+    host.zero_()
+    step()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        step()
+    for rep in range(3):
+        g = torch.Generator().manual_seed(rep)
+        flat.copy_(torch.randn(flat.numel(), generator=g))
+        host.copy_(torch.randn(host.numel(), generator=g))
+        ids.copy_(torch.randint(0, nrows, (ntok,), generator=g))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        got = rows.cpu(), staged.cpu()
+        rows.fill_(-1)
+        step()   # eager
+        torch.cuda.synchronize()
+        assert torch.equal(got[0], rows.cpu()) and torch.equal(got[1], staged.cpu())
+        bits = torch.from_numpy(oracle.cast_f32_bf16(flat.cpu().numpy()).view(np.int16)).view(nrows, row_len)
+        assert torch.equal(got[0], bits[ids.cpu()]) and torch.equal(got[1], host.bfloat16())
