@@ -117,7 +117,7 @@ int sf_cast_f32_f16_timed(const float* src, uint16_t* dst, size_t n,
  * pieces of workspace_elems (rounded down to a multiple of 8) through the
  * caller's device fp32 `workspace`: each piece is copied into it by DMA and
  * cast from it into dst, all in order on `stream`, so the workspace may be
- * reused once the stream has passed the call.  A workspace of fewer than 1 Mi
+ * reused once the stream has passed the call.  A workspace of fewer than 4 Mi
  * elements (at least 8 are required) is not used: the kernel reads any number.
  * host_src must be pinned host memory (SF_EINVAL otherwise: kernels and
  * asynchronous copies read no other), dst and workspace device memory.

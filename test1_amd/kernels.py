@@ -122,7 +122,7 @@ def stage_f32_bf16_(dst: torch.Tensor, host_src: torch.Tensor, workspace: torch.
     """dst[:] = RNE-bf16(host_src) for a pinned fp32 host tensor and a bf16 GPU
     tensor: up to 4 Mi elements by one kernel that reads the host tensor over
     the link, more piece by piece through the fp32 GPU tensor ``workspace``
-    (pieces of its size rounded down to 8 elements; one of fewer than 1 Mi is
+    (pieces of its size rounded down to 8 elements; one of fewer than 4 Mi is
     not used), all in order on ``stream``; ``workspace`` is free again once the
     stream has passed the call."""
     _check_stage_args(dst, host_src)

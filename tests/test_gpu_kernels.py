@@ -127,12 +127,12 @@ def test_cast_full_llama_layer(dev):
 
 
 @pytest.mark.parametrize("n,ws", [(0, 8), (1, 8), (13, 8), (100_003, 4099), ((1 << 22) + 5, 1 << 20),
-                                  (1 << 20, 1 << 22), (5_300_003, 1_050_001), (5_300_003, 1 << 23)])
+                                  (1 << 20, 1 << 22), (9_300_003, (4 << 20) + 11), (5_300_003, 1 << 23)])
 def test_stage_pinned_master_through_workspace(dev, n, ws):
     """Pinned fp32 host array -> bf16 device array, read by a kernel up to 4 Mi
-    elements and through a device workspace above (pieces of its size rounded
-    down to 8: several pieces, a ragged last one, a workspace larger than the
-    array), bit-exact against the oracle; the stream's order makes one
+    elements, or with a smaller workspace, and through a device workspace above
+    (pieces of its size rounded down to 8: several pieces, a ragged last one, a
+    workspace larger than the array), bit-exact against the oracle; the stream's order makes one
     workspace enough, and the array ends where it should (the element after it
     untouched)."""
     x = pinned_empty(n, torch.float32)

@@ -20,7 +20,7 @@ def stage(entry, dst, src):
     if entry == "noalloc":
         kernels.stage_f32_bf16_noalloc_(dst, src)
     else:
-        kernels.stage_f32_bf16_(dst, src, torch.empty(1 << 20, dtype=torch.float32, device=dst.device))
+        kernels.stage_f32_bf16_(dst, src, torch.empty(1 << 22, dtype=torch.float32, device=dst.device))
 
 
 @pytest.mark.parametrize("entry", ["workspace", "noalloc"])

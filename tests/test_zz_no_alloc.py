@@ -28,7 +28,7 @@ def test_noalloc_stage_matches_workspace_stage(dev):
     # (elements, piece): three pieces of the whole scratch with a ragged last
     # one, a smaller input in pieces of an odd size, and one that a kernel
     # reads without them
-    cases = [(2 * scratch + 100_003, 0), (5_300_003, 1_050_001), (1_000_003, 4099)]
+    cases = [(2 * scratch + 100_003, 0), (9_300_003, (4 << 20) + 11), (1_000_003, 4099)]
     g = torch.Generator().manual_seed(11)
     bufs = []
     for n, chunk in cases:
