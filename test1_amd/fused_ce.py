@@ -43,7 +43,7 @@ def _traced() -> bool:
     JIT trace, or a dispatch mode, ``make_fx``'s among them, to which the
     tensors themselves are plain ones.  What is called through pointers is not
     in such a record: a graph made of it would return memory that nothing
-    fills."""
+    fills.  Asked first: a compiler does not follow the other questions."""
     return (torch.compiler.is_compiling() or torch._C._is_tracing() or torch._C._len_torch_dispatch_stack() > 0
             or torch._ops._len_torch_dispatch_stack_pre_dispatch() > 0)
 
@@ -67,12 +67,12 @@ def _kernels_take(hidden: torch.Tensor, weight: torch.Tensor, labels: torch.Tens
     (mixed types or devices, other label types), the empty cases, autocast to
     another type (it would round the products), a traced call, and tensor
     subclasses."""
-    return (hidden.device.type == "cuda" and weight.device == hidden.device and labels.device == hidden.device
+    return (not _traced()
+            and hidden.device.type == "cuda" and weight.device == hidden.device and labels.device == hidden.device
             and hidden.dtype in _DTYPES and weight.dtype == hidden.dtype and labels.dtype == torch.int64
             and hidden.numel() > 0 and weight.numel() > 0 and weight.shape[0] < 1 << 31
             and hidden.shape[0] < 1 << 31
             and not (torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != hidden.dtype)
-            and not _traced()
             and type(hidden) in _PLAIN and type(weight) in _PLAIN and type(labels) in _PLAIN)
 
 
@@ -340,13 +340,12 @@ class ChunkedLinearCrossEntropy(torch.autograd.Function):
         saved = (grad_hidden, *weight_parts, n_valid)
         # The kernels take what the forward saved, unless hooks brought it back
         # otherwise or the backward itself is differentiated, batched or traced.
-        if (grad_hidden.device.type == "cuda" and all(t.device == grad_hidden.device for t in saved)
+        if (not _traced() and grad_hidden.device.type == "cuda" and all(t.device == grad_hidden.device for t in saved)
                 and grad_hidden.dtype == ctx.weight_dtype and all(t.numel() > 0 for t in saved)
                 and all(t.is_contiguous() for t in saved)
                 and grad_loss.device == n_valid.device and grad_loss.dtype == torch.float32
                 and not (torch.is_grad_enabled() and grad_loss.requires_grad)
                 and _memory_is_value(grad_loss)
-                and not _traced()
                 and all(type(t) is torch.Tensor for t in (grad_loss, *saved))
                 and grad_hidden.dtype in _DTYPES
                 and all(t.data_ptr() % 16 == 0 for t in saved[:-1])):

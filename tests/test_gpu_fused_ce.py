@@ -279,6 +279,25 @@ def test_a_traced_graph_computes_on_its_own_inputs(dev, n, chunk, pre_dispatch):
 
 
 @pytest.mark.parametrize("n,chunk", [(40, 0), (300, 128)])   # weight gradient in the backward, in the forward
+def test_compiled_in_one_graph(dev, n, chunk):
+    """A compiler follows the call whole, to torch operations; inputs of other
+    values give their own results."""
+    def step(h, w, y):
+        return chunked_linear_cross_entropy(h, w, y, chunk_rows=chunk)
+
+    compiled = torch.compile(step, backend="aot_eager", fullgraph=True)
+    for seed in (1, 2):
+        gen = torch.Generator(device=dev).manual_seed(seed)
+        h = torch.randn(n, 64, generator=gen, device=dev).bfloat16().requires_grad_(True)
+        w = (torch.randn(500, 64, generator=gen, device=dev) * 0.05).bfloat16().requires_grad_(True)
+        y = torch.randint(0, 500, (n,), generator=gen, device=dev)
+        loss = compiled(h, w, y)
+        got = (loss.detach(), *torch.autograd.grad(loss, (h, w)))
+        for x, r in zip(got, exact(h, w, y, 1.0)):
+            assert rel(x, r) < 1e-2
+
+
+@pytest.mark.parametrize("n,chunk", [(40, 0), (300, 128)])   # weight gradient in the backward, in the forward
 def test_backward_of_a_batch_of_gradients_forward_mode_and_a_negated_one(dev, n, chunk):
     """What the backward is called with can be more than its memory: a batch
     (``is_grads_batched``, ``torch.func.vmap``), a dual tensor, a negated view."""
