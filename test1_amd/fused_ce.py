@@ -316,6 +316,11 @@ def _forward_torch(ctx, hidden: torch.Tensor, weight: torch.Tensor, labels: torc
     return loss_sum / n_valid
 
 
+def _saved_plain(t: torch.Tensor, dtype: torch.dtype, device: torch.device) -> bool:
+    return (type(t) is torch.Tensor and t.dtype == dtype and t.device == device and t.numel() > 0 and t.is_contiguous()
+            and t.data_ptr() % 16 == 0)
+
+
 class ChunkedLinearCrossEntropy(torch.autograd.Function):
     @staticmethod
     def forward(ctx, hidden: torch.Tensor, weight: torch.Tensor, labels: torch.Tensor, ignore_index: int,
@@ -337,18 +342,14 @@ class ChunkedLinearCrossEntropy(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_loss: torch.Tensor):
         grad_hidden, *weight_parts, n_valid = ctx.saved_tensors
-        saved = (grad_hidden, *weight_parts, n_valid)
         # The kernels take what the forward saved, unless hooks brought it back
         # otherwise or the backward itself is differentiated, batched or traced.
-        if (not _traced() and grad_hidden.device.type == "cuda" and all(t.device == grad_hidden.device for t in saved)
-                and grad_hidden.dtype == ctx.weight_dtype and all(t.numel() > 0 for t in saved)
-                and all(t.is_contiguous() for t in saved)
-                and grad_loss.device == n_valid.device and grad_loss.dtype == torch.float32
-                and not (torch.is_grad_enabled() and grad_loss.requires_grad)
-                and _memory_is_value(grad_loss)
-                and all(type(t) is torch.Tensor for t in (grad_loss, *saved))
-                and grad_hidden.dtype in _DTYPES
-                and all(t.data_ptr() % 16 == 0 for t in saved[:-1])):
+        dtype, dev = ctx.weight_dtype, grad_hidden.device
+        part = dtype if len(weight_parts) == 2 else torch.float32
+        if (not _traced() and dev.type == "cuda" and dtype in _DTYPES and _saved_plain(grad_hidden, dtype, dev)
+                and _saved_plain(n_valid, torch.float32, dev) and all(_saved_plain(t, part, dev) for t in weight_parts)
+                and type(grad_loss) is torch.Tensor and grad_loss.device == dev and grad_loss.dtype == torch.float32
+                and not (torch.is_grad_enabled() and grad_loss.requires_grad) and _memory_is_value(grad_loss)):
             with torch.cuda.device(grad_hidden.device):
                 if len(weight_parts) == 2:
                     g, hidden_t = weight_parts

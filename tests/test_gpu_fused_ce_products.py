@@ -185,6 +185,23 @@ def test_weight_gradient_in_the_backward_with_hooks_and_twice(dev):
     torch.testing.assert_close(slope, first[1].float().sum(), rtol=0.05, atol=0.05)
 
 
+@pytest.mark.parametrize("n", [100, 300])   # factors kept, gradient kept
+@pytest.mark.parametrize("bring_back", [lambda t: t.half() if t.dim() == 2 and t.dtype == torch.float32 else t,
+                                        lambda t: t.double(),
+                                        lambda t: t.t().contiguous().t() if t.dim() == 2 else t])
+def test_saved_tensors_brought_back_in_another_form(dev, n, bring_back):
+    """Hooks may return another type or layout than they were given."""
+    gen = torch.Generator(device=dev).manual_seed(n)
+    hid = torch.randn(n, 64, generator=gen, device=dev).bfloat16().requires_grad_(True)
+    wgt = (torch.randn(700, 64, generator=gen, device=dev) * 0.05).bfloat16().requires_grad_(True)
+    y = torch.randint(0, 700, (n,), generator=gen, device=dev)
+    want = torch.autograd.grad(chunked_linear_cross_entropy(hid, wgt, y), (hid, wgt))
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, bring_back):
+        got = torch.autograd.grad(chunked_linear_cross_entropy(hid, wgt, y), (hid, wgt))
+    for g, w in zip(got, want):
+        assert g.shape == w.shape and rel(g, w.double()) <= 2.0 ** -6   # the half's and bf16's rounding
+
+
 def test_parts_and_transposed_rows_in_a_captured_graph(dev, monkeypatch):
     """Replays with eager work between them; three chunks, the last one ragged."""
     monkeypatch.setattr(fused_ce, "_vocabulary_parts", lambda *a: 4)
